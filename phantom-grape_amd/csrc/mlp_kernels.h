@@ -97,6 +97,76 @@ __device__ inline void eval_k(cfloat* w, const float (&v)[K], float (&y)[K]) {
   }
 }
 
+// ------------------------------------------------- matrix-core forward pass
+// Inference-form forward pass of one input per lane for a whole wavefront,
+// the second layer on the matrix cores.  Bound: issue cycles of the SIMD,
+// about 600 for the 64 MFMAs and 560 for the 64 transcendentals (exp2 and rcp
+// of 32 activations, quarter rate) of 64 pairs; FP32 MFMA and vector
+// instructions do not overlap on this part.  eval_k above takes its weights
+// from scalar registers, and a vector instruction with a scalar operand
+// issues every 4 cycles (one with vector operands every 2 to 3): 1024 cycles
+// for the same second layer.
+//
+// v_mfma_f32_4x4x1_16b multiplies a 4-row column (A) with a 4-column row (B)
+// in each of 16 blocks: the block of lane l is l / 4, its column l % 4, so a
+// lane's B operand and its four results belong to the lane itself, and the
+// layout of the vector code (one pair per lane, s1[k] in register k) needs
+// no transposition.  A holds 16 blocks x 4 rows = 64 weights per register;
+// cbsz 4 broadcasts block abid to all sixteen: block k of register u holds
+// W2[4u..4u+3][k], so four registers hold the whole layer.  Each instruction
+// adds one product per result, in the order k = 0..15 with one rounding per
+// product: bit for bit the chain fmaf(W2[k][j], s1[j], z) of eval_k.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+struct WaveNet {
+  float w2[4];    // second-layer weights, see above
+  f32x4 b2[4];    // second-layer biases of units 4u..4u+3
+  float w1[kH], b1[kH], w3[kH], b3;
+};
+
+// The value in a vector register, whatever the compiler knows about it.
+__device__ inline float in_vgpr(float x) {
+  asm("" : "+v"(x));
+  return x;
+}
+
+__device__ inline WaveNet load_wave_net(const float* __restrict__ w) {
+  WaveNet n;
+  const int lane = threadIdx.x & 63;
+  for (int u = 0; u < 4; ++u) {
+    n.w2[u] = w[kW2 + kH * (4 * u + (lane & 3)) + (lane >> 2)];
+    for (int r = 0; r < 4; ++r) n.b2[u][r] = in_vgpr(w[kB2 + 4 * u + r]);
+  }
+  for (int j = 0; j < kH; ++j) {
+    n.w1[j] = in_vgpr(w[kW1 + j]);
+    n.b1[j] = in_vgpr(w[kB1 + j]);
+    n.w3[j] = in_vgpr(w[kW3 + j]);
+  }
+  n.b3 = in_vgpr(w[kB3]);
+  return n;
+}
+
+template <int K>
+__device__ inline void wave_layers12(const WaveNet& n, float v, f32x4 (&z)[4]) {
+  const float s1 = sig2(fmaf(n.w1[K], v, n.b1[K]));
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    z[u] = __builtin_amdgcn_mfma_f32_4x4x1f32(n.w2[u], s1, z[u], 4, K, 0);
+  if constexpr (K + 1 < kH) wave_layers12<K + 1>(n, v, z);
+}
+
+// y(v) of every lane; all 64 lanes of the wavefront must call it.
+__device__ inline float eval_wave(const WaveNet& n, float v) {
+  f32x4 z[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) z[u] = n.b2[u];
+  wave_layers12<0>(n, v, z);
+  float y = n.b3;
+#pragma unroll
+  for (int k = 0; k < kH; ++k) y = fmaf(n.w3[k], sig2(z[k / 4][k % 4]), y);
+  return y;
+}
+
 // ---------------------------------------------------------------- FP64 fit
 // The network is fitted by Levenberg-Marquardt on the weighted least-squares
 // loss sum_s wt_s (y(v_s) - t_s)^2.  Each iteration needs the residuals and

@@ -499,7 +499,9 @@ void launch_batch(int mode, int ngroups, const int* order, const int* ioff, cons
   hipLaunchKernelGGL(pgb::zero_counter, dim3(1), dim3(64), 0, st, counter);
   PGAMD_HIP_CHECK(hipGetLastError());
   if (ngroups <= 0) return;
-  const int blocks = std::max(1, std::min(ngroups, device_cu_count() * bpc));
+  // items: groups, or (network) up to 4 slices of 64 i-particles of each
+  const long long items = mode == 1 ? 4LL * ngroups : ngroups;
+  const int blocks = (int)std::min<long long>(items, (long long)device_cu_count() * bpc);
   const double ascale = (double)(float)(1.0 / g_tab.xscale);
   const pgb::Origin og{pos64, g_tab.xscale, (float)g_tab.xscale};
   pgb::TableCut tc{table_dev(st), table_quad_dev(st), g_tab.ntab, g_tab.frc_bit};

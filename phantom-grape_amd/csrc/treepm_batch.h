@@ -75,107 +75,167 @@ __device__ inline int take_item(int* counter, int* s_item) {
   return *s_item;
 }
 
-// Learned cut-off: a group's i-particles (up to 256 at a time) over 64, 128
-// or 256 lanes, the block's G = 256 / that wave groups splitting each j-tile
-// (the network's skip test wants every lane of a wavefront on the same j).
-__global__ __launch_bounds__(kThreads) void treepm_batch_mlp(
+// Learned cut-off.  Only pairs inside the cut-off are evaluated, 64 at a time
+// whatever i-particle they belong to: a wavefront marks the pairs of its 64
+// i-particles in reach, queues them in LDS one lane after the other, runs the
+// network over the queue with every lane busy, and each lane adds the results
+// of its own pairs in j order.
+//
+// A block's item is a slice of up to 64 i-particles of a group (slices q, q +
+// 4, ... for item 4 group + q), its wavefronts taking the units of j in turn:
+// unit (tile, g) holds every G-th j of a tile of kJTile, G = 4, 2 or 1 for a
+// block of up to 64, 128 or 256 i (kMlpBlockI at a time).  A unit's sum is
+// formed in FP32 and folded into FP64.
+//
+// Clumpy box of 2^18 particles (3.9e8 listed pairs, 70 % inside the cut-off,
+// 50 i-particles per group on average): 8.6-9.5 ms with one network pass per
+// j for all lanes of a wavefront (9.2e6 passes of 64 pairs, half of them
+// empty lanes or pairs out of reach; the queue needs 4.3e6), 5.2 ms with the
+// queue and the matrix cores, 3.3-3.5 ms with slices as items: with whole
+// groups the largest (256 i) ran on alone after the others.  Four blocks per
+// CU would fit the LDS only without the queue; three hold 130 registers.
+constexpr int kMlpBlockI = 256;
+constexpr int kMlpQueue = 1024;  // queued pairs per wavefront
+
+// Keeps a wavefront's LDS writes before its other lanes' reads.
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__global__ __launch_bounds__(kThreads, 3) void treepm_batch_mlp(
     int ngroups, const int* __restrict__ order, const int* __restrict__ ioff,
     const int* __restrict__ icnt, const int* __restrict__ ilist, const int* __restrict__ joff,
     const int* __restrict__ jcnt, const int* __restrict__ jlist,
     const float4* __restrict__ pos, Origin og, mlp::Cut mc, double ascale,
     double* __restrict__ acc, int* counter) {
-  __shared__ float4 s_j[kJTile];
+  constexpr int kWaves = kThreads / 64;
+  __shared__ float4 s_j[kWaves][kJTile], s_i[kWaves][64];
+  __shared__ float s_f[kWaves][kMlpQueue];
+  __shared__ unsigned short s_pair[kWaves][kMlpQueue];
   __shared__ double s_red[3][kThreads];
   __shared__ int s_item;
   const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  float4* wj = s_j[wave];
+  float4* wi = s_i[wave];
+  float* qf = s_f[wave];
+  unsigned short* qp = s_pair[wave];
+  const mlp::WaveNet net = mlp::load_wave_net(mc.w);
+  // r2 > 0 and r2 < r_c^2 (or the S2 core's radius^2) as one unsigned
+  // comparison of the float bits: 0 wraps round, NaN lies above
+  const unsigned rcb = __float_as_uint(mc.rc2) - 1u;
+  const unsigned ppb = mc.pp2 > 0.f ? __float_as_uint(mc.pp2) - 1u : 0u;
   for (;;) {
     const int it = take_item(counter, &s_item);
-    if (it >= ngroups) break;
-    const int grp = order ? order[it] : it;
+    if (it / 4 >= ngroups) break;
+    const int grp = order ? order[it / 4] : it / 4;
     const int i0 = ioff[grp], ni = icnt[grp];
     const int j0 = joff[grp], nj = jcnt[grp];
+    if ((it & 3) * 64 >= ni) continue;  // uniform: every thread read the same item
     double ox = 0.0, oy = 0.0, oz = 0.0;
-    if (og.pos64 && ni > 0) {
+    if (og.pos64) {
       const double* o = og.pos64 + 3 * (size_t)ilist[i0];
       ox = o[0];
       oy = o[1];
       oz = o[2];
     }
-    for (int ib = 0; ib < ni; ib += kThreads) {
-      const int nib = min(kThreads, ni - ib);
-      const int bi = nib <= 64 ? 64 : (nib <= 128 ? 128 : 256);
-      const int G = kThreads / bi;
-      const int il = tid % bi;
-      const int g = __builtin_amdgcn_readfirstlane(tid / bi);  // uniform per wave
-      const bool iv = il < nib;
-      const int ii = ilist[i0 + ib + (iv ? il : 0)];
+    for (int i1 = (it & 3) * 64; i1 < ni; i1 += kMlpBlockI) {
+      const int nib = min(kMlpBlockI, ni - i1 / kMlpBlockI * kMlpBlockI);
+      const int G = nib <= 64 ? 4 : (nib <= 128 ? 2 : 1);
+      const int nl = min(64, ni - i1);  // lanes with an i-particle
+      const bool iv = lane < nl;
+      const int ii = ilist[i0 + i1 + (iv ? lane : 0)];
       const float4 ip = load_pos<true>(pos, og, ii, ox, oy, oz);
-      double ax = 0.0, ay = 0.0, az = 0.0;
-      for (int jt = 0; jt < nj; jt += kJTile) {
+      wi[lane] = ip;
+      // so many j at a time that their pairs with nl lanes fit the queue
+      const int step = nl <= kMlpQueue / 32 ? 32 : kMlpQueue / 64;
+      // 0, or NaN for an i-particle without a finite position
+      double ax = (double)(ip.x - ip.x), ay = (double)(ip.y - ip.y), az = (double)(ip.z - ip.z);
+      const int units = G * ((nj + kJTile - 1) / kJTile);
+      for (int u = wave; u < units; u += kWaves) {
+        const int jt = u / G * kJTile, g = u % G;
         const int nt = min(kJTile, nj - jt);
-        __syncthreads();
-        if (tid < nt) s_j[tid] = load_pos<false>(pos, og, jlist[j0 + jt + tid], ox, oy, oz);
-        __syncthreads();
+        const int nsub = nt > g ? (nt - g + G - 1) / G : 0;  // j = jt + g + G t
+        for (int t = lane; t < nsub; t += 64)
+          wj[t] = load_pos<false>(pos, og, jlist[j0 + jt + g + G * t], ox, oy, oz);
+        wave_lds_sync();
         float fax = 0.f, fay = 0.f, faz = 0.f;
-        {
-          // This wave's j are jj = g + G t.  Pass 1 marks (64 t at a time,
-          // bit t of a wave-uniform mask) the j that some lane has inside
-          // the cut-off, and those inside the S2 core; pass 2 evaluates the
-          // network only for the first, four j per parameter pass, pass 3
-          // the core term for the second.  Pairs outside contribute exactly
-          // 0, as in the table path, so skipping them changes no sum.
-          const int nsub = nt > g ? (nt - g + G - 1) / G : 0;
-          for (int c0 = 0; c0 < nsub; c0 += 64) {
-            const int cn = min(64, nsub - c0);
-            unsigned long long mask = 0ull, cmask = 0ull;
-            for (int t = 0; t < cn; ++t) {
-              const float4 q = s_j[g + G * (c0 + t)];
-              const float dx = q.x - ip.x;
-              const float dy = q.y - ip.y;
-              const float dz = q.z - ip.z;
-              const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-              const bool in = iv && r2 > 0.f && r2 < mc.rc2;
-              if (__builtin_amdgcn_ballot_w64(in)) mask |= 1ull << t;
-              if (__builtin_amdgcn_ballot_w64(in && r2 < mc.pp2)) cmask |= 1ull << t;
-            }
-            for (int pass = 0; pass < 2; ++pass) {
-              unsigned long long mk = pass == 0 ? mask : cmask;
-              while (mk) {
-                float v[4], r2s[4], rs[4], rinvs[4], ddx[4], ddy[4], ddz[4];
-                bool inb[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                  const bool ok = mk != 0ull;
-                  const int t = ok ? __builtin_ctzll(mk) : 0;
-                  if (ok) mk &= mk - 1ull;
-                  const float4 q = s_j[g + G * (c0 + t)];
+        // 64 t at a time: the pairs inside the cut-off in t order (pass 0),
+        // then the second term of those inside the S2 core (pass 1).  Pairs
+        // outside contribute exactly 0, so leaving them out changes no sum.
+        for (int c0 = 0; c0 < nsub; c0 += 64) {
+          const int cn = min(64, nsub - c0);
+          const float4* sj = wj + c0;
+          unsigned long long core = 0ull;  // lane's pairs inside the core
+#pragma unroll 1
+          for (int pass = 0; pass < 2; ++pass) {
+            if (pass == 1 && !__builtin_amdgcn_ballot_w64(core != 0ull)) break;
+#pragma unroll 1
+            for (int s0 = 0; s0 < cn; s0 += step) {
+              const int sn = min(step, cn - s0);
+              unsigned m = 0u;  // bit t - s0
+              if (pass == 0) {
+                unsigned in_core = 0u;
+#pragma unroll 4
+                for (int t = 0; t < sn; ++t) {
+                  const float4 q = sj[s0 + t];
                   const float dx = q.x - ip.x;
                   const float dy = q.y - ip.y;
                   const float dz = q.z - ip.z;
                   const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                  const float rinv = __builtin_amdgcn_rsqf(r2);
-                  const float r = r2 * rinv;
-                  v[u] = pass == 0 ? mlp::cut_input(mc, r) : r * mc.inv_pp;
-                  inb[u] = ok && r2 > 0.f && r2 < (pass == 0 ? mc.rc2 : mc.pp2);
-                  r2s[u] = r2;
-                  rs[u] = r;
-                  rinvs[u] = rinv;
-                  ddx[u] = q.w * dx;
-                  ddy[u] = q.w * dy;
-                  ddz[u] = q.w * dz;
+                  const unsigned b = __float_as_uint(r2) - 1u;
+                  m |= b < rcb ? 1u << t : 0u;
+                  in_core |= b < ppb ? 1u << t : 0u;
                 }
-                float y[4];
-                mlp::eval_k<4>(mlp::fresh(mlp::as_const(mc.w)), v, y);
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                  const float fm = pass == 0 ? mlp::cut_main(mc, y[u], rs[u], r2s[u], rinvs[u])
-                                             : y[u] * mc.cpp;
-                  const float f = inb[u] ? fm : 0.f;
-                  fax = fmaf(f, ddx[u], fax);
-                  fay = fmaf(f, ddy[u], fay);
-                  faz = fmaf(f, ddz[u], faz);
-                }
+                m = iv ? m : 0u;
+                core |= (unsigned long long)(iv ? in_core : 0u) << s0;
+              } else {
+                m = (unsigned)(core >> s0) & (step == 32 ? ~0u : (1u << step) - 1u);
               }
+              // queue slots: an exclusive sum of the lanes' counts, bit by bit
+              const int cnt = __popc(m);
+              int base = 0, total = 0;
+#pragma unroll
+              for (int b = 0; b < 6; ++b) {
+                const unsigned long long v = __builtin_amdgcn_ballot_w64((cnt >> b) & 1);
+                base += (int)__builtin_amdgcn_mbcnt_hi((unsigned)(v >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo((unsigned)v, 0u))
+                        << b;
+                total += __popcll(v) << b;
+              }
+              int k = base;
+              for (unsigned r = m; r != 0u; r &= r - 1u)
+                qp[k++] = (unsigned short)(lane << 6 | (s0 + __builtin_ctz(r)));
+              wave_lds_sync();
+#pragma unroll 1
+              for (int r0 = 0; r0 < total; r0 += 64) {
+                const int at = min(r0 + lane, total - 1);
+                const int code = qp[at];
+                const float4 q = sj[code & 63];
+                const float4 p = wi[code >> 6];
+                const float dx = q.x - p.x;
+                const float dy = q.y - p.y;
+                const float dz = q.z - p.z;
+                const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                const float rinv = __builtin_amdgcn_rsqf(r2);
+                const float r = r2 * rinv;
+                const float v = pass == 0 ? mlp::cut_input(mc, r) : r * mc.inv_pp;
+                const float y = mlp::eval_wave(net, v);
+                qf[at] = pass == 0 ? mlp::cut_main(mc, y, r, r2, rinv) : y * mc.cpp;
+              }
+              wave_lds_sync();
+              k = base;
+              for (unsigned r = m; r != 0u; r &= r - 1u) {
+                const float4 q = sj[s0 + __builtin_ctz(r)];
+                const float f = qf[k++];
+                fax = fmaf(f, q.w * (q.x - ip.x), fax);
+                fay = fmaf(f, q.w * (q.y - ip.y), fay);
+                faz = fmaf(f, q.w * (q.z - ip.z), faz);
+              }
+              wave_lds_sync();
             }
           }
         }
@@ -183,20 +243,17 @@ __global__ __launch_bounds__(kThreads) void treepm_batch_mlp(
         ay += (double)fay;
         az += (double)faz;
       }
-      if (G > 1) {
-        __syncthreads();
-        s_red[0][tid] = ax;
-        s_red[1][tid] = ay;
-        s_red[2][tid] = az;
-        __syncthreads();
-        if (g == 0)
-          for (int q = 1; q < G; ++q) {
-            ax += s_red[0][q * bi + il];
-            ay += s_red[1][q * bi + il];
-            az += s_red[2][q * bi + il];
-          }
-      }
-      if (g == 0 && iv) {
+      __syncthreads();
+      s_red[0][tid] = ax;
+      s_red[1][tid] = ay;
+      s_red[2][tid] = az;
+      __syncthreads();
+      if (tid < nl) {
+        for (int q = 1; q < kWaves; ++q) {
+          ax += s_red[0][64 * q + tid];
+          ay += s_red[1][64 * q + tid];
+          az += s_red[2][64 * q + tid];
+        }
         acc[3 * (size_t)ii + 0] = ax * ascale;
         acc[3 * (size_t)ii + 1] = ay * ascale;
         acc[3 * (size_t)ii + 2] = az * ascale;
