@@ -17,7 +17,6 @@
 #include "treepm_batch.h"
 #include "pm_kernels.h"
 
-#include <hipcub/device/device_radix_sort.hpp>
 #include <hipfft/hipfft.h>
 
 #include <algorithm>
@@ -1408,10 +1407,21 @@ namespace {
 struct PmCache {
   int M = 0;
   hipfftHandle fwd{}, inv{};
+  int batch = 1;  // transforms per execution of inv
   DevBuf rho, rhok, fk, f;
-  DevBuf keys, order, sort_tmp;  // particle sort by mesh cell (pm_keys)
+  DevBuf bricks;  // per brick: count, start; then the chunks and their number
+  DevBuf place, order, part;  // per particle: place in its brick, sorted index and data
   DevBuf fix;  // pm_mass_part's block sums, then the fixed-point scale
 };
+// The three inverse transforms run as one batch up to this mesh (36 -> 24 us
+// each at 128^3); beyond it one after the other, which needs a third of the
+// FFT's work memory.
+constexpr int kPmBatchMesh = 256;
+// Particles per brick from which the brick sort pays: below it the boxes of
+// 10^3 points are mostly empty and the particles go straight to the mesh.
+// Clumpy boxes on a 128^3 mesh, straight / sorted: 198 / 185 us at 4.0
+// particles per brick, 217 / 189 us at 7.3; 192^3 565 / 577 us at 4.7.
+constexpr int kPmPerBrick = 3;
 PmCache g_pm;
 std::mutex g_pm_mutex;
 
@@ -1427,7 +1437,10 @@ void pm_setup(PmCache& c, int M) {
   c.fk.reserve(sizeof(double2) * nk * 3);
   c.f.reserve(sizeof(double) * nr * 3);
   PGAMD_FFT_CHECK(hipfftPlan3d(&c.fwd, M, M, M, HIPFFT_D2Z));
-  PGAMD_FFT_CHECK(hipfftPlan3d(&c.inv, M, M, M, HIPFFT_Z2D));
+  c.batch = M <= kPmBatchMesh ? 3 : 1;
+  int dims[3] = {M, M, M};
+  PGAMD_FFT_CHECK(hipfftPlanMany(&c.inv, 3, dims, nullptr, 1, 0, nullptr, 1, 0, HIPFFT_Z2D,
+                                 c.batch));
   c.M = M;
 }
 
@@ -1460,36 +1473,58 @@ PGAMD_API int pg5t_pm_force(int n, const double* pos, const double* mass, int me
   double2* rhok = c.rhok.as<double2>();
   double2* fk = c.fk.as<double2>();
   double* f = c.f.as<double>();
-  PGAMD_HIP_CHECK(hipMemsetAsync(rho, 0, sizeof(double) * nr, st));
-  // particles sorted by the Morton code of their nearest mesh point
-  const int* order = nullptr;
+  const int nb = pm::brick_edges(mesh);
+  const long long nbricks = (long long)nb * nb * nb;
+  const bool sorted = n >= kPmPerBrick * nbricks;
+  int* nchunks = nullptr;
+  pm::Chunk* chunks = nullptr;
+  int* order = nullptr;
+  double4* part = nullptr;
+  const int max_chunks = sorted ? (int)(nbricks + n / pm::kChunk) : 0;
+  int* count = nullptr;
+  if (sorted) {
+    c.bricks.reserve(sizeof(pm::Chunk) * (size_t)max_chunks +
+                     sizeof(int) * (2 * (size_t)nbricks + 1));
+    chunks = c.bricks.as<pm::Chunk>();
+    count = reinterpret_cast<int*>(chunks + max_chunks);
+  }
+  c.fix.reserve(sizeof(double) * (pm::kMassBlocks + 1));
+  double* msum = c.fix.as<double>();
+  double* scale = msum + pm::kMassBlocks;
+  const unsigned zblocks = (unsigned)std::min<size_t>(8192, (nr / 2 + 255) / 256);
+  hipLaunchKernelGGL(pm::pm_begin, dim3(std::max<unsigned>(zblocks, pm::kMassBlocks)), dim3(256),
+                     0, st, nr, reinterpret_cast<double2*>(rho), sorted ? (int)nbricks : 0, count,
+                     n, mass, msum);
+  PGAMD_HIP_CHECK(hipGetLastError());
   if (n > 0) {
-    c.keys.reserve(2 * sizeof(unsigned) * (size_t)n);
-    c.order.reserve(2 * sizeof(int) * (size_t)n);
-    unsigned* kin = c.keys.as<unsigned>();
-    int* vin = c.order.as<int>();
-    hipLaunchKernelGGL(pm::pm_keys, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, pos, mesh, kin,
-                       vin);
-    PGAMD_HIP_CHECK(hipGetLastError());
-    // the keys interleave three coordinates of ceil(log2 mesh) bits each
-    int b = 1;
-    while ((1 << b) < mesh) ++b;
-    const int end_bit = 3 * b;
-    size_t tmp = 0;
-    PGAMD_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, kin, kin + n, vin, vin + n,
-                                                       n, 0, end_bit, st));
-    c.sort_tmp.reserve(tmp);
-    PGAMD_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(c.sort_tmp.ptr, tmp, kin, kin + n, vin,
-                                                       vin + n, n, 0, end_bit, st));
-    order = vin + n;
-    c.fix.reserve(sizeof(double) * (pm::kMassBlocks + 1));
-    double* part = c.fix.as<double>();
-    double* scale = part + pm::kMassBlocks;
-    hipLaunchKernelGGL(pm::pm_mass_part, dim3(pm::kMassBlocks), dim3(256), 0, st, n, mass, part);
-    hipLaunchKernelGGL(pm::pm_fix_scale, dim3(1), dim3(64), 0, st, part, mesh, scale);
-    hipLaunchKernelGGL(pm::pm_assign_sorted, dim3(ceil_div(n, pm::kAssignRun)),
-                       dim3(pm::kAssignThreads), 0, st, n, order, pos, mass, mesh, scale,
-                       reinterpret_cast<unsigned long long*>(rho));
+    unsigned long long* fixed = reinterpret_cast<unsigned long long*>(rho);
+    if (sorted) {
+      int* start = count + nbricks;
+      nchunks = start + nbricks;
+      c.place.reserve(sizeof(int2) * (size_t)n);
+      c.order.reserve(sizeof(int) * (size_t)n);
+      c.part.reserve(sizeof(double4) * (size_t)n);
+      int2* place = c.place.as<int2>();
+      order = c.order.as<int>();
+      part = c.part.as<double4>();
+      const dim3 cgrid(ceil_div(n, pm::kCountThreads * pm::kCountPer)), cblock(pm::kCountThreads);
+      if (nbricks <= pm::kLdsBricks)
+        hipLaunchKernelGGL(pm::pm_count<true>, cgrid, cblock, 0, st, n, pos, mesh, nb, count, place);
+      else
+        hipLaunchKernelGGL(pm::pm_count<false>, cgrid, cblock, 0, st, n, pos, mesh, nb, count,
+                           place);
+      hipLaunchKernelGGL(pm::pm_scan, dim3(1), dim3(1024), 0, st, (int)nbricks, count, start,
+                         chunks, nchunks, msum, mesh, scale);
+      hipLaunchKernelGGL(pm::pm_scatter, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, pos, mass,
+                         mesh, start, place, order, part);
+      hipLaunchKernelGGL(pm::pm_assign, dim3(max_chunks), dim3(pm::kBrickThreads), 0, st, nchunks,
+                         chunks, part, mesh, nb, scale, fixed);
+    } else {
+      hipLaunchKernelGGL(pm::pm_scan, dim3(1), dim3(1024), 0, st, 0, nullptr, nullptr, nullptr,
+                         nullptr, msum, mesh, scale);
+      hipLaunchKernelGGL(pm::pm_assign_direct, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, pos,
+                         mass, mesh, scale, fixed);
+    }
     hipLaunchKernelGGL(pm::pm_fix_to_double, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0,
                        st, nr, scale, rho);
     PGAMD_HIP_CHECK(hipGetLastError());
@@ -1498,12 +1533,15 @@ PGAMD_API int pg5t_pm_force(int n, const double* pos, const double* mass, int me
   hipLaunchKernelGGL(pm::pm_green, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, mesh,
                      eps_pm, rhok, fk);
   PGAMD_HIP_CHECK(hipGetLastError());
-  for (int d = 0; d < 3; ++d)
+  for (int d = 0; d < 3; d += c.batch)
     PGAMD_FFT_CHECK(hipfftExecZ2D(c.inv, reinterpret_cast<hipfftDoubleComplex*>(fk + d * nk),
                                   f + d * nr));
-  if (n > 0)
-    hipLaunchKernelGGL(pm::pm_interp, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, order, pos,
-                       mesh, f, f + nr, f + 2 * nr, acc);
+  if (sorted)
+    hipLaunchKernelGGL(pm::pm_interp, dim3(max_chunks), dim3(pm::kBrickThreads), 0, st, nchunks,
+                       chunks, order, part, mesh, nb, f, acc);
+  else if (n > 0)
+    hipLaunchKernelGGL(pm::pm_interp_direct, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, pos,
+                       mesh, f, acc);
   PGAMD_HIP_CHECK(hipGetLastError());
   return 0;
 }
