@@ -133,12 +133,18 @@ struct Lists {
   double* cells = nullptr;  // [ncells][10]
 };
 
-// One pinned int per process for scan totals; builds run one at a time under
-// the library's mutex.
+// Pinned ints for scan totals and other counts a kernel reports to the host;
+// builds run one at a time under the library's mutex.
+constexpr int kHostInts = 64;
 int* scan_total_host() {
   static int* p = nullptr;
-  if (!p) PGAMD_HIP_CHECK(hipHostMalloc((void**)&p, sizeof(int), hipHostMallocMapped));
+  if (!p) PGAMD_HIP_CHECK(hipHostMalloc((void**)&p, kHostInts * sizeof(int), hipHostMallocMapped));
   return p;
+}
+int* host_dev(int* host) {
+  int* dev = nullptr;
+  PGAMD_HIP_CHECK(hipHostGetDevicePointer((void**)&dev, host, 0));
+  return dev;
 }
 
 // Temporary storage for one build, released at its end.
@@ -169,19 +175,22 @@ struct Build {
     PGAMD_HIP_CHECK(hipStreamSynchronize(st));
     return v;
   }
+  // out[k] = sum in[0..k) for k < n, not waited for.
+  void scan_async(const int* in, int* out, int n) {
+    size_t b = 0;
+    PGAMD_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, b, in, out, n, st));
+    PGAMD_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(cub_tmp(b), b, in, out, n, st));
+  }
   // out[k] = sum in[0..k), out[n] = total (out has n + 1 entries); returns
   // total.  The total comes back through mapped pinned memory: one kernel and
   // a synchronisation for small n, the hipCUB scan for large n.
   int scan(const int* in, int* out, int n) {
     int* host = scan_total_host();
-    int* dev = nullptr;
-    PGAMD_HIP_CHECK(hipHostGetDevicePointer((void**)&dev, host, 0));
+    int* dev = host_dev(host);
     if (n <= kSmallScan) {
       hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kSmallScanThreads), 0, st, in, out, n, dev);
     } else {
-      size_t b = 0;
-      PGAMD_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, b, in, out, n, st));
-      PGAMD_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(cub_tmp(b), b, in, out, n, st));
+      scan_async(in, out, n);
       hipLaunchKernelGGL(k_scan_total, dim3(1), dim3(64), 0, st, in, out, n, dev);
     }
     PGAMD_HIP_CHECK(hipGetLastError());
@@ -306,73 +315,201 @@ struct Nodes {
 
 __device__ inline int digit(u64 key, int shift) { return (int)((key >> shift) & 7ULL); }
 
-// First index in [a, b) whose octant digit at `shift` is >= o (digits are
-// non-decreasing inside a node).
-__device__ inline int lower_digit(const u64* key, int a, int b, int shift, int o) {
-  while (a < b) {
-    const int mid = a + (b - a) / 2;
-    if (digit(key[mid], shift) < o)
-      a = mid + 1;
-    else
-      b = mid;
-  }
-  return a;
+// The whole octree from the sorted keys, without walking it level by level
+// (15 levels of split, scan and read-back took 0.45 ms of a 2^21-particle
+// build).  A cell of level l is a run of keys with the same first l digits,
+// and it is a node if its parent holds more than `split` particles:
+//   * particle i starts a cell at every level from a_i = 1 + the digits it
+//     shares with particle i - 1 (0 for i = 0);
+//   * its leaf is at level D_i, the first whose cell holds at most `split`
+//     particles (or kLevels): a cell holds more if two of its particles are
+//     `split` places apart, so D_i = 1 + the most digits shared by any pair
+//     (j, j + split) with i - split <= j <= i, a sliding maximum.
+// So the nodes that start at i are its cells of levels a_i .. D_i.  Counting
+// them per level and block of particles, one scan numbers the nodes level by
+// level, in particle order inside a level.
+__device__ inline int shared_digits(u64 x, u64 y) {
+  const u64 d = x ^ y;
+  return d == 0 ? kLevels : (__clzll((long long)d) - 1) / 3;
 }
 
-// Octant ranges of the nodes [a, b) of one level: eight threads per node,
-// thread o finding where octant o ends (the first index of the node's range
-// whose octant digit exceeds o), so the eight binary searches run side by
-// side.  end[8 * (k - a) + o] keeps the ends for k_split_fill; nchild[k - a]
-// = the number of non-empty octants (0 for a node that is not split).
-__global__ void k_split_count(int a, int b, Nodes nd, const u64* __restrict__ key, int split,
-                              int* __restrict__ end, int* __restrict__ nchild) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int k = a + (int)(t >> 3), o = (int)(t & 7);
-  int lo = 0, e = 0;
-  bool splits = false;
-  if (k < b) {
-    const int hi = nd.hi[k], lev = nd.lev[k];
-    lo = nd.lo[k];
-    e = lo;
-    splits = hi - lo > split && lev < kLevels;
-    if (splits) e = o == 7 ? hi : lower_digit(key, lo, hi, 3 * (kLevels - 1 - lev), o + 1);
-    end[8 * (size_t)(k - a) + o] = e;
+// out[i] = max of in[max(0, i - w + 1) .. i], w <= kMaxWindow + 1.  FIRST: in[j]
+// = 1 + the digits shared by keys j and j + split (0 if there is no such
+// key).  By doubling in LDS.
+constexpr int kWindowOut = 2048;
+constexpr int kMaxWindow = 1024;
+template <bool FIRST>
+__global__ __launch_bounds__(256) void k_window_max(int n, int split, int w,
+                                                    const u64* __restrict__ key,
+                                                    const unsigned char* __restrict__ in,
+                                                    unsigned char* __restrict__ out) {
+  __shared__ unsigned char buf[2][kWindowOut + kMaxWindow];
+  const int h = w - 1, m = kWindowOut + h;
+  const int j0 = blockIdx.x * kWindowOut - h;
+  for (int p = threadIdx.x; p < m; p += 256) {
+    const int j = j0 + p;
+    int v = 0;
+    if (FIRST) {
+      if (j >= 0 && j < n - split) v = 1 + shared_digits(key[j], key[j + split]);
+    } else if (j >= 0 && j < n) {
+      v = in[j];
+    }
+    buf[0][p] = (unsigned char)v;
   }
-  // a node's eight threads are one aligned group of eight lanes: octant o
-  // starts where octant o - 1 ends
-  const int lane = threadIdx.x & 63;
-  const int prev = __shfl(e, (lane + 63) & 63);
-  const unsigned long long m = __ballot(splits && e > (o == 0 ? lo : prev));
-  if (k < b && o == 0) nchild[k - a] = __popcll((m >> lane) & 0xffULL);
+  __syncthreads();
+  int cur = 0, len = 1;  // buf[cur][p] = max over [p - len + 1, p]
+  for (; 2 * len <= w; len *= 2) {
+    for (int p = threadIdx.x; p < m; p += 256)
+      buf[1 - cur][p] = max(buf[cur][p], p >= len ? buf[cur][p - len] : (unsigned char)0);
+    cur = 1 - cur;
+    __syncthreads();
+  }
+  for (int q = threadIdx.x; q < kWindowOut; q += 256) {
+    const int i = blockIdx.x * kWindowOut + q, p = q + h;
+    if (i < n) out[i] = max(buf[cur][p], buf[cur][p - (w - len)]);
+  }
 }
 
-// Children of the nodes [a, b) from the octant ends of k_split_count: eight
-// threads per node, thread o writing child o (numbered after the level, in
-// node order, then octant order).
-__global__ void k_split_fill(int a, int b, Nodes nd, const int* __restrict__ end,
-                             const int* __restrict__ off, double L) {
+constexpr int kTreeLevels = kLevels + 1;
+constexpr int kTreeRounds = 4;               // particles per thread of the two passes
+constexpr int kTreeBlock = 256 * kTreeRounds;  // particles per block
+
+// Levels a .. d of the nodes that start at particle i (a > d: none).
+__device__ inline void start_levels(int i, int n, const u64* __restrict__ key,
+                                    const unsigned char* __restrict__ leaf, int* a, int* d) {
+  *a = 1;
+  *d = 0;
+  if (i >= n) return;
+  *a = i == 0 ? 0 : 1 + shared_digits(key[i - 1], key[i]);
+  *d = min((int)leaf[i], kLevels);
+}
+
+// count[l * gridDim.x + block] = nodes of level l that start in the block.
+__global__ __launch_bounds__(256) void k_tree_count(int n, const u64* __restrict__ key,
+                                                    const unsigned char* __restrict__ leaf,
+                                                    int* __restrict__ count) {
+  __shared__ int s_cnt[4][kTreeLevels];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int mine = 0;  // lane l: nodes of level l seen by this wavefront
+  for (int r = 0; r < kTreeRounds; ++r) {
+    int a, d;
+    start_levels(blockIdx.x * kTreeBlock + r * 256 + threadIdx.x, n, key, leaf, &a, &d);
+    for (int l = 0; l < kTreeLevels; ++l) {
+      const int c = __popcll(__ballot(a <= l && l <= d));
+      mine += lane == l ? c : 0;
+    }
+  }
+  if (lane < kTreeLevels) s_cnt[wave][lane] = mine;
+  __syncthreads();
+  if (threadIdx.x < kTreeLevels)
+    count[threadIdx.x * gridDim.x + blockIdx.x] =
+        s_cnt[0][threadIdx.x] + s_cnt[1][threadIdx.x] + s_cnt[2][threadIdx.x] + s_cnt[3][threadIdx.x];
+}
+
+// host[l] = first node of level l, host[kTreeLevels] = number of nodes, from
+// the scan of k_tree_count's counts (nb blocks).
+__global__ void k_tree_levels(int nb, const int* __restrict__ count, const int* __restrict__ first,
+                              int* __restrict__ host) {
+  const int l = threadIdx.x;
+  if (l < kTreeLevels) host[l] = first[(size_t)l * nb];
+  if (l == kTreeLevels) {
+    const size_t e = (size_t)kTreeLevels * nb - 1;
+    host[l] = first[e] + count[e];
+  }
+}
+
+// Nodes' first particle, level and parent, and the parents' child links
+// (child[] is -1 before).  first[l * gridDim.x + block] = number of the
+// block's first node of level l.
+__global__ __launch_bounds__(256) void k_tree_fill(int n, const u64* __restrict__ key,
+                                                   const unsigned char* __restrict__ leaf,
+                                                   const int* __restrict__ first, Nodes nd) {
+  __shared__ int s_cnt[kTreeRounds][4][kTreeLevels];
+  __shared__ int s_first[kTreeLevels];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x < kTreeLevels) s_first[threadIdx.x] = first[threadIdx.x * gridDim.x + blockIdx.x];
+  int a[kTreeRounds], d[kTreeRounds];
+#pragma unroll
+  for (int r = 0; r < kTreeRounds; ++r) {
+    start_levels(blockIdx.x * kTreeBlock + r * 256 + threadIdx.x, n, key, leaf, &a[r], &d[r]);
+    for (int l = 0; l < kTreeLevels; ++l) {
+      const int c = __popcll(__ballot(a[r] <= l && l <= d[r]));
+      if (lane == l) s_cnt[r][wave][l] = c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kTreeRounds; ++r) {
+    const int i = blockIdx.x * kTreeBlock + r * 256 + threadIdx.x;
+    int up = 0;  // the last node of the level above that starts at or before i
+    for (int l = 0; l < kTreeLevels; ++l) {
+      int base = s_first[l];
+      for (int q = 0; q < r; ++q)
+        base += s_cnt[q][0][l] + s_cnt[q][1][l] + s_cnt[q][2][l] + s_cnt[q][3][l];
+      for (int q = 0; q < wave; ++q) base += s_cnt[r][q][l];
+      const bool starts = a[r] <= l && l <= d[r];
+      const u64 m = __ballot(starts);
+      const int below = __popcll(m & ((1ULL << lane) - 1ULL));
+      if (starts) {
+        const int id = base + below;
+        nd.lo[id] = i;
+        nd.lev[id] = l;
+        nd.par[id] = l == 0 ? -1 : up;
+        if (l > 0) nd.child[8 * (size_t)up + digit(key[i], 3 * (kLevels - l))] = id;
+      }
+      up = base + below + (starts ? 1 : 0) - 1;
+    }
+  }
+}
+
+// Each node's end and centre.  The end is the first key beyond lo with other
+// leading digits (doubling steps, then bisection); the centre is the root's
+// moved by a quarter of the side per level, in the order a walk from the
+// root adds them.
+__global__ __launch_bounds__(256) void k_tree_nodes(int nn, int n, const u64* __restrict__ key,
+                                                    double L, double c0, double c1, double c2,
+                                                    Nodes nd) {
 #pragma clang fp contract(off)
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int k = a + (int)(t >> 3), o = (int)(t & 7);
-  if (k >= b) return;
-  const int* e = end + 8 * (size_t)(k - a);
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k >= nn) return;
   const int lo = nd.lo[k], lev = nd.lev[k];
-  const int s0 = o == 0 ? lo : e[o - 1], s1 = e[o];
-  if (s1 <= s0) return;
-  int rank = 0;  // non-empty octants before o
-  for (int q = 0; q < o; ++q) rank += e[q] > (q == 0 ? lo : e[q - 1]);
-  const int id = b + off[k - a] + rank;
-  const double l = ldexp(L, -lev);  // L halved lev times, exactly
-  nd.lo[id] = s0;
-  nd.hi[id] = s1;
-  nd.par[id] = k;
-  nd.lev[id] = lev + 1;
-  for (int q = 0; q < 8; ++q) nd.child[8 * id + q] = -1;
-  // octant bits: x is bit 2, y bit 1, z bit 0
-  nd.c[3 * id + 0] = nd.c[3 * k + 0] + ((o & 4) ? 0.25 : -0.25) * l;
-  nd.c[3 * id + 1] = nd.c[3 * k + 1] + ((o & 2) ? 0.25 : -0.25) * l;
-  nd.c[3 * id + 2] = nd.c[3 * k + 2] + ((o & 1) ? 0.25 : -0.25) * l;
-  nd.child[8 * k + o] = id;
+  const u64 own = key[lo];
+  const int shift = 3 * (kLevels - lev);
+  int a = lo, step = 1;  // key[a] lies in the node
+  int b = n;             // key[b] does not (or b = n)
+  if (lev > 0) {
+    while (lo + step < n) {
+      if ((key[lo + step] >> shift) != (own >> shift)) {
+        b = lo + step;
+        break;
+      }
+      a = lo + step;
+      step *= 2;
+    }
+    while (b - a > 1) {
+      const int mid = a + (b - a) / 2;
+      if ((key[mid] >> shift) == (own >> shift))
+        a = mid;
+      else
+        b = mid;
+    }
+  }
+  nd.hi[k] = b;
+  double c[3] = {c0, c1, c2};
+  double l = L;
+  for (int q = 0; q < lev; ++q) {
+    const int o = digit(own, 3 * (kLevels - 1 - q));  // octant: x is bit 2, y bit 1, z bit 0
+    c[0] = c[0] + ((o & 4) ? 0.25 : -0.25) * l;
+    c[1] = c[1] + ((o & 2) ? 0.25 : -0.25) * l;
+    c[2] = c[2] + ((o & 1) ? 0.25 : -0.25) * l;
+    l *= 0.5;
+  }
+  for (int q = 0; q < 3; ++q) nd.c[3 * (size_t)k + q] = c[q];
+}
+
+__global__ __launch_bounds__(256) void k_fill_int4(size_t n4, int v, int4* __restrict__ out) {
+  const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
+  if (i < n4) out[i] = make_int4(v, v, v, v);
 }
 
 // Moments of the nodes [a, b) of one level, children already done.
@@ -452,9 +589,34 @@ __global__ void k_compact(int n, const int* __restrict__ flag, const int* __rest
   if (k < n && flag[k]) out[off[k]] = k;
 }
 
-__global__ void k_group_lo(int ng, const int* __restrict__ gnode, Nodes nd, int* __restrict__ lo) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g < ng) lo[g] = nd.lo[gnode[g]];
+// Groups by first particle: inside a level the nodes are in that order
+// already, so a group's rank is the sum over the levels of the groups that
+// start before it, by bisection.  gn: groups in node order, those of level l
+// at [off[level_start[l]], off[level_start[l + 1]]).
+struct LevelStarts {
+  int v[kLevels + 2];
+};
+__global__ __launch_bounds__(256) void k_group_order(int ng, const int* __restrict__ gn,
+                                                     const int* __restrict__ off, LevelStarts ls,
+                                                     Nodes nd, int* __restrict__ out) {
+  const int g = blockIdx.x * 256 + threadIdx.x;
+  if (g >= ng) return;
+  const int k = gn[g], lo = nd.lo[k];
+  int rank = 0;
+  for (int l = 0; l <= kLevels; ++l) {
+    if (ls.v[l] == ls.v[l + 1]) continue;
+    const int first = off[ls.v[l]];
+    int a = first, b = off[ls.v[l + 1]];
+    while (a < b) {
+      const int mid = a + (b - a) / 2;
+      if (nd.lo[gn[mid]] < lo)
+        a = mid + 1;
+      else
+        b = mid;
+    }
+    rank += a - first;
+  }
+  out[rank] = k;
 }
 
 __global__ void k_group_icnt(int ng, const int* __restrict__ gnode, Nodes nd,
@@ -909,7 +1071,7 @@ __global__ void k_pack_cells(int nc, const double* __restrict__ cells, float* __
 struct Octree {
   Nodes nd{};
   int nn = 0;
-  std::vector<int> level_start;  // level l occupies [level_start[l], level_start[l+1])
+  int level_start[kLevels + 2];  // level l occupies [level_start[l], level_start[l+1])
 };
 
 // Sorted keys, particles in Morton order and the octree.  m may be null.
@@ -928,74 +1090,51 @@ void build_octree(Build& B, Lists& R, int n, const double* x, const double* m,
   double* mm = m ? B.tmp.get<double>(n) : nullptr;
   hipLaunchKernelGGL(k_gather, grid_for(n), dim3(256), 0, st, n, perm, x, m, R.pos, mm, R.src);
   PGAMD_HIP_CHECK(hipGetLastError());
-  // node storage: grown per level (a level holds at most 8x the previous)
-  int cap = std::max(64, 2 * (n / std::max(1, split) + 1));
-  auto alloc_nodes = [&](int c) {
-    Nodes a;
-    a.lo = B.tmp.get<int>(c);
-    a.hi = B.tmp.get<int>(c);
-    a.par = B.tmp.get<int>(c);
-    a.lev = B.tmp.get<int>(c);
-    a.child = B.tmp.get<int>(8 * (size_t)c);
-    a.c = B.tmp.get<double>(3 * (size_t)c);
-    a.com = B.tmp.get<double>(3 * (size_t)c);
-    a.m = B.tmp.get<double>(c);
-    a.q = B.tmp.get<double>(6 * (size_t)c);
-    a.cell = B.tmp.get<int>(c);
-    return a;
-  };
-  T.nd = alloc_nodes(cap);
-  {
-    const int z = 0, minus1 = -1;
-    PGAMD_HIP_CHECK(hipMemcpyAsync(T.nd.lo, &z, sizeof(int), hipMemcpyHostToDevice, st));
-    PGAMD_HIP_CHECK(hipMemcpyAsync(T.nd.hi, &n, sizeof(int), hipMemcpyHostToDevice, st));
-    PGAMD_HIP_CHECK(hipMemcpyAsync(T.nd.par, &minus1, sizeof(int), hipMemcpyHostToDevice, st));
-    PGAMD_HIP_CHECK(hipMemcpyAsync(T.nd.lev, &z, sizeof(int), hipMemcpyHostToDevice, st));
-    std::vector<int> ch(8, -1);
-    PGAMD_HIP_CHECK(
-        hipMemcpyAsync(T.nd.child, ch.data(), 8 * sizeof(int), hipMemcpyHostToDevice, st));
-    const double c0[3] = {lo[0] + 0.5 * L, lo[1] + 0.5 * L, lo[2] + 0.5 * L};
-    PGAMD_HIP_CHECK(
-        hipMemcpyAsync(T.nd.c, c0, 3 * sizeof(double), hipMemcpyHostToDevice, st));
-    PGAMD_HIP_CHECK(hipStreamSynchronize(st));
+  // leaf level of every particle: the sliding maximum, in steps of at most
+  // kMaxWindow (maxima over windows of u and v give one over u + v - 1)
+  unsigned char* leaf = B.tmp.get<unsigned char>(n);
+  unsigned char* leaf2 = split > kMaxWindow ? B.tmp.get<unsigned char>(n) : nullptr;
+  const dim3 wgrid = grid_for(n, kWindowOut);
+  int left = split;  // of a window of split + 1
+  int w = std::min(left, kMaxWindow) + 1;
+  hipLaunchKernelGGL(k_window_max<true>, wgrid, dim3(256), 0, st, n, split, w, skey, nullptr, leaf);
+  for (left -= w - 1; left > 0; left -= w - 1) {
+    w = std::min(left, kMaxWindow) + 1;
+    hipLaunchKernelGGL(k_window_max<false>, wgrid, dim3(256), 0, st, n, split, w, nullptr, leaf,
+                       leaf2);
+    std::swap(leaf, leaf2);
   }
-  T.nn = 1;
-  T.level_start = {0, 1};
-  for (int lev = 0; lev < kLevels; ++lev) {
-    const int a = T.level_start[lev], b = T.level_start[lev + 1];
-    if (b == a) break;
-    int* nch = B.tmp.get<int>(b - a);
-    int* off = B.tmp.get<int>(b - a + 1);
-    int* end = B.tmp.get<int>(8 * (size_t)(b - a));
-    hipLaunchKernelGGL(k_split_count, grid_for(8LL * (b - a)), dim3(256), 0, st, a, b, T.nd, skey,
-                       split, end, nch);
-    PGAMD_HIP_CHECK(hipGetLastError());
-    const int add = B.scan(nch, off, b - a);
-    if (add == 0) {
-      T.level_start.push_back(b);
-      break;
-    }
-    if (b + add > cap) {  // grow: copy the nodes so far into larger arrays
-      int ncap = std::max(2 * cap, b + add);
-      Nodes g = alloc_nodes(ncap);
-      auto cp = [&](void* d, const void* s2, size_t bytes) {
-        PGAMD_HIP_CHECK(hipMemcpyAsync(d, s2, bytes, hipMemcpyDeviceToDevice, st));
-      };
-      cp(g.lo, T.nd.lo, b * sizeof(int));
-      cp(g.hi, T.nd.hi, b * sizeof(int));
-      cp(g.par, T.nd.par, b * sizeof(int));
-      cp(g.lev, T.nd.lev, b * sizeof(int));
-      cp(g.child, T.nd.child, 8 * (size_t)b * sizeof(int));
-      cp(g.c, T.nd.c, 3 * (size_t)b * sizeof(double));
-      T.nd = g;
-      cap = ncap;
-    }
-    hipLaunchKernelGGL(k_split_fill, grid_for(8LL * (b - a)), dim3(256), 0, st, a, b, T.nd, end,
-                       off, L);
-    PGAMD_HIP_CHECK(hipGetLastError());
-    T.level_start.push_back(b + add);
-    T.nn = b + add;
-  }
+  PGAMD_HIP_CHECK(hipGetLastError());
+  const int nb = (int)grid_for(n, kTreeBlock).x;
+  int* count = B.tmp.get<int>((size_t)kTreeLevels * nb);
+  int* first = B.tmp.get<int>((size_t)kTreeLevels * nb + 1);
+  hipLaunchKernelGGL(k_tree_count, dim3(nb), dim3(256), 0, st, n, skey, leaf, count);
+  PGAMD_HIP_CHECK(hipGetLastError());
+  B.scan_async(count, first, kTreeLevels * nb);
+  int* host = scan_total_host();
+  hipLaunchKernelGGL(k_tree_levels, dim3(1), dim3(64), 0, st, nb, count, first, host_dev(host));
+  PGAMD_HIP_CHECK(hipGetLastError());
+  PGAMD_HIP_CHECK(hipStreamSynchronize(st));
+  for (int l = 0; l < kLevels + 2; ++l) T.level_start[l] = static_cast<volatile int*>(host)[l];
+  T.nn = T.level_start[kLevels + 1];
+  Nodes& nd = T.nd;
+  const size_t c = (size_t)T.nn;
+  nd.lo = B.tmp.get<int>(c);
+  nd.hi = B.tmp.get<int>(c);
+  nd.par = B.tmp.get<int>(c);
+  nd.lev = B.tmp.get<int>(c);
+  nd.child = B.tmp.get<int>(8 * c);
+  nd.c = B.tmp.get<double>(3 * c);
+  nd.com = B.tmp.get<double>(3 * c);
+  nd.m = B.tmp.get<double>(c);
+  nd.q = B.tmp.get<double>(6 * c);
+  nd.cell = B.tmp.get<int>(c);
+  hipLaunchKernelGGL(k_fill_int4, grid_for(2 * c), dim3(256), 0, st, 2 * c, -1,
+                     reinterpret_cast<int4*>(nd.child));
+  hipLaunchKernelGGL(k_tree_fill, dim3(nb), dim3(256), 0, st, n, skey, leaf, first, nd);
+  hipLaunchKernelGGL(k_tree_nodes, grid_for(T.nn), dim3(256), 0, st, T.nn, n, skey, L,
+                     lo[0] + 0.5 * L, lo[1] + 0.5 * L, lo[2] + 0.5 * L, nd);
+  PGAMD_HIP_CHECK(hipGetLastError());
   *skey_out = skey;
   *mm_out = mm;
 }
@@ -1011,12 +1150,12 @@ int build_groups(Build& B, Lists& R, const Octree& T, int ncrit, int** gnode_out
   const int ng = B.scan(flag, off, nn);
   int* gn = B.tmp.get<int>(ng);
   int* gn_sorted = B.tmp.get<int>(ng);
-  int* lo = B.tmp.get<int>(ng);
-  int* lo_sorted = B.tmp.get<int>(ng);
   hipLaunchKernelGGL(k_compact, grid_for(nn), dim3(256), 0, st, nn, flag, off, gn);
-  hipLaunchKernelGGL(k_group_lo, grid_for(ng), dim3(256), 0, st, ng, gn, T.nd, lo);
+  LevelStarts ls;
+  for (int l = 0; l < kLevels + 2; ++l) ls.v[l] = T.level_start[l];
+  hipLaunchKernelGGL(k_group_order, grid_for(ng), dim3(256), 0, st, ng, gn, off, ls, T.nd,
+                     gn_sorted);
   PGAMD_HIP_CHECK(hipGetLastError());
-  B.sort_pairs(lo, lo_sorted, gn, gn_sorted, ng, 31);
   R.ng = ng;
   R.icnt = R.mem.get<int>(ng);
   R.ioff = R.mem.get<int>(ng + 1);
@@ -1155,11 +1294,10 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   double* mm = nullptr;
   build_octree(B, *R, n, x, m, lo, L, std::max(1, std::min(ncrit, nleaf)), T, &skey, &mm);
   // moments, deepest level first
-  for (int lev = (int)T.level_start.size() - 2; lev >= 0; --lev) {
+  for (int lev = kLevels; lev >= 0; --lev) {
     const int a = T.level_start[lev], b = T.level_start[lev + 1];
-    if (b > a)
-      hipLaunchKernelGGL(k_moments, grid_for(b - a, 64), dim3(64), 0, st, a, b, T.nd, R->pos,
-                         mm);
+    if (b == a) continue;
+    hipLaunchKernelGGL(k_moments, grid_for(b - a, 64), dim3(64), 0, st, a, b, T.nd, R->pos, mm);
     PGAMD_HIP_CHECK(hipGetLastError());
   }
   // cells: nodes with more than one particle, in node order
