@@ -424,29 +424,35 @@ __global__ void k_tree_levels(int nb, const int* __restrict__ count, const int* 
 __global__ __launch_bounds__(256) void k_tree_fill(int n, const u64* __restrict__ key,
                                                    const unsigned char* __restrict__ leaf,
                                                    const int* __restrict__ first, Nodes nd) {
-  __shared__ int s_cnt[kTreeRounds][4][kTreeLevels];
-  __shared__ int s_first[kTreeLevels];
+  // number of the first node of each level in wavefront 4 r + wave's particles
+  __shared__ int s_at[4 * kTreeRounds][kTreeLevels];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (threadIdx.x < kTreeLevels) s_first[threadIdx.x] = first[threadIdx.x * gridDim.x + blockIdx.x];
   int a[kTreeRounds], d[kTreeRounds];
 #pragma unroll
   for (int r = 0; r < kTreeRounds; ++r) {
     start_levels(blockIdx.x * kTreeBlock + r * 256 + threadIdx.x, n, key, leaf, &a[r], &d[r]);
     for (int l = 0; l < kTreeLevels; ++l) {
       const int c = __popcll(__ballot(a[r] <= l && l <= d[r]));
-      if (lane == l) s_cnt[r][wave][l] = c;
+      if (lane == l) s_at[4 * r + wave][l] = c;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < kTreeLevels) {
+    int run = first[threadIdx.x * gridDim.x + blockIdx.x];
+    for (int q = 0; q < 4 * kTreeRounds; ++q) {
+      const int c = s_at[q][threadIdx.x];
+      s_at[q][threadIdx.x] = run;
+      run += c;
     }
   }
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < kTreeRounds; ++r) {
     const int i = blockIdx.x * kTreeBlock + r * 256 + threadIdx.x;
+    const u64 own = i < n ? key[i] : 0;
     int up = 0;  // the last node of the level above that starts at or before i
     for (int l = 0; l < kTreeLevels; ++l) {
-      int base = s_first[l];
-      for (int q = 0; q < r; ++q)
-        base += s_cnt[q][0][l] + s_cnt[q][1][l] + s_cnt[q][2][l] + s_cnt[q][3][l];
-      for (int q = 0; q < wave; ++q) base += s_cnt[r][q][l];
+      const int base = s_at[4 * r + wave][l];
       const bool starts = a[r] <= l && l <= d[r];
       const u64 m = __ballot(starts);
       const int below = __popcll(m & ((1ULL << lane) - 1ULL));
@@ -455,7 +461,7 @@ __global__ __launch_bounds__(256) void k_tree_fill(int n, const u64* __restrict_
         nd.lo[id] = i;
         nd.lev[id] = l;
         nd.par[id] = l == 0 ? -1 : up;
-        if (l > 0) nd.child[8 * (size_t)up + digit(key[i], 3 * (kLevels - l))] = id;
+        if (l > 0) nd.child[8 * (size_t)up + digit(own, 3 * (kLevels - l))] = id;
       }
       up = base + below + (starts ? 1 : 0) - 1;
     }
@@ -507,68 +513,114 @@ __global__ __launch_bounds__(256) void k_tree_nodes(int nn, int n, const u64* __
   for (int q = 0; q < 3; ++q) nd.c[3 * (size_t)k + q] = c[q];
 }
 
+__global__ void k_fill_int(int n, int v, int* __restrict__ out) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) out[i] = v;
+}
+
+__global__ void k_copy_ints(int n, const int* __restrict__ in, int* __restrict__ out) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) out[i] = in[i];
+}
+
 __global__ __launch_bounds__(256) void k_fill_int4(size_t n4, int v, int4* __restrict__ out) {
   const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
   if (i < n4) out[i] = make_int4(v, v, v, v);
 }
 
-// Moments of the nodes [a, b) of one level, children already done.
-__global__ void k_moments(int a, int b, Nodes nd, const double* __restrict__ pos,
-                          const double* __restrict__ mm) {
+// Moments of one node; q[5] follows from the trace.
+__device__ inline void store_moments(const Nodes& nd, int k, double M, const double com[3],
+                                     double q[6]) {
 #pragma clang fp contract(off)
-  const int k = a + blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= b) return;
-  bool leaf = true;
-  for (int o = 0; o < 8; ++o) leaf = leaf && nd.child[8 * k + o] < 0;
-  double M = 0, c[3] = {0, 0, 0}, q[6] = {0, 0, 0, 0, 0, 0}, com[3];
-  if (leaf) {
-    for (int p = nd.lo[k]; p < nd.hi[k]; ++p) {
-      const double mi = mm ? mm[p] : 1.0;
-      M += mi;
-      for (int d = 0; d < 3; ++d) c[d] += mi * pos[3 * p + d];
-    }
-    for (int d = 0; d < 3; ++d) com[d] = M > 0 ? c[d] / M : nd.c[3 * k + d];
-    for (int p = nd.lo[k]; p < nd.hi[k]; ++p) {
-      const double mi = mm ? mm[p] : 1.0;
-      double dd[3];
-      for (int d = 0; d < 3; ++d) dd[d] = pos[3 * p + d] - com[d];
-      const double r2 = dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2];
-      int kk = 0;
-      for (int x = 0; x < 2; ++x)
-        for (int y = x; y < 3; ++y) {
-          double v = 3.0 * dd[x] * dd[y];
-          if (x == y) v -= r2;
-          q[kk++] += mi * v;
-        }
-    }
-  } else {
-    for (int o = 0; o < 8; ++o) {
-      const int ch = nd.child[8 * k + o];
-      if (ch < 0) continue;
-      M += nd.m[ch];
-      for (int d = 0; d < 3; ++d) c[d] += nd.m[ch] * nd.com[3 * ch + d];
-    }
-    for (int d = 0; d < 3; ++d) com[d] = M > 0 ? c[d] / M : nd.c[3 * k + d];
-    for (int o = 0; o < 8; ++o) {
-      const int ch = nd.child[8 * k + o];
-      if (ch < 0) continue;
-      double dd[3];
-      for (int d = 0; d < 3; ++d) dd[d] = nd.com[3 * ch + d] - com[d];
-      const double r2 = dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2];
-      int kk = 0;
-      for (int x = 0; x < 2; ++x)
-        for (int y = x; y < 3; ++y) {
-          double v = 3.0 * dd[x] * dd[y];
-          if (x == y) v -= r2;
-          q[kk] += nd.q[6 * ch + kk] + nd.m[ch] * v;
-          ++kk;
-        }
-    }
-  }
   nd.m[k] = M;
-  for (int d = 0; d < 3; ++d) nd.com[3 * k + d] = com[d];
+  for (int d = 0; d < 3; ++d) nd.com[3 * (size_t)k + d] = com[d];
   q[5] = -(q[0] + q[3]);
-  for (int t = 0; t < 6; ++t) nd.q[6 * k + t] = q[t];
+  for (int t = 0; t < 6; ++t) nd.q[6 * (size_t)k + t] = q[t];
+}
+
+__device__ inline bool is_leaf(const Nodes& nd, int k) {
+  const int4* c = reinterpret_cast<const int4*>(nd.child + 8 * (size_t)k);
+  const int4 a = c[0], b = c[1];
+  return (a.x & a.y & a.z & a.w & b.x & b.y & b.z & b.w) < 0;  // no child: all are -1
+}
+
+// Moments of every leaf: sums over its particles in order.
+__global__ __launch_bounds__(256) void k_leaf_moments(int nn, Nodes nd,
+                                                      const double* __restrict__ pos,
+                                                      const double* __restrict__ mm) {
+#pragma clang fp contract(off)
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k >= nn || !is_leaf(nd, k)) return;
+  const int lo = nd.lo[k], hi = nd.hi[k];
+  double M = 0, c[3] = {0, 0, 0}, q[6] = {0, 0, 0, 0, 0, 0}, com[3];
+  for (int p = lo; p < hi; ++p) {
+    const double mi = mm ? mm[p] : 1.0;
+    M += mi;
+    for (int d = 0; d < 3; ++d) c[d] += mi * pos[3 * (size_t)p + d];
+  }
+  for (int d = 0; d < 3; ++d) com[d] = M > 0 ? c[d] / M : nd.c[3 * (size_t)k + d];
+  for (int p = lo; p < hi; ++p) {
+    const double mi = mm ? mm[p] : 1.0;
+    double dd[3];
+    for (int d = 0; d < 3; ++d) dd[d] = pos[3 * (size_t)p + d] - com[d];
+    const double r2 = dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2];
+    int kk = 0;
+    for (int x = 0; x < 2; ++x)
+      for (int y = x; y < 3; ++y) {
+        double v = 3.0 * dd[x] * dd[y];
+        if (x == y) v -= r2;
+        q[kk++] += mi * v;
+      }
+  }
+  store_moments(nd, k, M, com, q);
+}
+
+// Moments of node k from its children's, in octant order.
+__device__ inline void combine_moments(const Nodes& nd, int k) {
+#pragma clang fp contract(off)
+  if (is_leaf(nd, k)) return;
+  double M = 0, c[3] = {0, 0, 0}, q[6] = {0, 0, 0, 0, 0, 0}, com[3];
+  for (int o = 0; o < 8; ++o) {
+    const int ch = nd.child[8 * (size_t)k + o];
+    if (ch < 0) continue;
+    M += nd.m[ch];
+    for (int d = 0; d < 3; ++d) c[d] += nd.m[ch] * nd.com[3 * (size_t)ch + d];
+  }
+  for (int d = 0; d < 3; ++d) com[d] = M > 0 ? c[d] / M : nd.c[3 * (size_t)k + d];
+  for (int o = 0; o < 8; ++o) {
+    const int ch = nd.child[8 * (size_t)k + o];
+    if (ch < 0) continue;
+    double dd[3];
+    for (int d = 0; d < 3; ++d) dd[d] = nd.com[3 * (size_t)ch + d] - com[d];
+    const double r2 = dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2];
+    int kk = 0;
+    for (int x = 0; x < 2; ++x)
+      for (int y = x; y < 3; ++y) {
+        double v = 3.0 * dd[x] * dd[y];
+        if (x == y) v -= r2;
+        q[kk] += nd.q[6 * (size_t)ch + kk] + nd.m[ch] * v;
+        ++kk;
+      }
+  }
+  store_moments(nd, k, M, com, q);
+}
+
+// The inner nodes [a, b) of one level, children already done.
+__global__ __launch_bounds__(64) void k_inner_moments(int a, int b, Nodes nd) {
+  const int k = a + blockIdx.x * 64 + threadIdx.x;
+  if (k < b) combine_moments(nd, k);
+}
+
+// The first levels' inner nodes in one block, level `top` - 1 first.
+struct LevelStarts {
+  int v[kLevels + 2];
+};
+constexpr int kTopNodes = 512;  // a level this small is left to the one block
+__global__ __launch_bounds__(kTopNodes) void k_top_moments(int top, LevelStarts ls, Nodes nd) {
+  for (int l = top - 1; l >= 0; --l) {
+    const int k = ls.v[l] + threadIdx.x;
+    if (k < ls.v[l + 1]) combine_moments(nd, k);
+    __threadfence_block();
+    __syncthreads();
+  }
 }
 
 // i-groups: nodes of <= ncrit particles whose parent holds more, and nodes
@@ -591,22 +643,22 @@ __global__ void k_compact(int n, const int* __restrict__ flag, const int* __rest
 
 // Groups by first particle: inside a level the nodes are in that order
 // already, so a group's rank is the sum over the levels of the groups that
-// start before it, by bisection.  gn: groups in node order, those of level l
-// at [off[level_start[l]], off[level_start[l + 1]]).
-struct LevelStarts {
-  int v[kLevels + 2];
-};
+// start before it, by bisection, a lane per level (32 lanes per group).  gn:
+// groups in node order, those of level l at [off[level.v[l]],
+// off[level.v[l + 1]]).
 __global__ __launch_bounds__(256) void k_group_order(int ng, const int* __restrict__ gn,
                                                      const int* __restrict__ off, LevelStarts ls,
                                                      Nodes nd, int* __restrict__ out) {
-  const int g = blockIdx.x * 256 + threadIdx.x;
-  if (g >= ng) return;
+  __shared__ int s_first[kLevels + 2];
+  if (threadIdx.x < kLevels + 2) s_first[threadIdx.x] = off[ls.v[threadIdx.x]];
+  __syncthreads();
+  const int g = blockIdx.x * 8 + threadIdx.x / 32, l = threadIdx.x % 32;
+  if (g >= ng) return;  // uniform per 32 lanes
   const int k = gn[g], lo = nd.lo[k];
   int rank = 0;
-  for (int l = 0; l <= kLevels; ++l) {
-    if (ls.v[l] == ls.v[l + 1]) continue;
-    const int first = off[ls.v[l]];
-    int a = first, b = off[ls.v[l + 1]];
+  if (l <= kLevels) {
+    const int first = s_first[l];
+    int a = first, b = s_first[l + 1];
     while (a < b) {
       const int mid = a + (b - a) / 2;
       if (nd.lo[gn[mid]] < lo)
@@ -614,9 +666,10 @@ __global__ __launch_bounds__(256) void k_group_order(int ng, const int* __restri
       else
         b = mid;
     }
-    rank += a - first;
+    rank = a - first;
   }
-  out[rank] = k;
+  for (int o = 16; o > 0; o >>= 1) rank += __shfl_xor(rank, o, 32);
+  if (l == 0) out[rank] = k;
 }
 
 __global__ void k_group_icnt(int ng, const int* __restrict__ gnode, Nodes nd,
@@ -872,36 +925,58 @@ __device__ inline double bh_box_d2(const double* __restrict__ gc, double li,
   return d2;
 }
 
-// Node data the Barnes-Hut walk reads for one child, in one 64-byte record:
-// centre of mass, particle range, cell index (nodes of more than one
-// particle) and the children as the first child's index plus an octant mask
-// (the children of a node are numbered consecutively in octant order).
-struct WalkNode {
-  int lo, hi, cell, first, mask, pad[3];
-  double com[3], pad2;
+// Node data the Barnes-Hut walk reads for one child: what it becomes if it is
+// opened, and its centre of mass (32 bytes), and for the lists its particle
+// range and cell index (nodes of more than one particle).  Arrays of 16 bytes
+// a node: the eight lanes that examine a node's children (numbered
+// consecutively in octant order) read 128 consecutive bytes of each, where
+// 64-byte records made every lane of every load a cache line of its own; the
+// walk is bound by the lookups and misses of the vector cache.
+struct WalkNodes {
+  int4* range;  // {lo, hi, cell, 0}
+  // {x, y} of the queue entry (below) and com x as two words
+  int4* ex;
+  double2* yz;  // com y, z
 };
-static_assert(sizeof(WalkNode) == 64, "one record per 64 bytes");
 
-__global__ void k_walk_nodes(int nn, Nodes nd, WalkNode* __restrict__ out) {
+// A node to be expanded: {first child, octant mask}, or a leaf (a node of up
+// to nleaf particles or one that the key cannot split), whose particles are
+// listed one by one: {lo, kLeafEntry | count}.
+constexpr unsigned kLeafEntry = 0x80000000u;
+
+struct WalkNode {
+  int x;
+  unsigned y;
+  double com[3];
+  __device__ inline bool leaf() const { return y & kLeafEntry; }
+  __device__ inline int count() const { return (int)(y & ~kLeafEntry); }  // of a leaf
+};
+
+__device__ inline WalkNode load_walk(const WalkNodes& w, int k) {
+  const int4 e = w.ex[k];
+  const double2 yz = w.yz[k];
+  return WalkNode{e.x, (unsigned)e.y,
+                  {__longlong_as_double((long long)((u64)(unsigned)e.w << 32 | (unsigned)e.z)), yz.x, yz.y}};
+}
+
+__global__ void k_walk_nodes(int nn, int nleaf, Nodes nd, WalkNodes out) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= nn) return;
-  WalkNode w;
-  for (int d = 0; d < 3; ++d) w.com[d] = nd.com[3 * k + d];
-  w.lo = nd.lo[k];
-  w.hi = nd.hi[k];
-  w.cell = w.hi - w.lo > 1 ? nd.cell[k] : -1;
-  w.first = -1;
-  w.mask = 0;
+  const int lo = nd.lo[k], hi = nd.hi[k];
+  int first = -1, mask = 0;
   for (int o = 7; o >= 0; --o) {
     const int ch = nd.child[8 * k + o];
     if (ch >= 0) {
-      w.first = ch;
-      w.mask |= 1 << o;
+      first = ch;
+      mask |= 1 << o;
     }
   }
-  w.pad[0] = w.pad[1] = w.pad[2] = 0;
-  w.pad2 = 0.0;
-  out[k] = w;
+  const bool leaf = hi - lo <= nleaf || mask == 0;
+  const u64 cx = (u64)__double_as_longlong(nd.com[3 * k]);
+  out.range[k] = make_int4(lo, hi, hi - lo > 1 ? nd.cell[k] : -1, 0);
+  out.ex[k] = make_int4(leaf ? lo : first, leaf ? (int)(kLeafEntry | (unsigned)(hi - lo)) : mask,
+                        (int)(unsigned)cx, (int)(unsigned)(cx >> 32));
+  out.yz[k] = make_double2(nd.com[3 * k + 1], nd.com[3 * k + 2]);
 }
 
 // Depth of the walk stack: the depth-first walk keeps at most 7 pending
@@ -918,6 +993,340 @@ __device__ inline int xcd_block(int b, int nb) {
   return x < r ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
 }
 
+// The host builder's walk (source.cpp:832-867) lists, for an opened node, its
+// children in octant order 7..0 (singletons and accepted cells), then what
+// its opened children list, octant 0 first.  The order of the lists is that
+// of a depth-first walk, but which nodes are opened does not depend on it:
+// k_bh_open (a wavefront per group) opens nodes breadth first, 8 queue entries
+// (64 children) a step and every one of them kept, and k_bh_list (a block per
+// group) sums what each entry's subtree lists and from it where its own
+// particles and cells go.  A depth-first walk can keep only the work of the
+// stack entries before the first one that opens children, and runs twice, the
+// first time for the list lengths: 0.67 + 0.81 ms for 2^21 particles at
+// theta = 0.5 (14029 groups that open 793 nodes on average), against 0.63 +
+// 0.31 ms.  Bound: the vector cache, whose lookups and misses of the
+// children's loads (64 lanes of 32 bytes a step) a step waits for.
+//
+// Leaves need no examining and go to the pool as they are found; the other
+// entries wait for their turn in a ring in LDS (those beyond its kOpenRing
+// places in their pool entry), so that a step's chain is one LDS read and the
+// children's loads.
+//
+// Entries live in chunks of a pool, handed to the groups as they need them:
+// {first child, masks, entry of the first opened child, 0}, masks: bits 0-7
+// children, 8-15 those that are single particles, 16-23 accepted cells (the
+// rest are opened); or a leaf.
+constexpr int kOpenChunk = 256;       // entries per chunk
+constexpr int kOpenGroupChunks = 64;  // per group at most: 14 bits of entry index
+constexpr int kOpenRing = 512;        // queued entries in LDS per wavefront
+constexpr int kOpenLevels = kLevels + 3;
+
+struct OpenPool {
+  int4* rec;    // [chunks][kOpenChunk]
+  int4* sum;    // the same: k_bh_list's working entries of groups too large for LDS
+  int* wait;    // the same: the entry at a ring position beyond the ring
+  int* used;    // [0] chunks handed out, [1] != 0: the pool or a group's table was too small,
+                // [2] != 0: some group is too large for k_bh_list's LDS
+  int* chunk;   // [group][kOpenGroupChunks]
+  int* level;   // [group][kOpenLevels]: first entry of each level, then the number of
+                // entries; the last int is the number of levels (0: no entries)
+  int chunks;
+};
+
+// Opened children, own particles and own cells of an entry.
+__device__ inline int open_count(unsigned b) {
+  return b & kLeafEntry ? 0 : __popc(b & 0xffu & ~(b >> 8) & ~(b >> 16));
+}
+__device__ inline int own_particles(unsigned b) {
+  return b & kLeafEntry ? (int)(b & ~kLeafEntry) : __popc(b & 0xff00u);
+}
+__device__ inline int own_cells(unsigned b) {
+  return b & kLeafEntry ? 0 : __popc(b & 0xff0000u);
+}
+
+constexpr int kListThreads = 256;
+constexpr int kListEntries = 1536;  // entries of a group that k_bh_list holds in LDS
+
+__global__ __launch_bounds__(64 * kWalkWaves) void k_bh_open(
+    int ng, const int* __restrict__ gnode, Nodes nd, WalkNodes wn, double L,
+    double th2, OpenPool pool, int* __restrict__ pcnt, int* __restrict__ ccnt) {
+#pragma clang fp contract(off)
+  __shared__ int s_chunk[kWalkWaves][kOpenGroupChunks];
+  // {first child, mask | level << 8 | entry << 13}
+  __shared__ int2 s_ring[kWalkWaves][kOpenRing];
+  const int lane = threadIdx.x & 63;
+  const int g = xcd_block(blockIdx.x, gridDim.x) * kWalkWaves + (threadIdx.x >> 6);
+  if (g >= ng) return;  // uniform per wavefront
+  int* chunk = s_chunk[threadIdx.x >> 6];
+  int2* ring = s_ring[threadIdx.x >> 6];
+  int* level = pool.level + (size_t)g * kOpenLevels;
+  const int gk = gnode[g];
+  const double gc[3] = {nd.c[3 * gk], nd.c[3 * gk + 1], nd.c[3 * gk + 2]};
+  const double li = 0.5 * ldexp(L, -nd.lev[gk]);
+  const WalkNode root = load_walk(wn, 0);
+  // the whole tree as one cell (source.cpp:832-840): no entries
+  if (bh_box_d2(gc, li, root.com) * th2 >= L * L) {
+    if (lane == 0) {
+      pcnt[g] = 0;
+      ccnt[g] = 1;
+      level[kOpenLevels - 1] = 0;
+    }
+    return;
+  }
+  int nch = 0;
+  // one more chunk for this group; false: none left
+  auto grow = [&]() {
+    int c = 0;
+    if (lane == 0) c = atomicAdd(&pool.used[0], 1);
+    c = __builtin_amdgcn_readfirstlane(c);
+    if (nch == kOpenGroupChunks || c >= pool.chunks) {
+      if (lane == 0) {
+        pool.used[1] = 1;
+        pcnt[g] = 0;
+        ccnt[g] = 0;
+        level[kOpenLevels - 1] = 0;
+      }
+      return false;
+    }
+    if (lane == 0) {
+      chunk[nch] = c;
+      pool.chunk[(size_t)g * kOpenGroupChunks + nch] = c;
+    }
+    ++nch;
+    return true;
+  };
+  auto at = [&](int k) { return (size_t)chunk[k / kOpenChunk] * kOpenChunk + k % kOpenChunk; };
+  // order LDS, or LDS and pool, writes before the reads of the wavefront's
+  // other lanes
+  auto lds_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  auto sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  };
+  if (!grow()) return;
+  lds_sync();
+  int np = 0, nc = 0;         // listed particles (leaves: this lane's) and cells
+  int tail = 1;               // entries
+  int head = 0, waiting = 1;  // ring positions: next to examine, end
+  if (root.leaf()) {
+    if (lane == 0) {
+      np = root.count();
+      pool.rec[at(0)] = make_int4(root.x, (int)root.y, 0, 0);
+    }
+    waiting = 0;
+  } else if (lane == 0) {
+    ring[0] = make_int2(root.x, (int)root.y);
+  }
+  // next = ring position of the first entry of the newest level
+  int nlev = 1, next = 0;
+  if (lane == 0) level[0] = 0;
+  const int e = lane >> 3, o = lane & 7;
+  while (head < waiting) {
+    lds_sync();
+    const int npop = min(8, waiting - head);
+    const bool valid = e < npop;
+    const int2 r = valid ? ring[(head + e) % kOpenRing] : make_int2(0, 0);
+    const unsigned b = (unsigned)r.y;
+    int kind = 0;  // 1 particle, 2 cell, 3 opened
+    WalkNode w{0, 0u, {0.0, 0.0, 0.0}};
+    const int lev = (int)(b >> 8 & 31u);
+    if ((b >> o) & 1u) {
+      const double l = ldexp(L, -lev);
+      const double s2 = 0.25 * l * l;  // child side squared
+      w = load_walk(wn, r.x + __popc(b & ((1u << o) - 1u)));
+      if (w.y == (kLeafEntry | 1u))
+        kind = 1;
+      else if (bh_box_d2(gc, li, w.com) * th2 > s2)
+        kind = 2;
+      else
+        kind = 3;
+    }
+    const bool inner = kind == 3 && !w.leaf();
+    const u64 mp = __ballot(kind == 1), mc = __ballot(kind == 2), ms = __ballot(kind == 3);
+    const u64 mi = __ballot(inner);
+    const u64 below = (1ULL << lane) - 1ULL;
+    const int opened = __popcll(ms);
+    while ((tail + opened - 1) / kOpenChunk >= nch) {
+      if (!grow()) return;
+      lds_sync();
+    }
+    head += npop;
+    if (kind == 1) ++np;
+    if (kind == 2) ++nc;
+    if (kind == 3) {
+      const int k = tail + __popcll(ms & below);
+      if (inner) {
+        const int q = waiting + __popcll(mi & below);
+        const int2 v = make_int2(w.x, (int)w.y | (lev + 1) << 8 | k << 13);
+        if (q < head + kOpenRing) {
+          ring[q % kOpenRing] = v;
+        } else {
+          pool.rec[at(k)] = make_int4(v.x, v.y, 0, 0);
+          pool.wait[at(q)] = k;
+        }
+      } else {
+        pool.rec[at(k)] = make_int4(w.x, (int)w.y, 0, 0);
+        np += w.count();
+      }
+    }
+    // places freed by this step, for entries that have waited in the pool
+    if (waiting > head - npop + kOpenRing) {
+      sync();
+      const int q = head - npop + kOpenRing + lane;
+      if (lane < npop && q < waiting) {
+        const int4 v = pool.rec[at(pool.wait[at(q)])];
+        ring[q % kOpenRing] = make_int2(v.x, v.y);
+      }
+    }
+    if (valid && o == 0) {
+      const unsigned m1 = (unsigned)(mp >> (8 * e)) & 0xffu, m2 = (unsigned)(mc >> (8 * e)) & 0xffu;
+      pool.rec[at((int)(b >> 13))] = make_int4(r.x, (int)((b & 0xffu) | m1 << 8 | m2 << 16),
+                                               tail + __popcll(ms & below), 0);
+    }
+    // a level's entries start where the first entry examined of the level
+    // before put its opened children
+    if (next < head) {
+      const u64 before = (1ULL << (8 * (next - head + npop))) - 1ULL;
+      if (lane == 0) level[nlev] = tail + __popcll(ms & before);
+      ++nlev;
+      next = waiting + __popcll(mi & before);
+    }
+    waiting += __popcll(mi);
+    tail += opened;
+  }
+  for (int d = 32; d > 0; d >>= 1) {
+    np += __shfl_xor(np, d);
+    nc += __shfl_xor(nc, d);
+  }
+  if (lane == 0) {
+    level[nlev] = tail;  // (the deepest level may have no entries)
+    level[kOpenLevels - 1] = nlev;
+    pcnt[g] = np;
+    ccnt[g] = nc;
+    if (tail > kListEntries) pool.used[2] = 1;
+  }
+}
+
+// The lists of k_bh_open's groups, one block each: the entries of a level
+// after the other, first deepest to root for what each entry's subtree lists,
+// then root to deepest for where each entry's particles and cells go, then
+// the lists, eight lanes per entry.  The working entries {masks, first opened
+// child, particles, cells} are in LDS, or (BIG) for groups of more than
+// kListEntries in the pool.
+template <bool BIG>
+__global__ __launch_bounds__(kListThreads) void k_bh_list(
+    int ng, OpenPool pool, const int4* __restrict__ range, const int* __restrict__ poff,
+    const int* __restrict__ coff, int* __restrict__ plist, int* __restrict__ clist) {
+  __shared__ int4 s_ent[BIG ? 1 : kListEntries];
+  __shared__ int s_x[BIG ? 1 : kListEntries];  // first child or particle
+  __shared__ int s_chunk[kOpenGroupChunks], s_level[kOpenLevels];
+  const int g = xcd_block(blockIdx.x, gridDim.x);
+  const int tid = threadIdx.x;
+  if (tid < kOpenLevels) s_level[tid] = pool.level[(size_t)g * kOpenLevels + tid];
+  if (tid < kOpenGroupChunks) s_chunk[tid] = pool.chunk[(size_t)g * kOpenGroupChunks + tid];
+  __syncthreads();
+  const int nlev = s_level[kOpenLevels - 1];
+  if (nlev == 0) return;  // uniform
+  const int n = s_level[nlev];
+  if (BIG != (n > kListEntries)) return;  // uniform
+  auto at = [&](int k) { return (size_t)s_chunk[k / kOpenChunk] * kOpenChunk + k % kOpenChunk; };
+  auto ent = [&](int k) -> int4& { return BIG ? pool.sum[at(k)] : s_ent[k]; };
+  for (int k = tid; k < n; k += kListThreads) {
+    const int4 r = pool.rec[at(k)];
+    const unsigned b = (unsigned)r.y;
+    ent(k) = make_int4(r.y, r.z, own_particles(b), own_cells(b));
+    if (!BIG) s_x[k] = r.x;
+  }
+  __syncthreads();
+  for (int v = nlev - 1; v >= 0; --v) {
+    for (int k = s_level[v] + tid; k < s_level[v + 1]; k += kListThreads) {
+      int4 r = ent(k);
+      const int m = open_count((unsigned)r.x);
+      for (int c = 0; c < m; ++c) {
+        const int4 t = ent(r.y + c);
+        r.z += t.z;
+        r.w += t.w;
+      }
+      if (m) ent(k) = r;
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    int4& r = ent(0);
+    r.z = 0;
+    r.w = 0;
+  }
+  __syncthreads();
+  for (int v = 0; v < nlev; ++v) {
+    for (int k = s_level[v] + tid; k < s_level[v + 1]; k += kListThreads) {
+      const int4 r = ent(k);
+      const unsigned b = (unsigned)r.x;
+      const int m = open_count(b);
+      int np = r.z + own_particles(b), nc = r.w + own_cells(b);
+      for (int c = 0; c < m; ++c) {
+        int4& t = ent(r.y + c);
+        const int tp = t.z, tc = t.w;
+        t.z = np;
+        t.w = nc;
+        np += tp;
+        nc += tc;
+      }
+    }
+    __syncthreads();
+  }
+  int* pl = plist + poff[g];
+  int* cl = clist + coff[g];
+  const int o = tid & 7;
+  const unsigned above = 0xffu & ~((2u << o) - 1u);  // octants listed before this one
+  for (int k0 = tid >> 3; k0 < n; k0 += 4 * (kListThreads / 8)) {
+    int4 r[4], w[4];
+    int x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {  // four entries' loads in flight
+      const int k = k0 + u * (kListThreads / 8);
+      r[u] = k < n ? ent(k) : make_int4(0, 0, 0, 0);
+      x[u] = k < n ? (BIG ? pool.rec[at(k)].x : s_x[k]) : 0;
+      const unsigned b = (unsigned)r[u].x;
+      if (!(b & kLeafEntry) && (((b >> 8 | b >> 16) >> o) & 1u))
+        w[u] = range[x[u] + __popc(b & ((1u << o) - 1u))];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const unsigned b = (unsigned)r[u].x, m1 = b >> 8 & 0xffu, m2 = b >> 16 & 0xffu;
+      if (b & kLeafEntry) {
+        const int cnt = (int)(b & ~kLeafEntry);
+        for (int p = o; p < cnt; p += 8) pl[r[u].z + p] = x[u] + p;
+      } else if ((m1 >> o) & 1u) {
+        pl[r[u].z + __popc(m1 & above)] = w[u].x;
+      } else if ((m2 >> o) & 1u) {
+        cl[r[u].w + __popc(m2 & above)] = w[u].z;
+      }
+    }
+  }
+}
+
+// Lists of one cell, the whole tree (groups that k_bh_open gave no entries).
+__global__ void k_bh_whole(int ng, const int* __restrict__ pcnt, const int* __restrict__ ccnt,
+                           WalkNodes wn, const int* __restrict__ coff,
+                           const int* __restrict__ gnode, Nodes nd, double L, double th2,
+                           int* __restrict__ clist) {
+#pragma clang fp contract(off)
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= ng || pcnt[g] != 0 || ccnt[g] != 1) return;
+  const int gk = gnode[g];
+  const double gc[3] = {nd.c[3 * gk], nd.c[3 * gk + 1], nd.c[3 * gk + 2]};
+  if (bh_box_d2(gc, 0.5 * ldexp(L, -nd.lev[gk]), load_walk(wn, 0).com) * th2 >= L * L)
+    clist[coff[g]] = wn.range[0].z;
+}
+
+// For builds whose groups open more nodes than k_bh_open's pool or chunk
+// tables hold (small theta).
+//
 // One wavefront per group: the depth-first walk of the host builder
 // (source.cpp:832-867 order: the children of an opened node are examined in
 // octant order 7..0, emitting singletons and accepted cells in that order and
@@ -933,8 +1342,8 @@ __device__ inline int xcd_block(int b, int nb) {
 // global loads: the children's records.
 template <bool FILL>
 __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_walk(
-    int ng, const int* __restrict__ gnode, Nodes nd, const WalkNode* __restrict__ wn, double L,
-    double th2, int nleaf, int* __restrict__ pcnt, int* __restrict__ ccnt,
+    int ng, const int* __restrict__ gnode, Nodes nd, WalkNodes wn, double L,
+    double th2, int* __restrict__ pcnt, int* __restrict__ ccnt,
     const int* __restrict__ poff, const int* __restrict__ coff, int* __restrict__ plist,
     int* __restrict__ clist) {
 #pragma clang fp contract(off)
@@ -951,15 +1360,15 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_walk(
   int np = 0, nc = 0;
   int* pl = FILL ? plist + poff[g] : nullptr;
   int* cl = FILL ? clist + coff[g] : nullptr;
+  const WalkNode root = load_walk(wn, 0);
   // the whole tree as one cell (source.cpp:832-840)
-  if (bh_box_d2(gc, li, wn[0].com) * th2 >= L * L) {
-    if (FILL && lane == 0) cl[0] = wn[0].cell;
+  if (bh_box_d2(gc, li, root.com) * th2 >= L * L) {
+    if (FILL && lane == 0) cl[0] = wn.range[0].z;
     nc = 1;
   } else {
     if (lane == 0)
-      stk[0] = wn[0].hi - wn[0].lo <= nleaf || wn[0].mask == 0
-                   ? make_int3(wn[0].lo, wn[0].hi, -1)
-                   : make_int3(wn[0].first, wn[0].mask, 0);
+      stk[0] = root.leaf() ? make_int3(root.x, root.x + root.count(), -1)
+                           : make_int3(root.x, (int)root.y, 0);
     int sp = 1;
     while (sp > 0) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -973,23 +1382,24 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_walk(
       if (e < npop) ent = stk[sp - 1 - e];
       const bool leaf = e < npop && ent.z < 0;
       int kind = 0;  // 1 particle, 2 cell, 3 push
-      int lo = 0, hi = 0, cell = 0, first = 0, mask = 0;
+      int lo = 0, cell = 0;
+      WalkNode w{0, 0u, {0.0, 0.0, 0.0}};
       if (e < npop && !leaf && ((ent.y >> o) & 1)) {
         const double l = ldexp(L, -ent.z);
         const double s2 = 0.25 * l * l;  // child side squared
-        const WalkNode* w = wn + ent.x + __popc(ent.y & ((1 << o) - 1));
-        const int4 r1 = *reinterpret_cast<const int4*>(w);
-        lo = r1.x;
-        hi = r1.y;
-        cell = r1.z;
-        first = r1.w;
-        mask = w->mask;
-        if (hi - lo == 1)
+        const int k = ent.x + __popc(ent.y & ((1 << o) - 1));
+        w = load_walk(wn, k);
+        if (w.y == (kLeafEntry | 1u))
           kind = 1;
-        else if (bh_box_d2(gc, li, w->com) * th2 > s2)
+        else if (bh_box_d2(gc, li, w.com) * th2 > s2)
           kind = 2;
         else
           kind = 3;
+        if (FILL) {
+          const int4 r = wn.range[k];
+          lo = r.x;
+          cell = r.z;
+        }
       }
       // The serial walk would expand the entries from the top until one
       // pushes children; those entries (ncommit of them) are done here, the
@@ -1019,9 +1429,8 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_walk(
       const u64 mpush = ms & (0xffULL << (8 * (ncommit - 1)));  // the last committed entry
       sp -= ncommit;
       if (kind == 3 && commit)
-        stk[sp + __popcll(mpush & above)] = hi - lo <= nleaf || mask == 0
-                                                ? make_int3(lo, hi, -1)
-                                                : make_int3(first, mask, ent.z + 1);
+        stk[sp + __popcll(mpush & above)] = w.leaf() ? make_int3(w.x, w.x + w.count(), -1)
+                                                     : make_int3(w.x, (int)w.y, ent.z + 1);
       np += __popcll(mp) + leaftot;
       nc += __popcll(mc);
       sp += __popcll(mpush);
@@ -1071,7 +1480,7 @@ __global__ void k_pack_cells(int nc, const double* __restrict__ cells, float* __
 struct Octree {
   Nodes nd{};
   int nn = 0;
-  int level_start[kLevels + 2];  // level l occupies [level_start[l], level_start[l+1])
+  LevelStarts level;  // level l occupies [v[l], v[l + 1])
 };
 
 // Sorted keys, particles in Morton order and the octree.  m may be null.
@@ -1115,8 +1524,8 @@ void build_octree(Build& B, Lists& R, int n, const double* x, const double* m,
   hipLaunchKernelGGL(k_tree_levels, dim3(1), dim3(64), 0, st, nb, count, first, host_dev(host));
   PGAMD_HIP_CHECK(hipGetLastError());
   PGAMD_HIP_CHECK(hipStreamSynchronize(st));
-  for (int l = 0; l < kLevels + 2; ++l) T.level_start[l] = static_cast<volatile int*>(host)[l];
-  T.nn = T.level_start[kLevels + 1];
+  for (int l = 0; l < kLevels + 2; ++l) T.level.v[l] = static_cast<volatile int*>(host)[l];
+  T.nn = T.level.v[kLevels + 1];
   Nodes& nd = T.nd;
   const size_t c = (size_t)T.nn;
   nd.lo = B.tmp.get<int>(c);
@@ -1151,9 +1560,7 @@ int build_groups(Build& B, Lists& R, const Octree& T, int ncrit, int** gnode_out
   int* gn = B.tmp.get<int>(ng);
   int* gn_sorted = B.tmp.get<int>(ng);
   hipLaunchKernelGGL(k_compact, grid_for(nn), dim3(256), 0, st, nn, flag, off, gn);
-  LevelStarts ls;
-  for (int l = 0; l < kLevels + 2; ++l) ls.v[l] = T.level_start[l];
-  hipLaunchKernelGGL(k_group_order, grid_for(ng), dim3(256), 0, st, ng, gn, off, ls, T.nd,
+  hipLaunchKernelGGL(k_group_order, grid_for(ng, 8), dim3(256), 0, st, ng, gn, off, T.level, T.nd,
                      gn_sorted);
   PGAMD_HIP_CHECK(hipGetLastError());
   R.ng = ng;
@@ -1293,13 +1700,18 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   u64* skey = nullptr;
   double* mm = nullptr;
   build_octree(B, *R, n, x, m, lo, L, std::max(1, std::min(ncrit, nleaf)), T, &skey, &mm);
-  // moments, deepest level first
-  for (int lev = kLevels; lev >= 0; --lev) {
-    const int a = T.level_start[lev], b = T.level_start[lev + 1];
-    if (b == a) continue;
-    hipLaunchKernelGGL(k_moments, grid_for(b - a, 64), dim3(64), 0, st, a, b, T.nd, R->pos, mm);
-    PGAMD_HIP_CHECK(hipGetLastError());
+  // moments: all leaves at once, then the inner nodes, deepest level first
+  // (2^21 particles: 62 + 103 + 28 us; 16 launches over whole levels took 240)
+  hipLaunchKernelGGL(k_leaf_moments, grid_for(T.nn), dim3(256), 0, st, T.nn, T.nd, R->pos, mm);
+  int top = 0;
+  while (top <= kLevels && T.level.v[top + 1] - T.level.v[top] <= kTopNodes) ++top;
+  for (int lev = kLevels; lev >= top; --lev) {
+    const int a = T.level.v[lev], b = T.level.v[lev + 1];
+    if (b > a)
+      hipLaunchKernelGGL(k_inner_moments, grid_for(b - a, 64), dim3(64), 0, st, a, b, T.nd);
   }
+  hipLaunchKernelGGL(k_top_moments, dim3(1), dim3(kTopNodes), 0, st, top, T.level, T.nd);
+  PGAMD_HIP_CHECK(hipGetLastError());
   // cells: nodes with more than one particle, in node order
   int* flag = B.tmp.get<int>(T.nn);
   int* off = B.tmp.get<int>(T.nn + 1);
@@ -1317,19 +1729,58 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   R->joff = R->mem.get<int>(ng + 1);
   R->ccnt = R->mem.get<int>(ng);
   R->coff = R->mem.get<int>(ng + 1);
-  WalkNode* wn = B.tmp.get<WalkNode>(T.nn);
-  hipLaunchKernelGGL(k_walk_nodes, grid_for(T.nn), dim3(256), 0, st, T.nn, T.nd, wn);
+  WalkNodes wn;
+  wn.range = B.tmp.get<int4>(T.nn);
+  wn.ex = B.tmp.get<int4>(T.nn);
+  wn.yz = B.tmp.get<double2>(T.nn);
+  hipLaunchKernelGGL(k_walk_nodes, grid_for(T.nn), dim3(256), 0, st, T.nn, nleaf, T.nd, wn);
   PGAMD_HIP_CHECK(hipGetLastError());
   const dim3 wgrid((ng + kWalkWaves - 1) / kWalkWaves), wblock(64 * kWalkWaves);
-  hipLaunchKernelGGL((k_bh_walk<false>), wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2, nleaf,
-                     R->jcnt, R->ccnt, nullptr, nullptr, nullptr, nullptr);
+  // About 900 opened nodes a group at theta = 0.5 and 2^21 particles; 1280
+  // of them, more for smaller theta (nodes within a distance 1 / theta).
+  const double more = std::min(8.0, std::max(1.0, std::pow(0.5 / theta, 3)));
+  OpenPool pool{};
+  pool.chunks = (int)std::min(1e6, 64.0 + 5.0 * ng * more);
+  const size_t entries = (size_t)pool.chunks * kOpenChunk;
+  pool.rec = B.tmp.get<int4>(entries);
+  pool.wait = B.tmp.get<int>(entries);
+  pool.chunk = B.tmp.get<int>((size_t)ng * (kOpenGroupChunks + kOpenLevels) + 3);
+  pool.level = pool.chunk + (size_t)ng * kOpenGroupChunks;
+  pool.used = pool.level + (size_t)ng * kOpenLevels;
+  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, 3, 0, pool.used);
+  hipLaunchKernelGGL(k_bh_open, wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2, pool,
+                     R->jcnt, R->ccnt);
   PGAMD_HIP_CHECK(hipGetLastError());
   R->nj = B.scan(R->jcnt, R->joff, ng);
+  int* host = scan_total_host();
+  hipLaunchKernelGGL(k_copy_ints, dim3(1), dim3(64), 0, st, 3, pool.used, host_dev(host) + 1);
+  PGAMD_HIP_CHECK(hipGetLastError());
   R->nc = B.scan(R->ccnt, R->coff, ng);
+  const bool opened = static_cast<volatile int*>(host)[2] == 0;
+  const bool big = static_cast<volatile int*>(host)[3] != 0;
+  if (!opened) {
+    hipLaunchKernelGGL((k_bh_walk<false>), wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2,
+                       R->jcnt, R->ccnt, nullptr, nullptr, nullptr, nullptr);
+    PGAMD_HIP_CHECK(hipGetLastError());
+    R->nj = B.scan(R->jcnt, R->joff, ng);
+    R->nc = B.scan(R->ccnt, R->coff, ng);
+  }
   R->jlist = R->mem.get<int>(R->nj);
   R->clist = R->mem.get<int>(R->nc);
-  hipLaunchKernelGGL((k_bh_walk<true>), wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2, nleaf,
-                     nullptr, nullptr, R->joff, R->coff, R->jlist, R->clist);
+  if (opened) {
+    hipLaunchKernelGGL(k_bh_list<false>, dim3(ng), dim3(kListThreads), 0, st, ng, pool, wn.range,
+                       R->joff, R->coff, R->jlist, R->clist);
+    if (big) {
+      pool.sum = B.tmp.get<int4>(entries);
+      hipLaunchKernelGGL(k_bh_list<true>, dim3(ng), dim3(kListThreads), 0, st, ng, pool, wn.range,
+                         R->joff, R->coff, R->jlist, R->clist);
+    }
+    hipLaunchKernelGGL(k_bh_whole, grid_for(ng), dim3(256), 0, st, ng, R->jcnt, R->ccnt, wn,
+                       R->coff, gnode, T.nd, L, th2, R->clist);
+  } else {
+    hipLaunchKernelGGL((k_bh_walk<true>), wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2,
+                       nullptr, nullptr, R->joff, R->coff, R->jlist, R->clist);
+  }
   PGAMD_HIP_CHECK(hipGetLastError());
   finish(B, *R, true);
   return R;

@@ -53,3 +53,18 @@ def test_bh_lists_at_block_and_window_edges(n, ncrit, nleaf, theta):
     h = pgamd.bh_lists(x, m, theta, ncrit, nleaf)
     d_x, d_m = dev(x), dev(m)
     check(h, pgamd.DevLists.bh(d_x.data_ptr(), d_m.data_ptr(), n, theta, ncrit, nleaf), True)
+
+
+# the walk's queue: entries in chunks of 256, at most 64 a group (16384 opened
+# nodes), from a pool of 5 to 40 chunks a group; beyond either the build falls
+# back to the depth-first walk
+@pytest.mark.parametrize("n,ncrit,nleaf,theta", [
+    (2000, 2000, 1, 0.01), (20000, 20000, 1, 0.01), (60000, 60000, 1, 0.01),
+    (30000, 64, 1, 0.05), (8000, 8, 3, 0.2), (700, 700, 700, 0.5), (5000, 32, 8, 40.0),
+])
+def test_bh_lists_at_queue_edges(n, ncrit, nleaf, theta):
+    import pgamd
+    m, x = ics.hernquist(n, n + 1)
+    h = pgamd.bh_lists(x, m, theta, ncrit, nleaf)
+    d_x, d_m = dev(x), dev(m)
+    check(h, pgamd.DevLists.bh(d_x.data_ptr(), d_m.data_ptr(), n, theta, ncrit, nleaf), True)
