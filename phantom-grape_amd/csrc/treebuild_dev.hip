@@ -17,6 +17,8 @@
 #include "pgamd_common.h"
 #include "pgamd_api.h"
 
+#include "radix_sort.h"
+
 #include <hipcub/device/device_radix_sort.hpp>
 #include <hipcub/device/device_scan.hpp>
 
@@ -147,6 +149,29 @@ int* host_dev(int* host) {
   return dev;
 }
 
+// Sorts of fewer pairs go to the library (its one-block and merge sorts), of
+// more to radix_sort.h: whole builds of 2^17 particles take 423 us (TreePM)
+// and 449 (Barnes-Hut) with the library's sorts, 421 and 482 with those; of
+// 2^18 particles 556 and 544 against 465 and 552, of 2^19 664 and 690 against
+// 510 and 649.
+constexpr int kCountingFrom = 1 << 18;
+// The upper bits of a 63-bit Morton key that are sorted first: they tell
+// apart cells of 2^-13 of the box, so few particles are left equal.
+constexpr int kFirstBits = 40;
+
+__global__ void k_iota(int n, int* __restrict__ v) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) v[i] = i;
+}
+
+__global__ void k_fill_int(int n, int v, int* __restrict__ out) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) out[i] = v;
+}
+
+inline dim3 grid_for(long long n, int threads = 256) {
+  return dim3((unsigned)std::max<long long>(1, (n + threads - 1) / threads));
+}
+
 // Temporary storage for one build, released at its end.
 struct Build {
   hipStream_t st;
@@ -197,11 +222,7 @@ struct Build {
     PGAMD_HIP_CHECK(hipStreamSynchronize(st));
     return *static_cast<volatile int*>(host);
   }
-  // Stable radix sort of (key, value) pairs; int keys must be >= 0.
-  void sort_pairs(const int* kin, int* kout, const int* vin, int* vout, int n, int end_bit) {
-    sort_pairs(reinterpret_cast<const unsigned*>(kin), reinterpret_cast<unsigned*>(kout), vin,
-               vout, n, end_bit);
-  }
+  // Stable library sort of (key, value) pairs.
   template <class K>
   void sort_pairs(const K* kin, K* kout, const int* vin, int* vout, int n, int end_bit) {
     if (n <= 0) return;
@@ -211,6 +232,39 @@ struct Build {
     PGAMD_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(cub_tmp(b), b, kin, kout, vin, vout, n, 0,
                                                        end_bit, st));
   }
+  // Stable sort of n keys (overwritten) by bits [0, bits) with the values 0
+  // .. n - 1: *skey and *perm are set to the sorted arrays.  Only the upper
+  // `first` bits take counting passes; pairs they leave equal are put in
+  // order by one more launch.  Returns the device flag (null if there is
+  // none) that it sets if a run of them is too long for that: the caller, with
+  // its next read-back, then sorts again with first = bits.
+  template <class K>
+  int* sort_keys(K* key, int n, int bits, int first, K** skey, int** perm) {
+    K* k[2] = {key, tmp.get<K>(n)};
+    int* v[2] = {tmp.get<int>(n), tmp.get<int>(n)};
+    if (n < kCountingFrom) {
+      hipLaunchKernelGGL(k_iota, grid_for(n), dim3(256), 0, st, n, v[0]);
+      sort_pairs(k[0], k[1], v[0], v[1], n, bits);
+      *skey = k[1];
+      *perm = v[1];
+      return nullptr;
+    }
+    int* scratch = tmp.get<int>(pgsort::scratch_ints(n) + 1);
+    int* long_run = nullptr;
+    const int shift = std::max(0, bits - first);
+    int cur = pgsort::radix_sort(n, k, v, shift, bits, scratch, st);
+    if (shift > 0) {
+      long_run = scratch + pgsort::scratch_ints(n);
+      hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, 1, 0, long_run);
+      hipLaunchKernelGGL(pgsort::radix_finish<K>, grid_for(n), dim3(256), 0, st, n, shift, k[cur],
+                         v[cur], k[1 - cur], v[1 - cur], long_run);
+      cur = 1 - cur;
+    }
+    PGAMD_HIP_CHECK(hipGetLastError());
+    *skey = k[cur];
+    *perm = v[cur];
+    return long_run;
+  }
 };
 
 // Bits needed to hold every value in [0, v].
@@ -218,10 +272,6 @@ inline int bits_for(long long v) {
   int b = 1;
   while ((1LL << b) <= v) ++b;
   return b;
-}
-
-inline dim3 grid_for(long long n, int threads = 256) {
-  return dim3((unsigned)std::max<long long>(1, (n + threads - 1) / threads));
 }
 
 // ------------------------------------------------------------ Morton keys
@@ -236,7 +286,7 @@ __device__ inline u64 spread3(u64 v) {
 }
 
 __global__ void k_keys(int n, const double* __restrict__ x, double lo0, double lo1, double lo2,
-                       double s, u64* __restrict__ key, int* __restrict__ idx) {
+                       double s, u64* __restrict__ key) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -249,7 +299,6 @@ __global__ void k_keys(int n, const double* __restrict__ x, double lo0, double l
     k |= spread3((u64)q) << (2 - d);
   }
   key[i] = k;
-  idx[i] = i;
 }
 
 // Bounding box: per-block min/max of each axis, then one block over those.
@@ -407,10 +456,12 @@ __global__ __launch_bounds__(256) void k_tree_count(int n, const u64* __restrict
 }
 
 // host[l] = first node of level l, host[kTreeLevels] = number of nodes, from
-// the scan of k_tree_count's counts (nb blocks).
+// the scan of k_tree_count's counts (nb blocks), and host[kTreeLevels + 1] =
+// *flag (0 for a null one).
 __global__ void k_tree_levels(int nb, const int* __restrict__ count, const int* __restrict__ first,
-                              int* __restrict__ host) {
+                              const int* __restrict__ flag, int* __restrict__ host) {
   const int l = threadIdx.x;
+  if (l == kTreeLevels + 1) host[l] = flag ? *flag : 0;
   if (l < kTreeLevels) host[l] = first[(size_t)l * nb];
   if (l == kTreeLevels) {
     const size_t e = (size_t)kTreeLevels * nb - 1;
@@ -511,10 +562,6 @@ __global__ __launch_bounds__(256) void k_tree_nodes(int nn, int n, const u64* __
     l *= 0.5;
   }
   for (int q = 0; q < 3; ++q) nd.c[3 * (size_t)k + q] = c[q];
-}
-
-__global__ void k_fill_int(int n, int v, int* __restrict__ out) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) out[i] = v;
 }
 
 __global__ void k_copy_ints(int n, const int* __restrict__ in, int* __restrict__ out) {
@@ -734,13 +781,12 @@ __device__ inline int cidx(const Grid& g, double v) {
   return c < 0 ? 0 : (c > g.nc - 1 ? g.nc - 1 : c);
 }
 
-__global__ void k_cell_of(int np, const double* __restrict__ pos, Grid g, int* __restrict__ cell,
-                          int* __restrict__ idx) {
+__global__ void k_cell_of(int np, const double* __restrict__ pos, Grid g,
+                          unsigned* __restrict__ cell) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
   cell[p] = (cidx(g, pos[3 * p]) * g.nc + cidx(g, pos[3 * p + 1])) * g.nc +
             cidx(g, pos[3 * p + 2]);
-  idx[p] = p;
 }
 
 // Positions in cell order: cpos[k] = pos[cpart[k]], so the list walk reads
@@ -754,14 +800,14 @@ __global__ void k_cell_pos(int np, const int* __restrict__ cpart, const double* 
 }
 
 // cstart[c] = first position of cell c in the sorted cell array (c <= ncell).
-__global__ void k_cell_start(int ncell, int np, const int* __restrict__ scell,
+__global__ void k_cell_start(int ncell, int np, const unsigned* __restrict__ scell,
                              int* __restrict__ cstart) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c > ncell) return;
   int a = 0, b = np;
   while (a < b) {
     const int mid = a + (b - a) / 2;
-    if (scell[mid] < c)
+    if (scell[mid] < (unsigned)c)
       a = mid + 1;
     else
       b = mid;
@@ -1488,17 +1534,49 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_walk(
 }
 
 // ------------------------------------------------------------ common tail
-// cost key: groups by decreasing icnt * (jcnt + 2 ccnt), ties by index.
+// cost key: groups by decreasing icnt * (jcnt + 2 ccnt), ties by index.  idx:
+// the groups (to be sorted), or their ranks cleared.
 __global__ void k_cost(int ng, const int* __restrict__ icnt, const int* __restrict__ jcnt,
                        const int* __restrict__ ccnt, u64* __restrict__ key, int* __restrict__ idx,
-                       unsigned long long* __restrict__ work) {
+                       bool by_rank, unsigned long long* __restrict__ work) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= ng) return;
   const long long c = (long long)icnt[g] * (jcnt[g] + (ccnt ? 2 * ccnt[g] : 0));
   key[g] = (u64)(LLONG_MAX - c);
-  idx[g] = g;
+  idx[g] = by_rank ? 0 : g;
   atomicAdd(&work[0], (unsigned long long)((long long)icnt[g] * jcnt[g]));
   if (ccnt) atomicAdd(&work[1], (unsigned long long)((long long)icnt[g] * ccnt[g]));
+}
+
+// order[] of k_cost's keys for up to kRankGroups groups: rank[g] (0 before)
+// gains the groups of one tile that come before g, then order[rank[g]] = g.
+// Every pair is compared, 14029 groups in 25 us; the library's sort of the
+// 64-bit keys took 61.
+constexpr int kRankGroups = 1 << 14;
+__global__ __launch_bounds__(256) void k_rank(int ng, const u64* __restrict__ key,
+                                              int* __restrict__ rank) {
+  __shared__ u64 s[256];
+  const int h0 = blockIdx.y * 256, g = blockIdx.x * 256 + threadIdx.x;
+  if (h0 + (int)threadIdx.x < ng) s[threadIdx.x] = key[h0 + threadIdx.x];
+  __syncthreads();
+  if (g >= ng) return;
+  const u64 own = key[g];
+  const int n = min(256, ng - h0);
+  int r = 0;
+  if (blockIdx.y == blockIdx.x) {
+    for (int h = 0; h < n; ++h) r += s[h] < own || (s[h] == own && h0 + h < g);
+  } else {
+    // a tie goes to the lower index; keys are below 2^63
+    const u64 end = own + (blockIdx.y < blockIdx.x);
+#pragma unroll 8
+    for (int h = 0; h < n; ++h) r += s[h] < end;
+  }
+  if (r) atomicAdd(&rank[g], r);
+}
+
+__global__ void k_rank_order(int ng, const int* __restrict__ rank, int* __restrict__ order) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g < ng) order[rank[g]] = g;
 }
 
 __global__ void k_pack(int np, const double* __restrict__ pos, const int* __restrict__ src,
@@ -1534,41 +1612,43 @@ void build_octree(Build& B, Lists& R, int n, const double* x, const double* m,
                   double** mm_out) {
   hipStream_t st = B.st;
   u64* key = B.tmp.get<u64>(n);
-  u64* skey = B.tmp.get<u64>(n);
-  int* idx = B.tmp.get<int>(n);
-  int* perm = B.tmp.get<int>(n);
   const double s = (double)(1 << kLevels) / L;
-  hipLaunchKernelGGL(k_keys, grid_for(n), dim3(256), 0, st, n, x, lo[0], lo[1], lo[2], s, key, idx);
-  PGAMD_HIP_CHECK(hipGetLastError());
-  B.sort_pairs(key, skey, idx, perm, n, 3 * kLevels);
   double* mm = m ? B.tmp.get<double>(n) : nullptr;
-  hipLaunchKernelGGL(k_gather, grid_for(n), dim3(256), 0, st, n, perm, x, m, R.pos, mm, R.src);
-  PGAMD_HIP_CHECK(hipGetLastError());
-  // leaf level of every particle: the sliding maximum, in steps of at most
-  // kMaxWindow (maxima over windows of u and v give one over u + v - 1)
   unsigned char* leaf = B.tmp.get<unsigned char>(n);
   unsigned char* leaf2 = split > kMaxWindow ? B.tmp.get<unsigned char>(n) : nullptr;
-  const dim3 wgrid = grid_for(n, kWindowOut);
-  int left = split;  // of a window of split + 1
-  int w = std::min(left, kMaxWindow) + 1;
-  hipLaunchKernelGGL(k_window_max<true>, wgrid, dim3(256), 0, st, n, split, w, skey, nullptr, leaf);
-  for (left -= w - 1; left > 0; left -= w - 1) {
-    w = std::min(left, kMaxWindow) + 1;
-    hipLaunchKernelGGL(k_window_max<false>, wgrid, dim3(256), 0, st, n, split, w, nullptr, leaf,
-                       leaf2);
-    std::swap(leaf, leaf2);
-  }
-  PGAMD_HIP_CHECK(hipGetLastError());
   const int nb = (int)grid_for(n, kTreeBlock).x;
   int* count = B.tmp.get<int>((size_t)kTreeLevels * nb);
   int* first = B.tmp.get<int>((size_t)kTreeLevels * nb + 1);
-  hipLaunchKernelGGL(k_tree_count, dim3(nb), dim3(256), 0, st, n, skey, leaf, count);
-  PGAMD_HIP_CHECK(hipGetLastError());
-  B.scan_async(count, first, kTreeLevels * nb);
   int* host = scan_total_host();
-  hipLaunchKernelGGL(k_tree_levels, dim3(1), dim3(64), 0, st, nb, count, first, host_dev(host));
-  PGAMD_HIP_CHECK(hipGetLastError());
-  PGAMD_HIP_CHECK(hipStreamSynchronize(st));
+  u64* skey = nullptr;
+  for (int bits = kFirstBits;; bits = 3 * kLevels) {
+    hipLaunchKernelGGL(k_keys, grid_for(n), dim3(256), 0, st, n, x, lo[0], lo[1], lo[2], s, key);
+    PGAMD_HIP_CHECK(hipGetLastError());
+    int* perm = nullptr;
+    const int* long_run = B.sort_keys(key, n, 3 * kLevels, bits, &skey, &perm);
+    hipLaunchKernelGGL(k_gather, grid_for(n), dim3(256), 0, st, n, perm, x, m, R.pos, mm, R.src);
+    // leaf level of every particle: the sliding maximum, in steps of at most
+    // kMaxWindow (maxima over windows of u and v give one over u + v - 1)
+    const dim3 wgrid = grid_for(n, kWindowOut);
+    int left = split;  // of a window of split + 1
+    int w = std::min(left, kMaxWindow) + 1;
+    hipLaunchKernelGGL(k_window_max<true>, wgrid, dim3(256), 0, st, n, split, w, skey, nullptr,
+                       leaf);
+    for (left -= w - 1; left > 0; left -= w - 1) {
+      w = std::min(left, kMaxWindow) + 1;
+      hipLaunchKernelGGL(k_window_max<false>, wgrid, dim3(256), 0, st, n, split, w, nullptr, leaf,
+                         leaf2);
+      std::swap(leaf, leaf2);
+    }
+    hipLaunchKernelGGL(k_tree_count, dim3(nb), dim3(256), 0, st, n, skey, leaf, count);
+    PGAMD_HIP_CHECK(hipGetLastError());
+    B.scan_async(count, first, kTreeLevels * nb);
+    hipLaunchKernelGGL(k_tree_levels, dim3(1), dim3(64), 0, st, nb, count, first, long_run,
+                       host_dev(host));
+    PGAMD_HIP_CHECK(hipGetLastError());
+    PGAMD_HIP_CHECK(hipStreamSynchronize(st));
+    if (static_cast<volatile int*>(host)[kTreeLevels + 1] == 0) break;  // no long run
+  }
   for (int l = 0; l < kLevels + 2; ++l) T.level.v[l] = static_cast<volatile int*>(host)[l];
   T.nn = T.level.v[kLevels + 1];
   Nodes& nd = T.nd;
@@ -1627,15 +1707,21 @@ void finish(Build& B, Lists& R, bool cells) {
   hipStream_t st = B.st;
   const int ng = (int)R.ng;
   u64* key = B.tmp.get<u64>(ng);
-  u64* skey = B.tmp.get<u64>(ng);
   int* idx = B.tmp.get<int>(ng);
   unsigned long long* work = B.tmp.get<unsigned long long>(2);
   PGAMD_HIP_CHECK(hipMemsetAsync(work, 0, 2 * sizeof(unsigned long long), st));
   R.order = R.mem.get<int>(ng);
   hipLaunchKernelGGL(k_cost, grid_for(ng), dim3(256), 0, st, ng, R.icnt, R.jcnt,
-                     cells ? R.ccnt : nullptr, key, idx, work);
+                     cells ? R.ccnt : nullptr, key, idx, ng <= kRankGroups, work);
+  if (ng <= kRankGroups) {
+    hipLaunchKernelGGL(k_rank, dim3(grid_for(ng).x, grid_for(ng).x), dim3(256), 0, st, ng, key,
+                       idx);
+    hipLaunchKernelGGL(k_rank_order, grid_for(ng), dim3(256), 0, st, ng, idx, R.order);
+  } else {
+    u64* skey = B.tmp.get<u64>(ng);
+    B.sort_pairs(key, skey, idx, R.order, ng, 64);
+  }
   PGAMD_HIP_CHECK(hipGetLastError());
-  B.sort_pairs(key, skey, idx, R.order, ng, 64);
   unsigned long long w[2];
   PGAMD_HIP_CHECK(hipMemcpyAsync(w, work, sizeof(w), hipMemcpyDeviceToHost, st));
   PGAMD_HIP_CHECK(hipStreamSynchronize(st));
@@ -1675,14 +1761,14 @@ Lists* treepm_build(int n, const double* x, double rcut, int ncrit, hipStream_t 
   gr.nc = std::max(1, (int)std::floor(gL / rcut));
   gr.h = gL / gr.nc;
   const int ncell = gr.nc * gr.nc * gr.nc;
-  int* cell = B.tmp.get<int>(np);
-  int* scell = B.tmp.get<int>(np);
-  int* idx = B.tmp.get<int>(np);
-  int* cpart = B.tmp.get<int>(np);
+  unsigned* cell = B.tmp.get<unsigned>(np);
+  unsigned* scell = nullptr;
+  int* cpart = nullptr;
   int* cstart = B.tmp.get<int>(ncell + 1);
-  hipLaunchKernelGGL(k_cell_of, grid_for(np), dim3(256), 0, st, np, R->pos, gr, cell, idx);
+  hipLaunchKernelGGL(k_cell_of, grid_for(np), dim3(256), 0, st, np, R->pos, gr, cell);
   PGAMD_HIP_CHECK(hipGetLastError());
-  B.sort_pairs(cell, scell, idx, cpart, np, bits_for(ncell));
+  const int cell_bits = bits_for(ncell);
+  B.sort_keys(cell, np, cell_bits, cell_bits, &scell, &cpart);
   hipLaunchKernelGGL(k_cell_start, grid_for(ncell + 1), dim3(256), 0, st, ncell, np, scell,
                      cstart);
   PGAMD_HIP_CHECK(hipGetLastError());
