@@ -6,18 +6,17 @@
 // kernels and reads Ctl back when it wants to know where the run stands.
 //
 // State (device, FP64, particle order = j address = id): x[n][3], v[n][3],
-// a[n][3], j[n][3], pot[n], t[n], dt[n], m[n].  One block step, with
-// t_next = min_i (t_i + dt_i) known from the step before:
-//   1. predict every j to t_next; active = { i : t_i + dt_i == t_next },
-//      appended to the active list with their predicted i data
-//      (predict_exmotion); the minimum of t + dt over the others
-//                                                          (pg6h_select)
+// a[n][3], j[n][3], pot[n], t[n], dt[n], m[n].  One block step:
+//   1. t_next = min_i (t_i + dt_i) from the minima of the step before; predict
+//      every j to it; active = { i : t_i + dt_i == t_next }, appended to the
+//      active list with their predicted i data (predict_exmotion); the minima
+//      of t + dt over the others                           (pg6h_select)
 //   2. force, jerk, pot of the active i against all j      (pg6h_force)
 //   3. sum of the j-range partials, corrector + new time step, j-memory
-//      update, reset of every time at the end of a dtmax window; the
-//      minimum of the new t + dt folded in, which makes the next t_next;
-//      step bookkeeping                                    (pg6h_finish)
-// The first t_next comes from pg6h_min_time after the start-up.
+//      update, reset of every time at the end of a dtmax window; minima of
+//      the new t + dt, whose minimum is the next t_next; step bookkeeping
+//                                                          (pg6h_finish)
+// The first minima come from pg6h_min_time after the start-up.
 // Every FP64 expression is written in the reference's operation order with
 // contraction off, so given the same forces the corrected state and the time
 // steps equal those of the reference's code bit for bit.  One deviation: the
@@ -27,6 +26,8 @@
 // pair sums run over the j addresses in a fixed order).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <climits>
+#include <cmath>
 #include "pg6_kernels.h"
 
 namespace pg6h {
@@ -76,29 +77,29 @@ __device__ inline double dt_startup(const Params& P, double t_gl, const double* 
 }
 
 // ---------------------------------------------------------------- control
-// Step state in device memory.  Written by pg6h_select (nact), pg6h_finish
-// (everything else, by its last block) and the host between runs (t_end).
+// Step state in device memory.  No kernel reads what its own other blocks
+// write here, so a step needs neither fences nor counted blocks: pg6h_select
+// reads the state between the steps and writes the step's own, pg6h_force and
+// pg6h_finish read that, and block 0 of pg6h_finish writes the state between
+// the steps.  The lengths of the active lists of this step and the next take
+// turns (pg6h_finish clears the next one's).
 struct Ctl {
-  unsigned long long tmin;       // bits of t_next = min(t + dt) for the next step
-  unsigned long long tmin_next;  // bits of min(t + dt) being folded for the step after
+  // between the steps: pg6h_finish, and the host between runs
   double t_gl;              // time inside the current window [0, dtmax)
   double t_end;             // a step is taken only while t_mod * dtmax + t_gl < t_end
   long long t_mod;          // completed windows (t = t_mod * dtmax + t_gl)
   long long nsteps;         // particle steps taken
   long long nblocks;        // block steps taken
-  int nact;                 // length of the active list being formed
   int last_nact;            // active particles of the last step taken
-  int done;                 // pg6h_finish blocks finished with the current step
   int bad;                  // particles whose step fell below dtmin
+  // of the step: pg6h_select
+  double tnext;             // min(t + dt)
+  int run;                  // 0: the step is past t_end and nothing is done
+  int turn;                 // the list length in use
+  int nact[2];              // length of the active list being formed
 };
 
-// +infinity as FP64 bits: the neutral element of the min over t + dt (all
-// t + dt are positive, so their bit patterns order as the values do).
-constexpr unsigned long long kInfBits = 0x7FF0000000000000ull;
-
-// Whether the step being queued is past the end of the run.  Every kernel of
-// a step evaluates it on the same Ctl fields, which only pg6h_finish's last
-// block changes, so all of them take the same decision.
+// Whether the step being queued is past the end of the run.
 __device__ inline bool pg6h_skip(const Ctl* c, double dtmax) {
 #pragma clang fp contract(off)
   return (double)c->t_mod * dtmax + c->t_gl >= c->t_end;
@@ -109,107 +110,167 @@ __device__ inline bool pg6h_skip(const Ctl* c, double dtmax) {
 // of kForceWaves wavefronts per (tile, range) item; wavefront w of the block
 // takes the w-th of kForceWaves equal pieces of the range (a multiple of 16
 // addresses, at least min_jper).  About `target` wavefronts of work in all.
-// Partials of range s for active slot k sit at s * stride + k.
 constexpr int kForceWaves = 8;
-// pg6h_force sums the seven components with one wavefront each
-static_assert(kForceWaves >= 7, "a block needs a wavefront per force component");
+// pg6h_force writes a record of kRec doubles per (range, active slot): ax,
+// ay, az, pot, jx, jy, jz and one unused, the eight wavefronts' threads in
+// that order.  Range s, slot k: record s * stride + k.
+constexpr int kRec = 8;
+static_assert(kForceWaves == kRec, "pg6h_force writes one component per thread");
 
+// What the host knows of the split before nact: with up to `tiles` tiles the
+// number of ranges is the largest there is, ns of jper addresses.
+struct Split {
+  int nj, blocks, max_ns, tiles, ns, jper;
+};
 struct Plan {
   int ntiles, ns, jper, stride;
 };
 
-__host__ __device__ inline Plan pg6h_plan(int nact, int nj, int target, int min_jper) {
+__host__ __device__ inline void pg6h_ranges(int nj, int want, int* ns, int* jper) {
+  const int q = 16 * kForceWaves;
+  *jper = ((nj + want - 1) / want + q - 1) / q * q;
+  *ns = (nj + *jper - 1) / *jper;
+}
+
+inline Split pg6h_split(int nj, int target, int min_jper) {
+  Split sp;
+  sp.nj = nj;
+  sp.blocks = target / kForceWaves;
+  sp.max_ns = nj / (kForceWaves * min_jper);
+  if (sp.max_ns < 1) sp.max_ns = 1;
+  // ceil(blocks / tiles) >= max_ns up to this many tiles
+  sp.tiles = sp.max_ns > 1 ? (sp.blocks - 1) / (sp.max_ns - 1) : INT_MAX;
+  pg6h_ranges(nj, sp.max_ns, &sp.ns, &sp.jper);
+  return sp;
+}
+
+__device__ inline Plan pg6h_plan(int nact, const Split& sp) {
   Plan p;
   p.ntiles = (nact + 63) / 64;
-  const int blocks = target / kForceWaves;
-  int ns = p.ntiles > 0 ? (blocks + p.ntiles - 1) / p.ntiles : 1;
-  if (ns > nj / (kForceWaves * min_jper)) ns = nj / (kForceWaves * min_jper);
-  if (ns < 1) ns = 1;
-  const int q = 16 * kForceWaves;
-  p.jper = ((nj + ns - 1) / ns + q - 1) / q * q;
-  p.ns = (nj + p.jper - 1) / p.jper;
   p.stride = p.ntiles * 64;
+  if (p.ntiles <= sp.tiles) {  // no division on a short step's way
+    p.ns = sp.ns;
+    p.jper = sp.jper;
+  } else {
+    pg6h_ranges(sp.nj, (sp.blocks + p.ntiles - 1) / p.ntiles, &p.ns, &p.jper);
+  }
   return p;
 }
 
 // ---------------------------------------------------------------- next time
-// Folds the wavefront minimum of v (lanes without a value pass 1e300) into
-// *dst.  The atomic's result is consumed so that it has completed before the
-// wavefront goes on.
-__device__ inline void fold_min(double v, unsigned long long* dst) {
-  for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
-  if ((threadIdx.x & 63) == 0 && v < 1e300) {
-    const unsigned long long old = atomicMin(dst, (unsigned long long)__double_as_longlong(v));
-    asm volatile("" ::"v"(old));
-  }
+// v of the lane that a DPP control names (within its row of 16).
+template <int CTRL>
+__device__ inline double dpp(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ inline double readlane(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// Minimum over the wavefront (all lanes active): rotations by 8, 4, 2 and 1
+// in the rows, then the four rows.
+__device__ inline double wave_min(double v) {
+  v = fmin(v, dpp<0x128>(v));
+  v = fmin(v, dpp<0x124>(v));
+  v = fmin(v, dpp<0x122>(v));
+  v = fmin(v, dpp<0x121>(v));
+  return fmin(fmin(readlane(v, 0), readlane(v, 16)), fmin(readlane(v, 32), readlane(v, 48)));
 }
 
-// The same for the whole block, with one atomic per block (all the block's
-// atomics on one address would queue behind each other).  Every thread of
-// the block calls it; thread 0 waits for the atomic's result (pg6h_finish's
-// last block relies on that).  Blocks of at most 1024 threads.
-__device__ inline void fold_min_block(double v, unsigned long long* dst) {
-  __shared__ double s_min[16];
-  for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
-  if ((threadIdx.x & 63) == 0) s_min[threadIdx.x / 64] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < (int)(blockDim.x + 63) / 64; ++w) v = fmin(v, s_min[w]);
-    if (v < 1e300) {
-      const unsigned long long old = atomicMin(dst, (unsigned long long)__double_as_longlong(v));
-      asm volatile("" ::"v"(old));
-    }
-  }
-}
-
-// t_next = min_i (t_i + dt_i) into Ctl::tmin (after the start-up).
-__global__ __launch_bounds__(256) void pg6h_min_time(int n, State S, Ctl* ctl) {
+// t_next = min_i (t_i + dt_i) is the minimum of mins[], one value per
+// wavefront of pg6h_finish; without a value 1e300.  This fills it after the
+// start-up, with the same grid.
+constexpr double kNoTime = 1e300;
+__global__ __launch_bounds__(256) void pg6h_min_time(int n, State S, double* __restrict__ mins) {
 #pragma clang fp contract(off)
-  double v = 1e300;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    v = fmin(v, S.t[i] + S.dt[i]);
-  fold_min(v, &ctl->tmin);
+  double v = kNoTime;
+  const int i0 = blockIdx.x * blockDim.x + threadIdx.x;
+  for (int i = i0; i < n; i += gridDim.x * blockDim.x) v = fmin(v, S.t[i] + S.dt[i]);
+  v = wave_min(v);
+  if ((threadIdx.x & 63) == 0) mins[i0 / 64] = v;
 }
 
 // ---------------------------------------------------------------- selection
-// Every j predicted to t_next (the board's predictor, pg6_predict_j); the
+// t_next; every j predicted to it (the board's predictor, pg6_predict_j); the
 // active particles (t + dt == t_next, global_time of banana01.c /
 // timestep.c:81-92) appended to the active list with their i data as
 // predict_exmotion (hermite.c:39-62) computes it: FP64 position and
-// velocity at t_next, id = address.  Block = 256 threads, one particle each.
+// velocity at t_next, id = address.  rest[block] = the smallest t + dt of the
+// block's particles that do not move (kNoTime: none).  Block = 256 threads,
+// one particle each.  All loads of a thread are issued before the first wait;
+// only the length of the list and what depends on it come after.
 __global__ __launch_bounds__(256) void pg6h_select(int n, State S, Params P, Ctl* ctl,
+                                                   const double* __restrict__ mins, int nmins,
                                                    pg6::JState js, pg6::JPred jp,
                                                    int* __restrict__ act,
                                                    double* __restrict__ ipos,
                                                    double* __restrict__ ivel,
-                                                   int* __restrict__ iid) {
+                                                   int* __restrict__ iid,
+                                                   double* __restrict__ rest) {
 #pragma clang fp contract(off)
-  if (pg6h_skip(ctl, P.dtmax)) return;
-  const double tnext = __longlong_as_double((long long)ctl->tmin);
+  __shared__ double s_min[4], s_rest[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i < n;
-  pg6::pg6_predict_j(i, valid, tnext, js, jp);
-  const double tn = valid ? S.t[i] + S.dt[i] : 1e300;
-  const bool a = valid && tn == tnext;
-  fold_min_block(a ? 1e300 : tn, &ctl->tmin_next);  // the particles that do not move
-  const unsigned long long mask = __ballot(a);
-  const int lane = threadIdx.x & 63;
-  int base = 0;
-  if (lane == 0 && mask != 0ull) base = atomicAdd(&ctl->nact, __popcll(mask));
-  base = __shfl(base, 0);
-  if (!a) return;
-  const int k = base + __popcll(mask & ((1ull << lane) - 1ull));
-  act[k] = i;
-  const double dt = tnext - S.t[i];
-  const double dt2 = dt * dt;
-  const double dt3 = dt * dt2;
-  for (int d = 0; d < 3; ++d) {
-    const double x = S.x[3 * i + d], v = S.v[3 * i + d];
-    const double ac = S.a[3 * i + d], j = S.j[3 * i + d];
-    ipos[3 * k + d] = x + v * dt + ac * dt2 * kSecond + j * dt3 * kThird;
-    ivel[3 * k + d] = v + ac * dt + j * dt2 * kSecond;
+  const pg6::JRaw raw = pg6::pg6_load_j(i, valid, js);
+  double t = 0.0, dts = 0.0, v = kNoTime;
+  if (valid) {
+    t = S.t[i];
+    dts = S.dt[i];
   }
-  iid[k] = i;
+  for (int q = threadIdx.x; q < nmins; q += 256) v = fmin(v, mins[q]);
+  if (pg6h_skip(ctl, P.dtmax)) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->run = 0;
+    return;
+  }
+  const int turn = (int)(ctl->nblocks & 1);
+  v = wave_min(v);
+  if (lane == 0) s_min[wave] = v;
+  __syncthreads();
+  v = fmin(fmin(s_min[0], s_min[1]), fmin(s_min[2], s_min[3]));
+  const double tnext = v < kNoTime ? v : (double)INFINITY;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    ctl->tnext = tnext;
+    ctl->turn = turn;
+    ctl->run = 1;
+  }
+  const double tn = valid ? t + dts : kNoTime;
+  const bool a = valid && tn == tnext;
+  const unsigned long long mask = __ballot(a);
+  int base = 0;
+  if (lane == 0 && mask != 0ull) base = atomicAdd(&ctl->nact[turn], __popcll(mask));
+  double x[3], vel[3], ac[3], j[3];
+  if (a)
+    for (int d = 0; d < 3; ++d) {
+      x[d] = S.x[3 * i + d];
+      vel[d] = S.v[3 * i + d];
+      ac[d] = S.a[3 * i + d];
+      j[d] = S.j[3 * i + d];
+    }
+  pg6::pg6_predict_j(i, valid, tnext, raw, jp);
+  const double r = wave_min(a ? kNoTime : tn);
+  if (lane == 0) s_rest[wave] = r;
+  base = __builtin_amdgcn_readfirstlane(base);
+  if (a) {
+    const int k = base + __popcll(mask & ((1ull << lane) - 1ull));
+    act[k] = i;
+    const double dt = tnext - t;
+    const double dt2 = dt * dt;
+    const double dt3 = dt * dt2;
+    for (int d = 0; d < 3; ++d) {
+      ipos[3 * k + d] = x[d] + vel[d] * dt + ac[d] * dt2 * kSecond + j[d] * dt3 * kThird;
+      ivel[3 * k + d] = vel[d] + ac[d] * dt + j[d] * dt2 * kSecond;
+    }
+    iid[k] = i;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    rest[blockIdx.x] = fmin(fmin(s_rest[0], s_rest[1]), fmin(s_rest[2], s_rest[3]));
 }
 
 // ---------------------------------------------------------------- force
@@ -219,20 +280,19 @@ __global__ __launch_bounds__(256) void pg6h_select(int n, State S, Params P, Ctl
 // sums over their pieces of a range are added in LDS in wavefront order and
 // written as one FP64 partial per range.
 __global__ __launch_bounds__(64 * kForceWaves) void pg6h_force(
-    int n, float eps2, Params P, const Ctl* ctl, int target, int min_jper,
-    const double* __restrict__ ipos, const double* __restrict__ ivel, const int* __restrict__ iid,
-    pg6::JPred jp, pg6::Partials part) {
-  if (pg6h_skip(ctl, P.dtmax)) return;
-  const int nact = ctl->nact;
-  const Plan pl = pg6h_plan(nact, n, target, min_jper);
+    int n, float eps2, const Ctl* ctl, Split split, const double* __restrict__ ipos,
+    const double* __restrict__ ivel, const int* __restrict__ iid, pg6::JPred jp,
+    double* __restrict__ part) {
+  if (!ctl->run) return;
+  const int nact = ctl->turn ? ctl->nact[1] : ctl->nact[0];
+  const Plan pl = pg6h_plan(nact, split);
   const int items = pl.ntiles * pl.ns;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int piece = pl.jper / kForceWaves;
-  double* dst[7] = {part.ax, part.ay, part.az, part.pot, part.jx, part.jy, part.jz};
-  __shared__ double red[7][kForceWaves][64];
+  __shared__ double red[7][kForceWaves * 64 + 8];  // the 8 spread the components over the banks
   for (int it = blockIdx.x; it < items; it += gridDim.x) {
-    const int tile = it % pl.ntiles, sp = it / pl.ntiles;
+    const int sp = pl.ntiles == 1 ? it : it / pl.ntiles, tile = it - sp * pl.ntiles;
     const int i = tile * 64 + lane;
     const int ic = i < nact ? i : nact - 1;  // padding lanes repeat the last slot
     const int j0 = min(n, sp * pl.jper + w * piece);
@@ -240,20 +300,20 @@ __global__ __launch_bounds__(64 * kForceWaves) void pg6h_force(
         ipos[3 * ic], ipos[3 * ic + 1], ipos[3 * ic + 2], (float)ivel[3 * ic],
         (float)ivel[3 * ic + 1], (float)ivel[3 * ic + 2], iid[ic], eps2, j0, min(n, j0 + piece),
         jp);
-    red[0][w][lane] = r.ax;
-    red[1][w][lane] = r.ay;
-    red[2][w][lane] = r.az;
-    red[3][w][lane] = r.pot;
-    red[4][w][lane] = r.jx;
-    red[5][w][lane] = r.jy;
-    red[6][w][lane] = r.jz;
+    red[0][threadIdx.x] = r.ax;
+    red[1][threadIdx.x] = r.ay;
+    red[2][threadIdx.x] = r.az;
+    red[3][threadIdx.x] = r.pot;
+    red[4][threadIdx.x] = r.jx;
+    red[5][threadIdx.x] = r.jy;
+    red[6][threadIdx.x] = r.jz;
     __syncthreads();
-    if (threadIdx.x < 7 * 64) {
-      const int c = threadIdx.x / 64;
+    const int slot = threadIdx.x / kRec, c = threadIdx.x % kRec;
+    const int k = tile * 64 + slot;
+    if (c < 7 && k < nact) {
       double sum = 0.0;
-      for (int q = 0; q < kForceWaves; ++q) sum += red[c][q][lane];
-      const int k = tile * 64 + lane;
-      if (k < nact) dst[c][(size_t)sp * pl.stride + k] = sum;
+      for (int q = 0; q < kForceWaves; ++q) sum += red[c][q * 64 + slot];
+      part[((size_t)sp * pl.stride + k) * kRec + c] = sum;
     }
     __syncthreads();
   }
@@ -283,43 +343,42 @@ __device__ inline void store_j(const State& S, int i, pg6::JState js) {
 }
 
 // ---------------------------------------------------------------- corrector
-// correct (hermite.c:66-110) and dt_criterion (timestep.c:50-79) for active
-// slot k = particle i, given its forces f = {ax, ay, az, pot, jx, jy, jz} at
-// the predicted position and velocity (ipos, ivel); then the j-memory
-// update.  A step that ends the dtmax window stores t = 0 (reset_time,
-// timestep.c:166-174: every particle is active then).  Returns the new
-// t + dt.
-__device__ inline double correct_one(int k, int i, const State& S, const Params& P,
-                                   const double* __restrict__ ipos,
-                                   const double* __restrict__ ivel, const double f[7],
-                                   const pg6::JState& js, int* bad) {
+// What the corrector needs of active slot k = particle i, in lane d of four:
+// the axis d (lane 3 repeats the last).
+struct Own {
+  double a0, j0, x1, v1, t, dts, m;
+};
+
+__device__ inline Own load_own(int k, int i, int d, const State& S,
+                               const double* __restrict__ ipos, const double* __restrict__ ivel) {
+  const size_t e = 3 * (size_t)i + min(d, 2), g = 3 * (size_t)k + min(d, 2);
+  return {S.a[e], S.j[e], ipos[g], ivel[g], S.t[i], S.dt[i], S.m[i]};
+}
+
+// correct (hermite.c:66-110) and dt_criterion (timestep.c:50-79) for the
+// particle i of four lanes, lane d < 3 with its axis and the force a1 and jerk
+// j1 along it, lane 3 with a1 = the potential; then the j-memory update.  A
+// step that ends the dtmax window stores t = 0 (reset_time, timestep.c:166-174:
+// every particle is active then).  Returns the new t + dt.
+__device__ inline double correct_quad(const Own& o, int i, int d, double a1, double j1,
+                                      const State& S, const Params& P, const pg6::JState& js,
+                                      int* bad) {
 #pragma clang fp contract(off)
-  const double dts = S.dt[i];
-  const double ts = S.t[i] + dts;  // p0.t (hermite.c:154)
+  const double dts = o.dts, a0 = o.a0, j0 = o.j0;
+  const double ts = o.t + dts;  // p0.t (hermite.c:154)
   const double dtsinv = 1.0 / dts;
-  const double a1[3] = {f[0], f[1], f[2]};
-  const double j1[3] = {f[4], f[5], f[6]};
-  double s0[3], c0[3], x1[3], v1[3];
-  for (int d = 0; d < 3; ++d) {
-    const double a0 = S.a[3 * i + d], j0 = S.j[3 * i + d];
-    x1[d] = ipos[3 * k + d];
-    v1[d] = ivel[3 * k + d];
-    s0[d] = 2.0 * (-3.0 * (a0 - a1[d]) - (2.0 * j0 + j1[d]) * dts) * dtsinv * dtsinv;
-    c0[d] = 6.0 * (2.0 * (a0 - a1[d]) + (j0 + j1[d]) * dts) * dtsinv * dtsinv * dtsinv;
-    x1[d] += s0[d] * dts * dts * dts * dts * kFourth + c0[d] * dts * dts * dts * dts * dts * kFifth;
-    v1[d] += s0[d] * dts * dts * dts * kThird + c0[d] * dts * dts * dts * dts * kFourth;
-  }
+  const double s0 = 2.0 * (-3.0 * (a0 - a1) - (2.0 * j0 + j1) * dts) * dtsinv * dtsinv;
+  const double c0 = 6.0 * (2.0 * (a0 - a1) + (j0 + j1) * dts) * dtsinv * dtsinv * dtsinv;
+  double x1 = o.x1, v1 = o.v1;
+  x1 += s0 * dts * dts * dts * dts * kFourth + c0 * dts * dts * dts * dts * dts * kFifth;
+  v1 += s0 * dts * dts * dts * kThird + c0 * dts * dts * dts * dts * kFourth;
   // dt_criterion
-  double s1[3];
-  for (int d = 0; d < 3; ++d) s1[d] = s0[d] + c0[d] * dts;
-  double acc = a1[0] * a1[0] + a1[1] * a1[1] + a1[2] * a1[2];
-  double jrk = j1[0] * j1[0] + j1[1] * j1[1] + j1[2] * j1[2];
-  double snp = s1[0] * s1[0] + s1[1] * s1[1] + s1[2] * s1[2];
-  double crc = c0[0] * c0[0] + c0[1] * c0[1] + c0[2] * c0[2];
-  acc = sqrt(acc);
-  jrk = sqrt(jrk);
-  snp = sqrt(snp);
-  crc = sqrt(crc);
+  const double s1 = s0 + c0 * dts;
+  auto norm = [](double e) {  // of the three axes' values
+    const double q = e * e;
+    return sqrt(dpp<0x00>(q) + dpp<0x55>(q) + dpp<0xAA>(q));
+  };
+  const double acc = norm(a1), jrk = norm(j1), snp = norm(s1), crc = norm(c0);
   const double dti = P.eta * sqrt((acc * snp + jrk * jrk) / (jrk * crc + snp * snp));
   double dtn = dts;
   if (dti < dtn) {
@@ -327,70 +386,99 @@ __device__ inline double correct_one(int k, int i, const State& S, const Params&
   } else if (dti > 2.0 * dtn) {
     if (calc_modulus(ts, 2.0 * dtn, P.dtmax) == 0.0) dtn = 2.0 * dtn;
   }
-  if (!(dtn >= P.dtmin)) atomicAdd(bad, 1);
-  for (int d = 0; d < 3; ++d) {
-    S.x[3 * i + d] = x1[d];
-    S.v[3 * i + d] = v1[d];
-    S.a[3 * i + d] = a1[d];
-    S.j[3 * i + d] = j1[d];
-  }
-  S.pot[i] = f[3];
   const double tnew = ts == P.dtmax ? 0.0 : ts;
-  S.t[i] = tnew;
-  S.dt[i] = dtn;
-  store_j(S, i, js);
+  const double over2 = 0.5, over6 = 1.0 / 6.0;  // of the j-memory, as store_j
+  if (d == 3) {
+    if (!(dtn >= P.dtmin)) atomicAdd(bad, 1);
+    S.pot[i] = a1;
+    S.t[i] = tnew;
+    S.dt[i] = dtn;
+    js.m[i] = o.m;
+    js.t[i] = tnew;
+    js.idx[i] = i;
+  } else {
+    const size_t e = 3 * (size_t)i + d;
+    S.x[e] = x1;
+    S.v[e] = v1;
+    S.a[e] = a1;
+    S.j[e] = j1;
+    (d == 0 ? js.x : d == 1 ? js.y : js.z)[i] = x1;
+    (d == 0 ? js.vx : d == 1 ? js.vy : js.vz)[i] = v1;
+    (d == 0 ? js.ax : d == 1 ? js.ay : js.az)[i] = a1 * over2;
+    (d == 0 ? js.kx : d == 1 ? js.ky : js.kz)[i] = j1 * over6;
+  }
   return tnew + dtn;
 }
 
-// Sums each active particle's j-range partials in a fixed order (one thread
+// Sums each active particle's j-range partials in a fixed order (four lanes
 // per particle for up to 16 ranges, one wavefront per particle with a fixed
-// butterfly for more), applies correct_one, folds the new t + dt into
-// Ctl::tmin_next, and lets the last block to finish close the step in Ctl.
-// Block = 256 threads.
-__global__ __launch_bounds__(256) void pg6h_finish(int n, Params P, Ctl* ctl, int target,
-                                                   int min_jper, const int* __restrict__ act,
-                                                   State S, const double* __restrict__ ipos,
+// butterfly for more), corrects it (correct_quad), and leaves in mins[], one
+// value per wavefront, the smallest new t + dt and of rest[nrest]; block 0
+// closes the step in Ctl.
+//
+// Half of the steps of 16384 particles move up to 7, so this is a chain of
+// latencies: the list, the particle and its partials in one flight, the sums,
+// the corrector with an axis per lane.  No step ends in atomics: the next
+// pg6h_select takes the minimum of mins[].  5 us a step, the integration of
+// 16384 particles 22 us a step; one lane a particle, each component's partials
+// apart, an atomic minimum and a count of the blocks that are done took 10 us
+// and 28.
+__global__ __launch_bounds__(256) void pg6h_finish(Params P, Ctl* ctl, Split split,
+                                                   const int* __restrict__ act, State S,
+                                                   const double* __restrict__ ipos,
                                                    const double* __restrict__ ivel,
-                                                   pg6::Partials part, pg6::JState js) {
+                                                   const double* __restrict__ part,
+                                                   const double* __restrict__ rest, int nrest,
+                                                   double* __restrict__ mins, pg6::JState js) {
 #pragma clang fp contract(off)
-  if (pg6h_skip(ctl, P.dtmax)) return;
-  const int nact = ctl->nact;
-  const double tnext = __longlong_as_double((long long)ctl->tmin);
-  const Plan pl = pg6h_plan(nact, n, target, min_jper);
-  const double* src[7] = {part.ax, part.ay, part.az, part.pot, part.jx, part.jy, part.jz};
-  double tmin = 1e300;  // smallest new t + dt seen by this thread
+  if (!ctl->run) return;
+  const int turn = ctl->turn;
+  const int nact = turn ? ctl->nact[1] : ctl->nact[0];
+  const int lane = threadIdx.x & 63;
+  // the block's wavefronts are those of distant particles: few ones spread over the CUs
+  const int w = (threadIdx.x / 64) * gridDim.x + blockIdx.x, nw = 4 * gridDim.x;
+  double tmin = kNoTime;
+  for (int b = w + nw * lane; b < nrest; b += nw * 64) tmin = fmin(tmin, rest[b]);
+  const Plan pl = pg6h_plan(nact, split);
+  const int d = lane & 3;
   if (pl.ns <= 16) {
-    const int k0 = blockIdx.x * blockDim.x + threadIdx.x;
-    for (int k = k0; k < nact; k += gridDim.x * blockDim.x) {
-      double f[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-      for (int sp = 0; sp < pl.ns; ++sp)
-        for (int c = 0; c < 7; ++c) f[c] += src[c][(size_t)sp * pl.stride + k];
-      tmin = fmin(tmin, correct_one(k, act[k], S, P, ipos, ivel, f, js, &ctl->bad));
+    for (int k = w * 16 + lane / 4; k < nact; k += nw * 16) {
+      const int i = act[k];
+      const Own o = load_own(k, i, d, S, ipos, ivel);
+      double a1 = 0.0, j1 = 0.0;
+      for (int sp = 0; sp < pl.ns; ++sp) {
+        const double* r = part + ((size_t)sp * pl.stride + k) * kRec + d;
+        a1 += r[0];
+        j1 += r[4];  // lane 3: unused
+      }
+      tmin = fmin(tmin, correct_quad(o, i, d, a1, j1, S, P, js, &ctl->bad));
     }
   } else {
-    const int lane = threadIdx.x & 63;
-    const int wpb = blockDim.x / 64;
-    for (int k = blockIdx.x * wpb + threadIdx.x / 64; k < nact; k += gridDim.x * wpb) {
-      double f[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-      for (int sp = lane; sp < pl.ns; sp += 64)
-        for (int c = 0; c < 7; ++c) f[c] += src[c][(size_t)sp * pl.stride + k];
-      // every lane ends with the same sums (a + b == b + a)
-      for (int o = 32; o > 0; o >>= 1)
-        for (int c = 0; c < 7; ++c) f[c] += __shfl_xor(f[c], o);
-      if (lane == 0)
-        tmin = fmin(tmin, correct_one(k, act[k], S, P, ipos, ivel, f, js, &ctl->bad));
+    for (int k = w; k < nact; k += nw) {
+      const int i = act[k];
+      double f[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      for (int sp = lane; sp < pl.ns; sp += 64) {
+        const double* r = part + ((size_t)sp * pl.stride + k) * kRec;
+        for (int c = 0; c < 7; ++c) f[c] += r[c];
+      }
+      const Own o = load_own(k, i, d, S, ipos, ivel);
+      // Butterfly over the lanes, each half of which goes on with half of
+      // the components: component c ends in the lanes 8 c to 8 c + 7.
+      for (int h = 4, x = 32; h >= 1; h >>= 1, x >>= 1)
+        for (int c = 0; c < h; ++c) {
+          const bool up = (lane & x) != 0;
+          const double keep = up ? f[c + h] : f[c], give = up ? f[c] : f[c + h];
+          f[c] = keep + __shfl_xor(give, x);
+        }
+      for (int x = 4; x >= 1; x >>= 1) f[0] += __shfl_xor(f[0], x);
+      const double a1 = __shfl(f[0], 8 * d), j1 = __shfl(f[0], 8 * (d + 4));
+      if (lane < 4) tmin = fmin(tmin, correct_quad(o, i, d, a1, j1, S, P, js, &ctl->bad));
     }
   }
-  fold_min_block(tmin, &ctl->tmin_next);
-  // The last block to get here closes the step.  It reads nothing that other
-  // blocks wrote in this kernel (only nact and t_next, read by every block
-  // before it counted itself done), so no memory fence is needed: a
-  // device-scope fence per block would write back the L2 of its XCD.
-  __shared__ int last;
-  __syncthreads();
-  if (threadIdx.x == 0) last = atomicAdd(&ctl->done, 1) == (int)gridDim.x - 1;
-  __syncthreads();
-  if (last && threadIdx.x == 0) {
+  tmin = wave_min(tmin);
+  if (lane == 0) mins[w] = tmin;
+  if (blockIdx.x == 0 && threadIdx.x == 192) {
+    const double tnext = ctl->tnext;
     ctl->last_nact = nact;
     ctl->nsteps += nact;
     ctl->nblocks += 1;
@@ -400,11 +488,7 @@ __global__ __launch_bounds__(256) void pg6h_finish(int n, Params P, Ctl* ctl, in
     } else {
       ctl->t_gl = tnext;
     }
-    ctl->nact = 0;
-    // every block's fold into tmin_next has completed (fold_min_block waits
-    // for it)
-    ctl->tmin = atomicExch(&ctl->tmin_next, kInfBits);
-    ctl->done = 0;
+    ctl->nact[1 - turn] = 0;
   }
 }
 

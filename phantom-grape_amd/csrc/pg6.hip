@@ -1562,9 +1562,11 @@ struct Hermite {
   double *ipos = nullptr, *ivel = nullptr, *acc1 = nullptr, *jrk1 = nullptr, *pot1 = nullptr;
   int* iid = nullptr;
   double* epart = nullptr;  // energy partial sums, 2 per block
-  Partials part{};
-  int target = 0, min_jper = 16;  // force split (pg6h_plan)
-  int min_blocks = 0, force_blocks = 0, finish_blocks = 0;
+  double* part = nullptr;  // pg6h::kRec per range and slot
+  double* rest = nullptr;  // per block of pg6h_select
+  double* mins = nullptr;  // per wavefront of pg6h_finish
+  pg6h::Split split{};
+  int force_blocks = 0, finish_blocks = 0;
   HostBuf host;  // pinned: a Ctl image, then t_end
   // a captured batch of kGraphSteps steps, and the board arrays it was captured with
   hipGraphExec_t graph = nullptr;
@@ -1597,12 +1599,13 @@ void hermite_enqueue(Board& b, Hermite& h, hipStream_t st) {
   const int n = h.n;
   board_use_stream(b, st);
   hipLaunchKernelGGL(pg6h::pg6h_select, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, h.S, h.P,
-                     h.ctl, b.js, b.jp, h.act, h.ipos, h.ivel, h.iid);
+                     h.ctl, h.mins, 4 * h.finish_blocks, b.js, b.jp, h.act, h.ipos, h.ivel, h.iid,
+                     h.rest);
   hipLaunchKernelGGL(pg6h::pg6h_force, dim3(h.force_blocks), dim3(64 * pg6h::kForceWaves), 0, st,
-                     n, (float)h.eps2,
-                     h.P, h.ctl, h.target, h.min_jper, h.ipos, h.ivel, h.iid, b.jp, h.part);
-  hipLaunchKernelGGL(pg6h::pg6h_finish, dim3(h.finish_blocks), dim3(256), 0, st, n, h.P, h.ctl,
-                     h.target, h.min_jper, h.act, h.S, h.ipos, h.ivel, h.part, b.js);
+                     n, (float)h.eps2, h.ctl, h.split, h.ipos, h.ivel, h.iid, b.jp, h.part);
+  hipLaunchKernelGGL(pg6h::pg6h_finish, dim3(h.finish_blocks), dim3(256), 0, st, h.P, h.ctl,
+                     h.split, h.act, h.S, h.ipos, h.ivel, h.part, h.rest, ceil_div(n, 256), h.mins,
+                     b.js);
   PGAMD_HIP_CHECK(hipGetLastError());
   b.nj_pred = -1;  // the board's predictions now belong to the integrator
   b.sort_age = kSortAge;  // its corrector moves every particle: rebuild the order
@@ -1686,14 +1689,13 @@ PGAMD_API int pg6_hermite_init(int n, const double* x, const double* v, const do
   h.P.dtmax = dtmax;
   h.P.dtmin = dtmax / std::pow(2.0, 51.0);  // initialize_timestep (timestep.c:18-22)
   const int cus = device_cu_count();
-  h.target = 16 * cus;  // wavefront items per force launch: 4 per SIMD
-  h.min_blocks = std::min(ceil_div(n, 256), 4 * cus);
+  const int target = 16 * cus;  // wavefront items per force launch: 4 per SIMD
+  h.split = pg6h::pg6h_split(n, target, 16);
   h.force_blocks = 4 * cus * 4 / pg6h::kForceWaves;  // 4 wavefronts per SIMD
-  // blocks of 256 threads: a wavefront per active particle of a typical block
-  // step (a few hundred), and few blocks to count in Ctl::done
-  h.finish_blocks = std::max(1, std::min(ceil_div(n, 256), cus));
+  // a wavefront per active particle of a step of up to 4 per CU
+  h.finish_blocks = std::min(ceil_div(n, 4), cus);
   // largest force split: ns * ntiles <= target / kForceWaves + ntiles (pg6h_plan)
-  const size_t nsplit_i = ((size_t)h.target / pg6h::kForceWaves + ceil_div(n, 64)) * 64;
+  const size_t nsplit_i = ((size_t)target / pg6h::kForceWaves + ceil_div(n, 64)) * 64;
   // state: x, v, a, j (3n each), pot, t, dt, m (n each)
   h.state.reserve(sizeof(double) * (size_t)n * 16);
   double* d = h.state.as<double>();
@@ -1705,28 +1707,27 @@ PGAMD_API int pg6_hermite_init(int n, const double* x, const double* v, const do
   h.S.t = d + 13 * (size_t)n;
   h.S.dt = d + 14 * (size_t)n;
   h.S.m = d + 15 * (size_t)n;
-  // work: ipos, ivel, acc1, jrk1 (3n each), pot1 (n), epart (2 * blocks), partials (7 *
-  // nsplit_i), Ctl; act, iid (n each)
+  // work: partials (kRec * nsplit_i; records aligned to their 64 bytes), Ctl, ipos, ivel, acc1,
+  // jrk1 (3n each), pot1 (n), epart (2 * blocks), mins (finish wavefronts), rest (select
+  // blocks); act, iid (n each)
+  const int nrest = ceil_div(n, 256), nmins = 4 * h.finish_blocks;
   const size_t dbytes =
-      sizeof(double) * ((size_t)n * 13 + 2 * kHermBlocks + 7 * nsplit_i) + 256;
+      sizeof(double) * (pg6h::kRec * nsplit_i + (size_t)n * 13 + 2 * kHermBlocks + nmins + nrest) + 256;
   const size_t ibytes = sizeof(int) * ((size_t)n * 2);
   h.work.reserve(dbytes + ibytes);
-  double* w = h.work.as<double>();
+  h.part = h.work.as<double>();
+  static_assert(sizeof(pg6h::Ctl) <= 256, "Ctl fits its slot");
+  h.ctl = reinterpret_cast<pg6h::Ctl*>(h.part + pg6h::kRec * nsplit_i);
+  double* w = reinterpret_cast<double*>(h.ctl) + 32;
   h.ipos = w;
   h.ivel = w + 3 * (size_t)n;
   h.acc1 = w + 6 * (size_t)n;
   h.jrk1 = w + 9 * (size_t)n;
   h.pot1 = w + 12 * (size_t)n;
   h.epart = w + 13 * (size_t)n;
-  double* pp = h.epart + 2 * kHermBlocks;
-  double** pf[7] = {&h.part.ax, &h.part.ay, &h.part.az, &h.part.pot,
-                    &h.part.jx, &h.part.jy, &h.part.jz};
-  for (int k = 0; k < 7; ++k) *pf[k] = pp + (size_t)k * nsplit_i;
-  h.part.rmax = nullptr;
-  h.part.nn = nullptr;
-  static_assert(sizeof(pg6h::Ctl) <= 256, "Ctl fits its slot");
-  h.ctl = reinterpret_cast<pg6h::Ctl*>(pp + 7 * nsplit_i);
-  int* wi = reinterpret_cast<int*>(reinterpret_cast<char*>(h.ctl) + 256);
+  h.mins = h.epart + 2 * kHermBlocks;
+  h.rest = h.mins + nmins;
+  int* wi = reinterpret_cast<int*>(h.rest + nrest);
   h.act = wi;
   h.iid = wi + n;
   h.host.reserve(512);
@@ -1748,8 +1749,6 @@ PGAMD_API int pg6_hermite_init(int n, const double* x, const double* v, const do
   // control block: t = 0, n particle steps and 1 block step (the start-up)
   pg6h::Ctl* c = h.host.as<pg6h::Ctl>();
   *c = pg6h::Ctl{};
-  c->tmin = pg6h::kInfBits;
-  c->tmin_next = pg6h::kInfBits;
   c->t_end = HUGE_VAL;
   c->nsteps = n;
   c->nblocks = 1;
@@ -1766,7 +1765,7 @@ PGAMD_API int pg6_hermite_init(int n, const double* x, const double* v, const do
   hermite_force(b, h, n);
   hipLaunchKernelGGL(pg6h::pg6h_startup, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, h.S, h.P,
                      h.acc1, h.jrk1, h.pot1, b.js, &h.ctl->bad);
-  hipLaunchKernelGGL(pg6h::pg6h_min_time, dim3(h.min_blocks), dim3(256), 0, st, n, h.S, h.ctl);
+  hipLaunchKernelGGL(pg6h::pg6h_min_time, dim3(h.finish_blocks), dim3(256), 0, st, n, h.S, h.mins);
   PGAMD_HIP_CHECK(hipGetLastError());
   const pg6h::Ctl r = hermite_read(h, st);
   b.predict_flag = 1;

@@ -106,28 +106,41 @@ __device__ inline double pg6_pred_vel(double dt, double v, double a2, double j6)
   return v + (2.0 * a2) * dt + (3.0 * j6) * dt * dt;
 }
 
+// The j-memory of one particle (valid = j < nj).
+struct JRaw {
+  double x, y, z, vx, vy, vz, ax, ay, az, kx, ky, kz, m, t;
+  int idx;
+};
+__device__ inline JRaw pg6_load_j(int j, bool valid, const JState& js) {
+  JRaw r{};
+  if (valid)
+    r = {js.x[j],  js.y[j],  js.z[j],  js.vx[j], js.vy[j], js.vz[j], js.ax[j], js.ay[j],
+         js.az[j], js.kx[j], js.ky[j], js.kz[j], js.m[j],  js.t[j],  js.idx[j]};
+  return r;
+}
+
 // Predicts j-particle j (valid = j < nj) to time ti into every JPred array,
 // and returns its two-float record in rec[3] (left unset if !valid).
 // Called by whole wavefronts whose lane l holds j = 64 w + l, so that the
 // wavefront fills in the id range of j-chunk w.
-__device__ inline void pg6_predict_j(int j, bool valid, double ti, const JState& js,
+__device__ inline void pg6_predict_j(int j, bool valid, double ti, const JRaw& js,
                                      const JPred& jp, float4* rec = nullptr) {
   int id = 0;
   if (valid) {
-    const double dt = ti - js.t[j];
-    const double x = pg6_pred_pos(dt, js.x[j], js.vx[j], js.ax[j], js.kx[j]);
-    const double y = pg6_pred_pos(dt, js.y[j], js.vy[j], js.ay[j], js.ky[j]);
-    const double z = pg6_pred_pos(dt, js.z[j], js.vz[j], js.az[j], js.kz[j]);
+    const double dt = ti - js.t;
+    const double x = pg6_pred_pos(dt, js.x, js.vx, js.ax, js.kx);
+    const double y = pg6_pred_pos(dt, js.y, js.vy, js.ay, js.ky);
+    const double z = pg6_pred_pos(dt, js.z, js.vz, js.az, js.kz);
     jp.x[j] = x;
     jp.y[j] = y;
     jp.z[j] = z;
     float4 vm;
-    vm.x = (float)pg6_pred_vel(dt, js.vx[j], js.ax[j], js.kx[j]);
-    vm.y = (float)pg6_pred_vel(dt, js.vy[j], js.ay[j], js.ky[j]);
-    vm.z = (float)pg6_pred_vel(dt, js.vz[j], js.az[j], js.kz[j]);
-    vm.w = (float)js.m[j];
+    vm.x = (float)pg6_pred_vel(dt, js.vx, js.ax, js.kx);
+    vm.y = (float)pg6_pred_vel(dt, js.vy, js.ay, js.ky);
+    vm.z = (float)pg6_pred_vel(dt, js.vz, js.az, js.kz);
+    vm.w = (float)js.m;
     jp.vm[j] = vm;
-    id = js.idx[j];
+    id = js.idx;
     jp.id[j] = id;
     const float hx = (float)x, hy = (float)y, hz = (float)z;
     float4* r = jp.rec + 3 * (size_t)j;
@@ -151,6 +164,10 @@ __device__ inline void pg6_predict_j(int j, bool valid, double ti, const JState&
     hi = max(hi, __shfl_xor(hi, o));
   }
   if ((j % kChunk) == 0 && valid) jp.crange[j / kChunk] = make_int2(lo, hi);
+}
+__device__ inline void pg6_predict_j(int j, bool valid, double ti, const JState& js,
+                                     const JPred& jp, float4* rec = nullptr) {
+  pg6_predict_j(j, valid, ti, pg6_load_j(j, valid, js), jp, rec);
 }
 
 // Block = 256 threads, one j per thread.
