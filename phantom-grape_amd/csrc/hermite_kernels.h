@@ -274,6 +274,39 @@ __global__ __launch_bounds__(256) void pg6h_select(int n, State S, Params P, Ctl
 }
 
 // ---------------------------------------------------------------- force
+// pg6::pg6_range_h for a range of at most kStage addresses (one tile of it),
+// the same sums: the wavefront's lanes read all records at once into its
+// `stage`, where pg6_range_h waits for scalar loads of four records after
+// four (a step's force on up to 64 particles of 16384: 4.9 us, so 6.5).  Every
+// pair is tested by id, which costs less than the loads and exchanges that
+// show where it can be left out.  Longer ranges are bound by the pairs, where
+// reading the records from LDS gained nothing.
+constexpr int kStage = 32;
+__device__ inline pg6::RangeSums short_range(double xi, double yi, double zi, float vxi, float vyi,
+                                             float vzi, int idi, float eps2, int j0, int j1,
+                                             const pg6::JPred& jp, float4* stage) {
+  const int lane = threadIdx.x & 63;
+  const float4* rec = jp.rec + 3 * (size_t)j0;
+  for (int e = lane; e < 3 * (j1 - j0); e += 64) stage[e] = rec[e];
+  const float xih = (float)xi, yih = (float)yi, zih = (float)zi;
+  const float xil = (float)(xi - (double)xih);
+  const float yil = (float)(yi - (double)yih);
+  const float zil = (float)(zi - (double)zih);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  pg6::TileAcc t{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0u};
+#pragma unroll 4
+  for (int j = 0; j < j1 - j0; ++j) {
+    const float4 a = stage[3 * j], b = stage[3 * j + 1], c = stage[3 * j + 2];
+    pg6::pg6_pair_h<true, false>(t, (a.x - xih) + (b.x - xil), (a.y - yih) + (b.y - yil),
+                                 (a.z - zih) + (b.z - zil), b.w - vxi, c.x - vyi, c.y - vzi, a.w,
+                                 eps2, __float_as_int(c.z) == idi, 0u);
+  }
+  return {(double)t.ax, (double)t.ay, (double)t.az, (double)t.pot,
+          (double)t.jx, (double)t.jy, (double)t.jz, 0.f, -1};
+}
+
 // Acc, jerk and pot of the active list against all n j-particles with the
 // two-float pair loop (pg6::pg6_range_h).  Block = kForceWaves wavefronts;
 // blocks walk the (i-tile, j-range) items of pg6h_plan.  The wavefronts'
@@ -291,15 +324,19 @@ __global__ __launch_bounds__(64 * kForceWaves) void pg6h_force(
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int piece = pl.jper / kForceWaves;
   __shared__ double red[7][kForceWaves * 64 + 8];  // the 8 spread the components over the banks
+  __shared__ float4 stage[kForceWaves][3 * kStage];
   for (int it = blockIdx.x; it < items; it += gridDim.x) {
     const int sp = pl.ntiles == 1 ? it : it / pl.ntiles, tile = it - sp * pl.ntiles;
     const int i = tile * 64 + lane;
     const int ic = i < nact ? i : nact - 1;  // padding lanes repeat the last slot
-    const int j0 = min(n, sp * pl.jper + w * piece);
-    const pg6::RangeSums r = pg6::pg6_range_h<false>(
-        ipos[3 * ic], ipos[3 * ic + 1], ipos[3 * ic + 2], (float)ivel[3 * ic],
-        (float)ivel[3 * ic + 1], (float)ivel[3 * ic + 2], iid[ic], eps2, j0, min(n, j0 + piece),
-        jp);
+    const int j0 = min(n, sp * pl.jper + w * piece), j1 = min(n, j0 + piece);
+    const double x = ipos[3 * ic], y = ipos[3 * ic + 1], z = ipos[3 * ic + 2];
+    const float vx = (float)ivel[3 * ic], vy = (float)ivel[3 * ic + 1],
+                vz = (float)ivel[3 * ic + 2];
+    const pg6::RangeSums r =
+        piece <= kStage
+            ? short_range(x, y, z, vx, vy, vz, iid[ic], eps2, j0, j1, jp, stage[w])
+            : pg6::pg6_range_h<false>(x, y, z, vx, vy, vz, iid[ic], eps2, j0, j1, jp);
     red[0][threadIdx.x] = r.ax;
     red[1][threadIdx.x] = r.ay;
     red[2][threadIdx.x] = r.az;
