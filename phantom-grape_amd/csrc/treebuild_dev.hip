@@ -79,46 +79,80 @@ struct Mem {
 };
 
 // out[n] = out[n - 1] + in[n - 1] (0 for n = 0): the total of an exclusive
-// scan, also written to *host (mapped pinned memory).
+// scan, also written to *host (mapped pinned memory) unless it is null.
 __global__ void k_scan_total(const int* __restrict__ in, int* __restrict__ out, int n,
                              int* __restrict__ host) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     const int t = n > 0 ? out[n - 1] + in[n - 1] : 0;
     out[n] = t;
-    *host = t;
+    if (host) *host = t;
   }
 }
 
-// Exclusive scan of n <= kSmallScan ints in one block: thread q sums its
-// consecutive chunk, the block scans the chunk sums, thread q writes its
-// chunk's prefixes.  out[n] = total, also written to *host.
+// Exclusive scan of n <= kSmallScan ints in one block: all of a thread's
+// loads (four consecutive ints of every tile) go out together, wavefronts scan
+// their part of each tile, the block scans the wavefronts' sums.  out[n] =
+// total, also written to *host (unless null).  14029 ints: 5 us; the library's
+// scan and a launch for the total take 9, in three launches.
 constexpr int kSmallScanThreads = 1024;
-constexpr int kSmallScan = 4 * kSmallScanThreads;
+constexpr int kScanTiles = 8;
+constexpr int kSmallScan = 4 * kSmallScanThreads * kScanTiles;
 __global__ __launch_bounds__(kSmallScanThreads) void k_scan_small(const int* __restrict__ in,
                                                                   int* __restrict__ out, int n,
                                                                   int* __restrict__ host) {
-  __shared__ int s[kSmallScanThreads];
-  const int q = threadIdx.x;
-  const int per = (n + kSmallScanThreads - 1) / kSmallScanThreads;
-  const int a = min(n, q * per), b = min(n, a + per);
-  int sum = 0;
-  for (int i = a; i < b; ++i) sum += in[i];
-  s[q] = sum;
+  constexpr int kWaves = kSmallScanThreads / 64, kSums = kWaves * kScanTiles;
+  __shared__ int s[kSums];  // tile by tile
+  const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+  int v[kScanTiles][4], end[kScanTiles];
+#pragma unroll
+  for (int t = 0; t < kScanTiles; ++t) {
+    const int i = 4 * (t * kSmallScanThreads + (int)threadIdx.x);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[t][q] = i + q < n ? in[i + q] : 0;
+  }
+#pragma unroll
+  for (int t = 0; t < kScanTiles; ++t) {
+    if (4 * t * kSmallScanThreads < n) {  // uniform
+      int e = v[t][0] + v[t][1] + v[t][2] + v[t][3];
+      for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(e, o);
+        if (lane >= o) e += x;
+      }
+      end[t] = e;
+      if (lane == 63) s[t * kWaves + wave] = e;
+    } else if (lane == 63) {
+      s[t * kWaves + wave] = 0;
+    }
+  }
   __syncthreads();
-  for (int d = 1; d < kSmallScanThreads; d <<= 1) {  // inclusive Hillis-Steele scan
-    const int v = q >= d ? s[q - d] : 0;
-    __syncthreads();
-    s[q] += v;
-    __syncthreads();
+  if (wave == 0) {  // inclusive scan of the sums
+    int run = 0;
+    for (int k = 0; k < kSums; k += 64) {
+      int e = s[k + lane];
+      for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(e, o);
+        if (lane >= o) e += x;
+      }
+      s[k + lane] = run + e;
+      run += __builtin_amdgcn_readlane(e, 63);
+    }
+    if (lane == 0) {
+      out[n] = run;
+      if (host) *host = run;
+    }
   }
-  int run = s[q] - sum;  // exclusive prefix of this chunk
-  for (int i = a; i < b; ++i) {
-    out[i] = run;
-    run += in[i];
-  }
-  if (q == kSmallScanThreads - 1) {
-    out[n] = s[q];
-    *host = s[q];
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < kScanTiles; ++t) {
+    if (4 * t * kSmallScanThreads >= n) break;
+    const int k = t * kWaves + wave;
+    int at = (k > 0 ? s[k - 1] : 0) + end[t] - (v[t][0] + v[t][1] + v[t][2] + v[t][3]);
+    const int i = 4 * (t * kSmallScanThreads + (int)threadIdx.x);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (i + q < n) out[i + q] = at;
+      at += v[t][q];
+    }
   }
 }
 
@@ -135,10 +169,18 @@ struct Lists {
   double* cells = nullptr;  // [ncells][10]
 };
 
-// Pinned ints for scan totals and other counts a kernel reports to the host;
-// builds run one at a time under the library's mutex.
+// Pinned ints in which kernels report counts to the host; builds run one at a
+// time under the library's mutex.
 constexpr int kHostInts = 64;
-int* scan_total_host() {
+enum HostSlot {
+  kSlotLevels = 0,  // k_tree_levels
+  kSlotTotal = 32,  // scan totals
+  kSlotTotal2 = 33,
+  kSlotPool = 34,  // OpenPool::used
+  kSlotWork = 40,  // two 64-bit sums
+  kSlotBox = 48,   // six doubles
+};
+int* host_ints() {
   static int* p = nullptr;
   if (!p) PGAMD_HIP_CHECK(hipHostMalloc((void**)&p, kHostInts * sizeof(int), hipHostMallocMapped));
   return p;
@@ -150,10 +192,10 @@ int* host_dev(int* host) {
 }
 
 // Sorts of fewer pairs go to the library (its one-block and merge sorts), of
-// more to radix_sort.h: whole builds of 2^17 particles take 423 us (TreePM)
-// and 449 (Barnes-Hut) with the library's sorts, 421 and 482 with those; of
-// 2^18 particles 556 and 544 against 465 and 552, of 2^19 664 and 690 against
-// 510 and 649.
+// more to radix_sort.h: whole builds of 2^17 particles take 378 us (TreePM)
+// and 400 (Barnes-Hut) with the library's sorts, 348 and 418 with those; of
+// 2^18 particles 505 and 497 against 380 and 488, of 2^19 610 and 636 against
+// 429 and 584.
 constexpr int kCountingFrom = 1 << 18;
 // The upper bits of a 63-bit Morton key that are sorted first: they tell
 // apart cells of 2^-13 of the box, so few particles are left equal.
@@ -193,34 +235,24 @@ struct Build {
     }
     return cub;
   }
-  template <class T>
-  T read(const T* d) {
-    T v;
-    PGAMD_HIP_CHECK(hipMemcpyAsync(&v, d, sizeof(T), hipMemcpyDeviceToHost, st));
-    PGAMD_HIP_CHECK(hipStreamSynchronize(st));
-    return v;
-  }
-  // out[k] = sum in[0..k) for k < n, not waited for.
-  void scan_async(const int* in, int* out, int n) {
-    size_t b = 0;
-    PGAMD_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, b, in, out, n, st));
-    PGAMD_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(cub_tmp(b), b, in, out, n, st));
-  }
-  // out[k] = sum in[0..k), out[n] = total (out has n + 1 entries); returns
-  // total.  The total comes back through mapped pinned memory: one kernel and
-  // a synchronisation for small n, the hipCUB scan for large n.
-  int scan(const int* in, int* out, int n) {
-    int* host = scan_total_host();
-    int* dev = host_dev(host);
+  // out[k] = sum in[0..k), out[n] = total (out has n + 1 entries), not waited
+  // for; the total goes to the host's slot (-1: none) through mapped memory.
+  void scan(const int* in, int* out, int n, int slot) {
+    int* dev = slot < 0 ? nullptr : host_dev(host_ints()) + slot;
     if (n <= kSmallScan) {
       hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kSmallScanThreads), 0, st, in, out, n, dev);
     } else {
-      scan_async(in, out, n);
+      size_t b = 0;
+      PGAMD_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, b, in, out, n, st));
+      PGAMD_HIP_CHECK(hipcub::DeviceScan::ExclusiveSum(cub_tmp(b), b, in, out, n, st));
       hipLaunchKernelGGL(k_scan_total, dim3(1), dim3(64), 0, st, in, out, n, dev);
     }
     PGAMD_HIP_CHECK(hipGetLastError());
+  }
+  // What the kernels queued so far have reported.
+  const volatile int* wait() {
     PGAMD_HIP_CHECK(hipStreamSynchronize(st));
-    return *static_cast<volatile int*>(host);
+    return host_ints();
   }
   // Stable library sort of (key, value) pairs.
   template <class K>
@@ -235,35 +267,29 @@ struct Build {
   // Stable sort of n keys (overwritten) by bits [0, bits) with the values 0
   // .. n - 1: *skey and *perm are set to the sorted arrays.  Only the upper
   // `first` bits take counting passes; pairs they leave equal are put in
-  // order by one more launch.  Returns the device flag (null if there is
-  // none) that it sets if a run of them is too long for that: the caller, with
-  // its next read-back, then sorts again with first = bits.
+  // order by one more launch.  *long_run (0 before) is set if a run of them is
+  // too long for that: the caller, with its next read-back, then sorts again
+  // with first = bits.
   template <class K>
-  int* sort_keys(K* key, int n, int bits, int first, K** skey, int** perm) {
+  void sort_keys(K* key, int n, int bits, int first, K** skey, int** perm, int* long_run) {
     K* k[2] = {key, tmp.get<K>(n)};
     int* v[2] = {tmp.get<int>(n), tmp.get<int>(n)};
+    int cur = 1;
     if (n < kCountingFrom) {
       hipLaunchKernelGGL(k_iota, grid_for(n), dim3(256), 0, st, n, v[0]);
       sort_pairs(k[0], k[1], v[0], v[1], n, bits);
-      *skey = k[1];
-      *perm = v[1];
-      return nullptr;
-    }
-    int* scratch = tmp.get<int>(pgsort::scratch_ints(n) + 1);
-    int* long_run = nullptr;
-    const int shift = std::max(0, bits - first);
-    int cur = pgsort::radix_sort(n, k, v, shift, bits, scratch, st);
-    if (shift > 0) {
-      long_run = scratch + pgsort::scratch_ints(n);
-      hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, 1, 0, long_run);
-      hipLaunchKernelGGL(pgsort::radix_finish<K>, grid_for(n), dim3(256), 0, st, n, shift, k[cur],
-                         v[cur], k[1 - cur], v[1 - cur], long_run);
-      cur = 1 - cur;
+    } else {
+      const int shift = std::max(0, bits - first);
+      cur = pgsort::radix_sort(n, k, v, shift, bits, tmp.get<int>(pgsort::scratch_ints(n)), st);
+      if (shift > 0) {
+        hipLaunchKernelGGL(pgsort::radix_finish<K>, grid_for(n), dim3(256), 0, st, n, shift,
+                           k[cur], v[cur], k[1 - cur], v[1 - cur], long_run);
+        cur = 1 - cur;
+      }
     }
     PGAMD_HIP_CHECK(hipGetLastError());
     *skey = k[cur];
     *perm = v[cur];
-    return long_run;
   }
 };
 
@@ -286,9 +312,10 @@ __device__ inline u64 spread3(u64 v) {
 }
 
 __global__ void k_keys(int n, const double* __restrict__ x, double lo0, double lo1, double lo2,
-                       double s, u64* __restrict__ key) {
+                       double s, u64* __restrict__ key, int* __restrict__ long_run) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) *long_run = 0;  // for sort_keys
   if (i >= n) return;
   const double lo[3] = {lo0, lo1, lo2};
   u64 k = 0;
@@ -457,16 +484,12 @@ __global__ __launch_bounds__(256) void k_tree_count(int n, const u64* __restrict
 
 // host[l] = first node of level l, host[kTreeLevels] = number of nodes, from
 // the scan of k_tree_count's counts (nb blocks), and host[kTreeLevels + 1] =
-// *flag (0 for a null one).
-__global__ void k_tree_levels(int nb, const int* __restrict__ count, const int* __restrict__ first,
-                              const int* __restrict__ flag, int* __restrict__ host) {
+// *flag.
+__global__ void k_tree_levels(int nb, const int* __restrict__ first, const int* __restrict__ flag,
+                              int* __restrict__ host) {
   const int l = threadIdx.x;
-  if (l == kTreeLevels + 1) host[l] = flag ? *flag : 0;
-  if (l < kTreeLevels) host[l] = first[(size_t)l * nb];
-  if (l == kTreeLevels) {
-    const size_t e = (size_t)kTreeLevels * nb - 1;
-    host[l] = first[e] + count[e];
-  }
+  if (l == kTreeLevels + 1) host[l] = *flag;
+  if (l <= kTreeLevels) host[l] = first[(size_t)l * nb];
 }
 
 // Nodes' first particle, level and parent, and the parents' child links
@@ -733,41 +756,76 @@ __global__ void k_group_ilist(int ng, const int* __restrict__ gnode, Nodes nd,
 }
 
 // ------------------------------------------------------------ TreePM
-__global__ void k_ghost_count(int n, const double* __restrict__ pos, double rcut,
-                              int* __restrict__ cnt) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
+// Periodic images of particle p within rcut of the box.
+__device__ inline int ghosts_of(const double* __restrict__ pos, int p, double rcut) {
   int c = 1;
   for (int d = 0; d < 3; ++d) {
-    const double v = pos[3 * p + d];
+    const double v = pos[3 * (size_t)p + d];
     c *= 1 + (v >= 1.0 - rcut ? 1 : 0) + (v < rcut ? 1 : 0);
   }
-  cnt[p] = c - 1;
+  return c - 1;
 }
 
-__global__ void k_ghost_fill(int n, const int* __restrict__ goff, double rcut,
-                             double* __restrict__ pos, int* __restrict__ src) {
-#pragma clang fp contract(off)
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const double x0 = pos[3 * p], x1 = pos[3 * p + 1], x2 = pos[3 * p + 2];
-  int lo_s[3], hi_s[3];
-  const double xp[3] = {x0, x1, x2};
-  for (int d = 0; d < 3; ++d) {
-    lo_s[d] = xp[d] >= 1.0 - rcut ? -1 : 0;
-    hi_s[d] = xp[d] < rcut ? 1 : 0;
+// Inclusive scan of v over a block of 256 threads.
+__device__ inline int scan256(int v) {
+  __shared__ int s[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int x = __shfl_up(v, o);
+    if (lane >= o) v += x;
   }
-  int o = n + goff[p];
-  for (int sx = lo_s[0]; sx <= hi_s[0]; ++sx)
-    for (int sy = lo_s[1]; sy <= hi_s[1]; ++sy)
-      for (int sz = lo_s[2]; sz <= hi_s[2]; ++sz) {
-        if (!sx && !sy && !sz) continue;
-        pos[3 * o + 0] = x0 + sx;
-        pos[3 * o + 1] = x1 + sy;
-        pos[3 * o + 2] = x2 + sz;
-        src[o] = src[p];
-        ++o;
-      }
+  __syncthreads();
+  if (lane == 63) s[wave] = v;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) v += s[w];
+  return v;
+}
+
+// Ghosts per block of kGhostBlock particles, four consecutive ones a thread.
+constexpr int kGhostBlock = 1024;
+__global__ __launch_bounds__(256) void k_ghost_count(int n, const double* __restrict__ pos,
+                                                     double rcut, int* __restrict__ cnt) {
+  const int p0 = blockIdx.x * kGhostBlock + 4 * threadIdx.x;
+  int c = 0;
+  for (int q = 0; q < 4; ++q)
+    if (p0 + q < n) c += ghosts_of(pos, p0 + q, rcut);
+  c = scan256(c);
+  if (threadIdx.x == 255) cnt[blockIdx.x] = c;
+}
+
+// Ghosts in particle order after the n particles; goff: of each block.
+__global__ __launch_bounds__(256) void k_ghost_fill(int n, const int* __restrict__ goff,
+                                                    double rcut, double* __restrict__ pos,
+                                                    int* __restrict__ src) {
+#pragma clang fp contract(off)
+  const int p0 = blockIdx.x * kGhostBlock + 4 * threadIdx.x;
+  int c[4], sum = 0;
+  for (int q = 0; q < 4; ++q) {
+    c[q] = p0 + q < n ? ghosts_of(pos, p0 + q, rcut) : 0;
+    sum += c[q];
+  }
+  size_t o = (size_t)n + goff[blockIdx.x] + scan256(sum) - sum;
+  for (int q = 0; q < 4; ++q) {
+    if (c[q] == 0) continue;
+    const size_t p = p0 + q;
+    const double x0 = pos[3 * p], x1 = pos[3 * p + 1], x2 = pos[3 * p + 2];
+    int lo_s[3], hi_s[3];
+    const double xp[3] = {x0, x1, x2};
+    for (int d = 0; d < 3; ++d) {
+      lo_s[d] = xp[d] >= 1.0 - rcut ? -1 : 0;
+      hi_s[d] = xp[d] < rcut ? 1 : 0;
+    }
+    for (int sx = lo_s[0]; sx <= hi_s[0]; ++sx)
+      for (int sy = lo_s[1]; sy <= hi_s[1]; ++sy)
+        for (int sz = lo_s[2]; sz <= hi_s[2]; ++sz) {
+          if (!sx && !sy && !sz) continue;
+          pos[3 * o + 0] = x0 + sx;
+          pos[3 * o + 1] = x1 + sy;
+          pos[3 * o + 2] = x2 + sz;
+          src[o] = src[p];
+          ++o;
+        }
+  }
 }
 
 struct Grid {
@@ -1534,6 +1592,15 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_walk(
 }
 
 // ------------------------------------------------------------ common tail
+// Clears coff[ng + 1] and ccnt[ng] (null: neither) and the two sums of k_cost.
+__global__ void k_clear(int ng, int* __restrict__ coff, int* __restrict__ ccnt,
+                        unsigned long long* __restrict__ work) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g < 2) work[g] = 0;
+  if (coff && g <= ng) coff[g] = 0;
+  if (ccnt && g < ng) ccnt[g] = 0;
+}
+
 // cost key: groups by decreasing icnt * (jcnt + 2 ccnt), ties by index.  idx:
 // the groups (to be sorted), or their ranks cleared.
 __global__ void k_cost(int ng, const int* __restrict__ icnt, const int* __restrict__ jcnt,
@@ -1619,13 +1686,14 @@ void build_octree(Build& B, Lists& R, int n, const double* x, const double* m,
   const int nb = (int)grid_for(n, kTreeBlock).x;
   int* count = B.tmp.get<int>((size_t)kTreeLevels * nb);
   int* first = B.tmp.get<int>((size_t)kTreeLevels * nb + 1);
-  int* host = scan_total_host();
+  int* long_run = B.tmp.get<int>(1);
   u64* skey = nullptr;
   for (int bits = kFirstBits;; bits = 3 * kLevels) {
-    hipLaunchKernelGGL(k_keys, grid_for(n), dim3(256), 0, st, n, x, lo[0], lo[1], lo[2], s, key);
+    hipLaunchKernelGGL(k_keys, grid_for(n), dim3(256), 0, st, n, x, lo[0], lo[1], lo[2], s, key,
+                       long_run);
     PGAMD_HIP_CHECK(hipGetLastError());
     int* perm = nullptr;
-    const int* long_run = B.sort_keys(key, n, 3 * kLevels, bits, &skey, &perm);
+    B.sort_keys(key, n, 3 * kLevels, bits, &skey, &perm, long_run);
     hipLaunchKernelGGL(k_gather, grid_for(n), dim3(256), 0, st, n, perm, x, m, R.pos, mm, R.src);
     // leaf level of every particle: the sliding maximum, in steps of at most
     // kMaxWindow (maxima over windows of u and v give one over u + v - 1)
@@ -1642,14 +1710,14 @@ void build_octree(Build& B, Lists& R, int n, const double* x, const double* m,
     }
     hipLaunchKernelGGL(k_tree_count, dim3(nb), dim3(256), 0, st, n, skey, leaf, count);
     PGAMD_HIP_CHECK(hipGetLastError());
-    B.scan_async(count, first, kTreeLevels * nb);
-    hipLaunchKernelGGL(k_tree_levels, dim3(1), dim3(64), 0, st, nb, count, first, long_run,
-                       host_dev(host));
+    B.scan(count, first, kTreeLevels * nb, -1);
+    hipLaunchKernelGGL(k_tree_levels, dim3(1), dim3(64), 0, st, nb, first, long_run,
+                       host_dev(host_ints()) + kSlotLevels);
     PGAMD_HIP_CHECK(hipGetLastError());
-    PGAMD_HIP_CHECK(hipStreamSynchronize(st));
-    if (static_cast<volatile int*>(host)[kTreeLevels + 1] == 0) break;  // no long run
+    const volatile int* host = B.wait() + kSlotLevels;
+    for (int l = 0; l < kLevels + 2; ++l) T.level.v[l] = host[l];
+    if (host[kTreeLevels + 1] == 0) break;  // no long run
   }
-  for (int l = 0; l < kLevels + 2; ++l) T.level.v[l] = static_cast<volatile int*>(host)[l];
   T.nn = T.level.v[kLevels + 1];
   Nodes& nd = T.nd;
   const size_t c = (size_t)T.nn;
@@ -1674,14 +1742,26 @@ void build_octree(Build& B, Lists& R, int n, const double* x, const double* m,
 }
 
 // Groups of the octree sorted by first particle; fills ioff/icnt/ilist.
-int build_groups(Build& B, Lists& R, const Octree& T, int ncrit, int** gnode_out) {
+// flag_groups queues their count (kSlotTotal), build_groups runs after a
+// wait().
+struct GroupFlags {
+  int *flag, *off;
+};
+GroupFlags flag_groups(Build& B, const Octree& T, int ncrit) {
+  const int nn = T.nn;
+  const GroupFlags f{B.tmp.get<int>(nn), B.tmp.get<int>(nn + 1)};
+  hipLaunchKernelGGL(k_group_flag, grid_for(nn), dim3(256), 0, B.st, nn, T.nd, ncrit, f.flag);
+  PGAMD_HIP_CHECK(hipGetLastError());
+  B.scan(f.flag, f.off, nn, kSlotTotal);
+  return f;
+}
+
+int build_groups(Build& B, Lists& R, int n, const Octree& T, const GroupFlags& f,
+                 int** gnode_out) {
   hipStream_t st = B.st;
   const int nn = T.nn;
-  int* flag = B.tmp.get<int>(nn);
-  int* off = B.tmp.get<int>(nn + 1);
-  hipLaunchKernelGGL(k_group_flag, grid_for(nn), dim3(256), 0, st, nn, T.nd, ncrit, flag);
-  PGAMD_HIP_CHECK(hipGetLastError());
-  const int ng = B.scan(flag, off, nn);
+  const int *flag = f.flag, *off = f.off;
+  const int ng = host_ints()[kSlotTotal];
   int* gn = B.tmp.get<int>(ng);
   int* gn_sorted = B.tmp.get<int>(ng);
   hipLaunchKernelGGL(k_compact, grid_for(nn), dim3(256), 0, st, nn, flag, off, gn);
@@ -1693,7 +1773,8 @@ int build_groups(Build& B, Lists& R, const Octree& T, int ncrit, int** gnode_out
   R.ioff = R.mem.get<int>(ng + 1);
   hipLaunchKernelGGL(k_group_icnt, grid_for(ng), dim3(256), 0, st, ng, gn_sorted, T.nd, R.icnt);
   PGAMD_HIP_CHECK(hipGetLastError());
-  R.ni = B.scan(R.icnt, R.ioff, ng);
+  B.scan(R.icnt, R.ioff, ng, -1);
+  R.ni = n;  // every particle is in one group
   R.ilist = R.mem.get<int>(R.ni);
   if (ng > 0)
     hipLaunchKernelGGL(k_group_ilist, dim3(ng), dim3(256), 0, st, ng, gn_sorted, T.nd, R.ioff,
@@ -1709,7 +1790,8 @@ void finish(Build& B, Lists& R, bool cells) {
   u64* key = B.tmp.get<u64>(ng);
   int* idx = B.tmp.get<int>(ng);
   unsigned long long* work = B.tmp.get<unsigned long long>(2);
-  PGAMD_HIP_CHECK(hipMemsetAsync(work, 0, 2 * sizeof(unsigned long long), st));
+  hipLaunchKernelGGL(k_clear, grid_for(cells ? 1 : ng + 1), dim3(256), 0, st, ng,
+                     cells ? nullptr : R.coff, cells ? nullptr : R.ccnt, work);
   R.order = R.mem.get<int>(ng);
   hipLaunchKernelGGL(k_cost, grid_for(ng), dim3(256), 0, st, ng, R.icnt, R.jcnt,
                      cells ? R.ccnt : nullptr, key, idx, ng <= kRankGroups, work);
@@ -1721,10 +1803,13 @@ void finish(Build& B, Lists& R, bool cells) {
     u64* skey = B.tmp.get<u64>(ng);
     B.sort_pairs(key, skey, idx, R.order, ng, 64);
   }
+  hipLaunchKernelGGL(k_copy_ints, dim3(1), dim3(64), 0, st, 4, reinterpret_cast<int*>(work),
+                     host_dev(host_ints()) + kSlotWork);
   PGAMD_HIP_CHECK(hipGetLastError());
   unsigned long long w[2];
-  PGAMD_HIP_CHECK(hipMemcpyAsync(w, work, sizeof(w), hipMemcpyDeviceToHost, st));
-  PGAMD_HIP_CHECK(hipStreamSynchronize(st));
+  const volatile int* h = B.wait() + kSlotWork;
+  for (int k = 0; k < 2; ++k)
+    w[k] = (unsigned)h[2 * k] | (unsigned long long)(unsigned)h[2 * k + 1] << 32;
   R.work_pp = (long long)w[0];
   R.work_pc = cells ? (long long)w[1] : 0;
 }
@@ -1742,16 +1827,19 @@ Lists* treepm_build(int n, const double* x, double rcut, int ncrit, hipStream_t 
   double* mm = nullptr;
   const double lo[3] = {0, 0, 0};
   build_octree(B, *R, n, x, nullptr, lo, 1.0, std::max(1, ncrit), T, &skey, &mm);
-  int* gnode = nullptr;
-  const int ng = build_groups(B, *R, T, ncrit, &gnode);
+  const GroupFlags gf = flag_groups(B, T, ncrit);
   // ghosts
-  int* gcnt = B.tmp.get<int>(n);
-  int* goff = B.tmp.get<int>(n + 1);
-  hipLaunchKernelGGL(k_ghost_count, grid_for(n), dim3(256), 0, st, n, R->pos, rcut, gcnt);
+  const int gblocks = (int)grid_for(n, kGhostBlock).x;
+  int* gcnt = B.tmp.get<int>(gblocks);
+  int* goff = B.tmp.get<int>(gblocks + 1);
+  hipLaunchKernelGGL(k_ghost_count, dim3(gblocks), dim3(256), 0, st, n, R->pos, rcut, gcnt);
   PGAMD_HIP_CHECK(hipGetLastError());
-  const int nghost = B.scan(gcnt, goff, n);
-  hipLaunchKernelGGL(k_ghost_fill, grid_for(n), dim3(256), 0, st, n, goff, rcut, R->pos, R->src);
+  B.scan(gcnt, goff, gblocks, kSlotTotal2);
+  hipLaunchKernelGGL(k_ghost_fill, dim3(gblocks), dim3(256), 0, st, n, goff, rcut, R->pos, R->src);
   PGAMD_HIP_CHECK(hipGetLastError());
+  const int nghost = B.wait()[kSlotTotal2];
+  int* gnode = nullptr;
+  const int ng = build_groups(B, *R, n, T, gf, &gnode);
   const int np = n + nghost;
   R->np = np;
   // grid over [-rcut, 1 + rcut) with cells of side >= rcut
@@ -1768,7 +1856,7 @@ Lists* treepm_build(int n, const double* x, double rcut, int ncrit, hipStream_t 
   hipLaunchKernelGGL(k_cell_of, grid_for(np), dim3(256), 0, st, np, R->pos, gr, cell);
   PGAMD_HIP_CHECK(hipGetLastError());
   const int cell_bits = bits_for(ncell);
-  B.sort_keys(cell, np, cell_bits, cell_bits, &scell, &cpart);
+  B.sort_keys(cell, np, cell_bits, cell_bits, &scell, &cpart, nullptr);
   hipLaunchKernelGGL(k_cell_start, grid_for(ncell + 1), dim3(256), 0, st, ncell, np, scell,
                      cstart);
   PGAMD_HIP_CHECK(hipGetLastError());
@@ -1786,20 +1874,20 @@ Lists* treepm_build(int n, const double* x, double rcut, int ncrit, hipStream_t 
   hipLaunchKernelGGL(k_treepm_cand, grid_for(ng, 4), dim3(256), 0, st, ng, box, gr, cstart, rcut,
                      ccand);
   PGAMD_HIP_CHECK(hipGetLastError());
-  const int ncand = B.scan(ccand, soff, ng);
+  B.scan(ccand, soff, ng, kSlotTotal);
+  const int ncand = B.wait()[kSlotTotal];
   int* scratch = B.tmp.get<int>(std::max(ncand, 1));
   hipLaunchKernelGGL(k_treepm_jlist, grid_for(ng, 4), dim3(256), 0, st, ng, box, cpos,
                      gr, cstart, cpart, rcut, R->jcnt, soff, scratch);
   PGAMD_HIP_CHECK(hipGetLastError());
-  R->nj = B.scan(R->jcnt, R->joff, ng);
+  B.scan(R->jcnt, R->joff, ng, kSlotTotal);
+  R->nj = B.wait()[kSlotTotal];
   R->jlist = R->mem.get<int>(R->nj);
   hipLaunchKernelGGL(k_pack_lists, grid_for(ng, 4), dim3(256), 0, st, ng, soff, R->jcnt, R->joff,
                      scratch, R->jlist);
   PGAMD_HIP_CHECK(hipGetLastError());
   R->coff = R->mem.get<int>(ng + 1);
   R->ccnt = R->mem.get<int>(ng);
-  PGAMD_HIP_CHECK(hipMemsetAsync(R->coff, 0, sizeof(int) * (size_t)(ng + 1), st));
-  PGAMD_HIP_CHECK(hipMemsetAsync(R->ccnt, 0, sizeof(int) * (size_t)std::max(ng, 1), st));
   R->clist = R->mem.get<int>(1);
   R->cells = R->mem.get<double>(10);
   finish(B, *R, false);
@@ -1813,13 +1901,13 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   // bounding box -> cube side, as the host builder
   const int nb = 256;
   double* part = B.tmp.get<double>(6 * nb);
-  double* bb = B.tmp.get<double>(6);
   hipLaunchKernelGGL(k_bbox_part, dim3(nb), dim3(256), 0, st, n, x, part);
-  hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(64), 0, st, nb, part, bb);
+  hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(64), 0, st, nb, part,
+                     reinterpret_cast<double*>(host_dev(host_ints()) + kSlotBox));
   PGAMD_HIP_CHECK(hipGetLastError());
   double h[6];
-  PGAMD_HIP_CHECK(hipMemcpyAsync(h, bb, sizeof(h), hipMemcpyDeviceToHost, st));
-  PGAMD_HIP_CHECK(hipStreamSynchronize(st));
+  const volatile double* box = reinterpret_cast<const volatile double*>(B.wait() + kSlotBox);
+  for (int k = 0; k < 6; ++k) h[k] = box[k];
   const double lo[3] = {h[0], h[1], h[2]};
   double L = 0;
   for (int d = 0; d < 3; ++d) L = std::max(L, h[3 + d] - h[d]);
@@ -1848,13 +1936,15 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   int* off = B.tmp.get<int>(T.nn + 1);
   hipLaunchKernelGGL(k_cell_flag, grid_for(T.nn), dim3(256), 0, st, T.nn, T.nd, flag);
   PGAMD_HIP_CHECK(hipGetLastError());
-  R->ncells = B.scan(flag, off, T.nn);
+  B.scan(flag, off, T.nn, kSlotTotal2);
+  const GroupFlags gf = flag_groups(B, T, ncrit);
+  R->ncells = B.wait()[kSlotTotal2];
   R->cells = R->mem.get<double>(10 * (size_t)R->ncells);
   hipLaunchKernelGGL(k_cell_fill, grid_for(T.nn), dim3(256), 0, st, T.nn, T.nd, flag, off,
                      R->cells);
   PGAMD_HIP_CHECK(hipGetLastError());
   int* gnode = nullptr;
-  const int ng = build_groups(B, *R, T, ncrit, &gnode);
+  const int ng = build_groups(B, *R, n, T, gf, &gnode);
   const double th2 = theta * theta;
   R->jcnt = R->mem.get<int>(ng);
   R->joff = R->mem.get<int>(ng + 1);
@@ -1882,19 +1972,25 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   hipLaunchKernelGGL(k_bh_open, wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2, pool,
                      R->jcnt, R->ccnt);
   PGAMD_HIP_CHECK(hipGetLastError());
-  R->nj = B.scan(R->jcnt, R->joff, ng);
-  int* host = scan_total_host();
-  hipLaunchKernelGGL(k_copy_ints, dim3(1), dim3(64), 0, st, 3, pool.used, host_dev(host) + 1);
+  auto offsets = [&] {
+    B.scan(R->jcnt, R->joff, ng, kSlotTotal);
+    B.scan(R->ccnt, R->coff, ng, kSlotTotal2);
+    const volatile int* host = B.wait();
+    R->nj = host[kSlotTotal];
+    R->nc = host[kSlotTotal2];
+    return host;
+  };
+  hipLaunchKernelGGL(k_copy_ints, dim3(1), dim3(64), 0, st, 3, pool.used,
+                     host_dev(host_ints()) + kSlotPool);
   PGAMD_HIP_CHECK(hipGetLastError());
-  R->nc = B.scan(R->ccnt, R->coff, ng);
-  const bool opened = static_cast<volatile int*>(host)[2] == 0;
-  const bool big = static_cast<volatile int*>(host)[3] != 0;
+  const volatile int* host = offsets();
+  const bool opened = host[kSlotPool + 1] == 0;
+  const bool big = host[kSlotPool + 2] != 0;
   if (!opened) {
     hipLaunchKernelGGL((k_bh_walk<false>), wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2,
                        R->jcnt, R->ccnt, nullptr, nullptr, nullptr, nullptr);
     PGAMD_HIP_CHECK(hipGetLastError());
-    R->nj = B.scan(R->jcnt, R->joff, ng);
-    R->nc = B.scan(R->ccnt, R->coff, ng);
+    offsets();
   }
   R->jlist = R->mem.get<int>(R->nj);
   R->clist = R->mem.get<int>(R->nc);

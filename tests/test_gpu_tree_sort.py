@@ -40,3 +40,16 @@ def test_bh_lists_ordered_by_cost(n, ncrit):
     h = pgamd.bh_lists(x, m, 1.0, ncrit, 8)
     d_x, d_m = dev(x), dev(m)
     check(h, pgamd.DevLists.bh(d_x.data_ptr(), d_m.data_ptr(), n, 1.0, ncrit, 8), True)
+
+
+# one group a particle: counts per group in tiles of 4096 of one block, up to
+# eight of them, and more; ghosts in blocks of 1024 particles
+@pytest.mark.parametrize("n", [4095, 4096, 4097, 8193, 32767, 32768, 32769])
+def test_treepm_lists_at_scan_edges(n):
+    import pgamd
+    x = np.random.default_rng(n).random((n, 3))
+    h = pgamd.treepm_lists(x, 0.04, 1)
+    d_x = dev(x)
+    L = pgamd.DevLists.treepm(d_x.data_ptr(), n, 0.04, 1)
+    assert L.info()["ngroups"] == n
+    check(h, L, False)
