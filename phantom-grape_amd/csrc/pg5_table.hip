@@ -1408,6 +1408,8 @@ struct PmCache {
   int M = 0;
   hipfftHandle fwd{}, inv{};
   int batch = 1;  // transforms per execution of inv
+  bool planes = false;  // fwd and inv over (y, z) only, pm_green_x between them
+  DevBuf twiddle;  // of pm_green_x: M factors from M on
   DevBuf rho, rhok, fk, f;
   DevBuf bricks;  // per brick: count, start; then the chunks and their number
   DevBuf place, order, part;  // per particle: place in its brick, sorted index and data
@@ -1425,6 +1427,27 @@ constexpr int kPmPerBrick = 3;
 PmCache g_pm;
 std::mutex g_pm_mutex;
 
+// Meshes whose transforms along x are pm_green_x's: the powers of two whose
+// columns fit a block.
+bool pm_by_planes(int M) { return M == 32 || M == 64 || M == 128 || M == 256; }
+
+// exp(-2 pi i j / M) for all of them, from the first octant's values.
+void pm_twiddles(PmCache& c) {
+  std::vector<double2> tw(512);
+  for (int M = 32; M <= 256; M *= 2)
+    for (int j = 0; j < M; ++j) {
+      const int r = j % (M / 4);
+      const bool low = r <= M / 8;
+      const double t = 2.0 * M_PI * (low ? r : M / 4 - r) / M;
+      const double cs = low ? std::cos(t) : std::sin(t), sn = low ? std::sin(t) : std::cos(t);
+      const double quarter[4][2] = {{cs, -sn}, {-sn, -cs}, {-cs, sn}, {sn, cs}};
+      tw[M + j] = make_double2(quarter[4 * j / M][0], quarter[4 * j / M][1]);
+    }
+  c.twiddle.reserve(sizeof(double2) * tw.size());
+  PGAMD_HIP_CHECK(
+      hipMemcpy(c.twiddle.ptr, tw.data(), sizeof(double2) * tw.size(), hipMemcpyHostToDevice));
+}
+
 void pm_setup(PmCache& c, int M) {
   if (c.M == M) return;
   if (c.M) {
@@ -1436,11 +1459,20 @@ void pm_setup(PmCache& c, int M) {
   c.rhok.reserve(sizeof(double2) * nk);
   c.fk.reserve(sizeof(double2) * nk * 3);
   c.f.reserve(sizeof(double) * nr * 3);
-  PGAMD_FFT_CHECK(hipfftPlan3d(&c.fwd, M, M, M, HIPFFT_D2Z));
-  c.batch = M <= kPmBatchMesh ? 3 : 1;
   int dims[3] = {M, M, M};
-  PGAMD_FFT_CHECK(hipfftPlanMany(&c.inv, 3, dims, nullptr, 1, 0, nullptr, 1, 0, HIPFFT_Z2D,
-                                 c.batch));
+  c.planes = pm_by_planes(M);
+  if (c.planes && !c.twiddle.ptr) pm_twiddles(c);
+  if (c.planes) {
+    c.batch = 3;
+    PGAMD_FFT_CHECK(hipfftPlanMany(&c.fwd, 2, dims, nullptr, 1, 0, nullptr, 1, 0, HIPFFT_D2Z, M));
+    PGAMD_FFT_CHECK(hipfftPlanMany(&c.inv, 2, dims, nullptr, 1, 0, nullptr, 1, 0, HIPFFT_Z2D,
+                                   3 * M));
+  } else {
+    c.batch = M <= kPmBatchMesh ? 3 : 1;
+    PGAMD_FFT_CHECK(hipfftPlan3d(&c.fwd, M, M, M, HIPFFT_D2Z));
+    PGAMD_FFT_CHECK(hipfftPlanMany(&c.inv, 3, dims, nullptr, 1, 0, nullptr, 1, 0, HIPFFT_Z2D,
+                                   c.batch));
+  }
   c.M = M;
 }
 
@@ -1530,8 +1562,19 @@ PGAMD_API int pg5t_pm_force(int n, const double* pos, const double* mass, int me
     PGAMD_HIP_CHECK(hipGetLastError());
   }
   PGAMD_FFT_CHECK(hipfftExecD2Z(c.fwd, rho, reinterpret_cast<hipfftDoubleComplex*>(rhok)));
-  hipLaunchKernelGGL(pm::pm_green, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, mesh,
-                     eps_pm, rhok, fk);
+  if (c.planes) {
+    const dim3 grid((unsigned)(nk / mesh / pm::kCols)), block(2 * mesh);
+    const double2* tw = c.twiddle.as<double2>() + mesh;
+    switch (mesh) {
+      case 32: hipLaunchKernelGGL(pm::pm_green_x<32>, grid, block, 0, st, eps_pm, tw, rhok, fk); break;
+      case 64: hipLaunchKernelGGL(pm::pm_green_x<64>, grid, block, 0, st, eps_pm, tw, rhok, fk); break;
+      case 128: hipLaunchKernelGGL(pm::pm_green_x<128>, grid, block, 0, st, eps_pm, tw, rhok, fk); break;
+      default: hipLaunchKernelGGL(pm::pm_green_x<256>, grid, block, 0, st, eps_pm, tw, rhok, fk);
+    }
+  } else {
+    hipLaunchKernelGGL(pm::pm_green, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, mesh,
+                       eps_pm, rhok, fk);
+  }
   PGAMD_HIP_CHECK(hipGetLastError());
   for (int d = 0; d < 3; d += c.batch)
     PGAMD_FFT_CHECK(hipfftExecZ2D(c.inv, reinterpret_cast<hipfftDoubleComplex*>(fk + d * nk),

@@ -343,6 +343,23 @@ __device__ inline double s2_form(double k, double a) {
 
 __device__ inline double sinc(double x) { return fabs(x) < 1e-12 ? 1.0 : sin(x) / x; }
 
+// Potential per density of a mode (kx, ky, kz) with window w = sinc sinc sinc,
+// scaled by 1/M^3; 0 for the mean and for Nyquist modes (the gradient of one
+// has no real counterpart).
+__device__ inline double green(int M, double a, double kx, double ky, double kz, double w,
+                               bool nyquist) {
+  const double k2 = kx * kx + ky * ky + kz * kz;
+  if (!(k2 > 0.0) || nyquist) return 0.0;
+  const double w3 = w * w * w;
+  const double s = s2_form(sqrt(k2), a);
+  return -4.0 * 3.14159265358979323846 * s * s / (k2 * w3 * w3) /
+         ((double)M * (double)M * (double)M);
+}
+__device__ inline double wave_number(int i, int M) {
+  const double tp = 2.0 * 3.14159265358979323846;
+  return tp * (i <= M / 2 - 1 || M == 1 ? i : i - M);
+}
+
 // rhok: M x M x (M/2+1) complex (double2); out: 3 such arrays, the
 // transformed accelerations of each axis, already scaled by 1/M^3.
 __global__ void pm_green(int M, double a, const double2* __restrict__ rhok,
@@ -354,30 +371,119 @@ __global__ void pm_green(int M, double a, const double2* __restrict__ rhok,
   const int iz = (int)(k % Mz);
   const int iy = (int)((k / Mz) % M);
   const int ix = (int)(k / ((size_t)Mz * M));
-  const double tp = 2.0 * 3.14159265358979323846;
-  const double kx = tp * (ix <= M / 2 - 1 || M == 1 ? ix : ix - M);
-  const double ky = tp * (iy <= M / 2 - 1 || M == 1 ? iy : iy - M);
-  const double kz = tp * iz;
-  const double k2 = kx * kx + ky * ky + kz * kz;
-  double2 f[3] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
-  // the gradient of a Nyquist mode has no real counterpart: dropped
-  const bool nyq = ix == M / 2 || iy == M / 2 || iz == M / 2;
-  if (k2 > 0.0 && !nyq) {
-    const double h2 = 0.5 / M;
-    const double w = sinc(kx * h2) * sinc(ky * h2) * sinc(kz * h2);
-    const double w3 = w * w * w;
-    const double s = s2_form(sqrt(k2), a);
-    const double g = -4.0 * 3.14159265358979323846 * s * s / (k2 * w3 * w3) /
-                     ((double)M * (double)M * (double)M);
-    const double2 r = rhok[k];
-    const double pr = r.x * g, pi = r.y * g;  // phi_k
-    const double kv[3] = {kx, ky, kz};
-    for (int d = 0; d < 3; ++d) {  // -i k phi = (k pi, -k pr)
-      f[d].x = kv[d] * pi;
-      f[d].y = -kv[d] * pr;
+  const double kv[3] = {wave_number(ix, M), wave_number(iy, M),
+                        2.0 * 3.14159265358979323846 * iz};
+  const double h2 = 0.5 / M;
+  const double g = green(M, a, kv[0], kv[1], kv[2],
+                         sinc(kv[0] * h2) * sinc(kv[1] * h2) * sinc(kv[2] * h2),
+                         ix == M / 2 || iy == M / 2 || iz == M / 2);
+  const double2 r = rhok[k];
+  const double pr = r.x * g, pi = r.y * g;  // phi_k
+  for (int d = 0; d < 3; ++d)               // -i k phi = (k pi, -k pr)
+    fk[d * nk + k] = make_double2(kv[d] * pi, -kv[d] * pr);
+}
+
+__device__ inline double2 cadd(double2 a, double2 b) { return {a.x + b.x, a.y + b.y}; }
+__device__ inline double2 csub(double2 a, double2 b) { return {a.x - b.x, a.y - b.y}; }
+__device__ inline double2 cmul(double2 a, double2 w) {
+  return {a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x};
+}
+
+// Forward transform of kCols columns of M = 2^p points, a thread holding the
+// points b + k M/4 of one column in v[k], before and after.  Radix-4 passes of
+// the self-sorting (Stockham) form: pass s = 1, 4, 16, ... combines the
+// points b + k M/4, which every pass reads, and leaves them at q + s (4 p + k)
+// with p = b / s, q = b % s; an odd power ends with a radix-2 pass.  s: the
+// columns in LDS; tw[j] = exp(-2 pi i j / M).
+constexpr int kCols = 8;
+template <int M>
+__device__ inline void fft_columns(double2 v[4], double2 (*s)[kCols], const double2* tw, int b,
+                                   int col) {
+#pragma unroll
+  for (int st = 1; M / st >= 4; st *= 4) {
+    const int p = b / st, q = b % st;
+    const double2 ac = cadd(v[0], v[2]), am = csub(v[0], v[2]);
+    const double2 bd = cadd(v[1], v[3]), bm = csub(v[1], v[3]);
+    const double2 jb = {-bm.y, bm.x};
+    v[0] = cadd(ac, bd);
+    v[1] = csub(am, jb);
+    v[2] = csub(ac, bd);
+    v[3] = cadd(am, jb);
+    if (M / st == 4) break;  // p = 0: in place, no factors
+#pragma unroll
+    for (int k = 1; k < 4; ++k) v[k] = cmul(v[k], tw[k * p * st]);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s[q + st * (4 * p + k)][col] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = s[b + k * (M / 4)][col];
+    if (M / st == 8) {
+      const double2 a = v[0], c = v[1];
+      v[0] = cadd(a, v[2]);
+      v[2] = csub(a, v[2]);
+      v[1] = cadd(c, v[3]);
+      v[3] = csub(c, v[3]);
+      break;
     }
   }
-  for (int d = 0; d < 3; ++d) fk[d * nk + k] = f[d];
+}
+
+// pm_green between the two transforms along x: rhok holds the density's
+// transforms over (y, z) of each x plane, and fk gets what is left to be
+// transformed back over (y, z), so that the modes pass through memory once.
+// The y and z components share their transform along x (k_y and k_z do not
+// depend on it).  Block = 2 M threads: kCols neighbouring (y, z) columns of M
+// points, M/4 threads each.
+//
+// A mesh of 128^3: 22.8 us, of which 15 would move the 17 MB read and 51 MB
+// written at the rate of a copy; the library's passes along x took 13 and
+// 25.4, pm_green 22.2 between them.  Bound: memory, with the FP64 functions of
+// green() behind it.
+template <int M>
+__global__ __launch_bounds__(2 * M) void pm_green_x(double a, const double2* __restrict__ twiddle,
+                                                    const double2* __restrict__ rhok,
+                                                    double2* __restrict__ fk) {
+  constexpr int Mz = M / 2 + 1, kStride = M * Mz;
+  static_assert(kStride % kCols == 0, "whole blocks of columns");
+  __shared__ double2 s[M][kCols];
+  __shared__ double2 tw[M];
+  __shared__ double s_sinc[M / 2 + 1];
+  const int tid = threadIdx.x, col = tid % kCols, b = tid / kCols;
+  const int c = blockIdx.x * kCols + col;
+  const double2* src = rhok + c;
+  double2 v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = src[(size_t)(b + k * (M / 4)) * kStride];
+  if (tid < M) tw[tid] = twiddle[tid];
+  if (tid <= M / 2) s_sinc[tid] = sinc(2.0 * 3.14159265358979323846 * tid * (0.5 / M));
+  __syncthreads();
+  fft_columns<M>(v, s, tw, b, col);
+  const int iy = c / Mz, iz = c % Mz;
+  const double ky = wave_number(iy, M), kz = 2.0 * 3.14159265358979323846 * iz;
+  const double wy = s_sinc[iy <= M / 2 ? iy : M - iy], wz = s_sinc[iz];
+  double2 fx[4], fp[4];  // real and imaginary parts swapped: the forward transform inverts
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int ix = b + k * (M / 4);
+    const double kx = wave_number(ix, M);
+    const double g = green(M, a, kx, ky, kz, s_sinc[ix <= M / 2 ? ix : M - ix] * wy * wz,
+                           ix == M / 2 || iy == M / 2 || iz == M / 2);
+    const double pr = v[k].x * g, pi = v[k].y * g;  // phi_k; -i k phi = (k pi, -k pr)
+    fx[k] = make_double2(-kx * pr, kx * pi);
+    fp[k] = make_double2(-pr, pi);
+  }
+  fft_columns<M>(fx, s, tw, b, col);
+  fft_columns<M>(fp, s, tw, b, col);
+  double2* dst = fk + c;
+  constexpr size_t nk = (size_t)M * kStride;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const size_t e = (size_t)(b + k * (M / 4)) * kStride;
+    dst[e] = make_double2(fx[k].y, fx[k].x);
+    dst[nk + e] = make_double2(ky * fp[k].y, ky * fp[k].x);
+    dst[2 * nk + e] = make_double2(kz * fp[k].y, kz * fp[k].x);
+  }
 }
 
 // TSC interpolation of a chunk of sorted particles: the block loads the
