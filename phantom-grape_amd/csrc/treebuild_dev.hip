@@ -847,14 +847,18 @@ __global__ void k_cell_of(int np, const double* __restrict__ pos, Grid g,
             cidx(g, pos[3 * p + 2]);
 }
 
-// Positions in cell order: cpos[k] = pos[cpart[k]], so the list walk reads
-// each row of cells as one contiguous range.
+// Candidates in cell order: cpos[k] = position of particle cpart[k] rounded to
+// FP32 and its index, so the list walk reads each row of cells as one
+// contiguous range.  *wide is set if a coordinate lies outside [-2, 2], where
+// kFineReach does not hold.
 __global__ void k_cell_pos(int np, const int* __restrict__ cpart, const double* __restrict__ pos,
-                           double* __restrict__ cpos) {
+                           float4* __restrict__ cpos, int* __restrict__ wide) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= np) return;
   const int p = cpart[k];
-  for (int d = 0; d < 3; ++d) cpos[3 * k + d] = pos[3 * p + d];
+  const double x = pos[3 * (size_t)p], y = pos[3 * (size_t)p + 1], z = pos[3 * (size_t)p + 2];
+  cpos[k] = make_float4((float)x, (float)y, (float)z, __int_as_float(p));
+  if (!(fmax(fmax(fabs(x), fabs(y)), fabs(z)) <= 2.0)) *wide = 1;
 }
 
 // cstart[c] = first position of cell c in the sorted cell array (c <= ncell).
@@ -911,20 +915,39 @@ __device__ inline bool in_reach(const double bx[6], const double v[3], double rc
   return d2 < rc2;
 }
 
+// The squared distance of in_reach in FP32, from positions and box sides of at
+// most 2 in size rounded to FP32: the sides' distances e are off by at most 3
+// roundings of 2^-23, so near the cut-off the sum of e^2 is off by less than
+// 2 sqrt(3) rcut 2^-21 + rcut^2 2^-20.  Farther from rcut^2 than `fine`, more
+// than twice that, the FP32 comparison is the FP64 one.
+__device__ inline float reach2(const float bx[6], float4 v) {
+  const float x = fmaxf(fmaxf(bx[0] - v.x, v.x - bx[3]), 0.f);
+  const float y = fmaxf(fmaxf(bx[1] - v.y, v.y - bx[4]), 0.f);
+  const float z = fmaxf(fmaxf(bx[2] - v.z, v.z - bx[5]), 0.f);
+  return x * x + y * y + z * z;
+}
+inline float fine_reach(double rcut) { return (float)(4e-6 * rcut + 4e-6 * rcut * rcut + 1e-11); }
+
 // One wavefront per group walks the grid cells around the group box and
 // writes the particles in reach to jlist[joff[g]...] and their number to
 // jcnt[g], in cell order (cells by x, y, z index; a cell's particles by
 // index).  The cells of one (x, y) row are consecutive, so a row is one range
-// of the cell-sorted particles (cpos: positions in that order).  The rows'
+// of the cell-sorted particles.  The rows'
 // ranges are read by the lanes side by side, then kJlistDepth pieces of 64
 // candidates at a time, whatever rows they belong to, so that their loads
-// overlap: row after row and one piece at a time, each waited for, the walk
-// of a 2^20-particle box took 346 us.
+// overlap.  The few candidates that FP32 cannot tell in or out (reach2; all of
+// them where *wide) are decided by the FP64 positions.
+//
+// Bound: what the L2 delivers.  2^20-particle box, 7e7 candidates: 346 us with
+// FP64 positions and one piece at a time, each waited for; 177 with four in
+// flight (28 bytes a candidate); 145 with 16 bytes a candidate.
 constexpr int kJlistDepth = 4;
 __global__ __launch_bounds__(256) void k_treepm_jlist(int ng, const double* __restrict__ box,
-                                                      const double* __restrict__ cpos, Grid gr,
+                                                      const float4* __restrict__ cpos, Grid gr,
                                                       const int* __restrict__ cstart,
-                                                      const int* __restrict__ cpart, double rcut,
+                                                      const double* __restrict__ pos,
+                                                      const int* __restrict__ wide, float fine,
+                                                      double rcut,
                                                       int* __restrict__ jcnt,
                                                       const int* __restrict__ joff,
                                                       int* __restrict__ jlist) {
@@ -940,6 +963,9 @@ __global__ __launch_bounds__(256) void k_treepm_jlist(int ng, const double* __re
     c0[d] = cidx(gr, bx[d] - rcut);
     c1[d] = cidx(gr, bx[3 + d] + rcut);
   }
+  float bf[6];
+  for (int d = 0; d < 6; ++d) bf[d] = (float)bx[d];
+  const float rc2f = (float)rc2, tol = *wide ? INFINITY : fine;
   int count = 0;
   int* out = jlist + joff[g];
   const int ny = c1[1] - c0[1] + 1, nrows = (c1[0] - c0[0] + 1) * ny;
@@ -962,8 +988,7 @@ __global__ __launch_bounds__(256) void k_treepm_jlist(int ng, const double* __re
     const int total = __builtin_amdgcn_readlane(end, 63);
     for (int p0 = 0; p0 < total; p0 += kJlistDepth) {
       bool in[kJlistDepth];
-      int part[kJlistDepth];
-      double v[kJlistDepth][3];
+      float4 v[kJlistDepth];
 #pragma unroll
       for (int u = 0; u < kJlistDepth; ++u) {
         // the row of piece p0 + u: the last that begins at or before it
@@ -973,15 +998,20 @@ __global__ __launch_bounds__(256) void k_treepm_jlist(int ng, const double* __re
                       64 * (p - __builtin_amdgcn_readlane(begin, row));
         const int k = a + lane, e = __builtin_amdgcn_readlane(k1, row);
         in[u] = p0 + u < total && k < e;
-        const size_t kk = (size_t)(k < e ? k : a);
-        part[u] = cpart[kk];
-        for (int d = 0; d < 3; ++d) v[u][d] = cpos[3 * kk + d];
+        v[u] = cpos[k < e ? k : a];
       }
 #pragma unroll
       for (int u = 0; u < kJlistDepth; ++u) {
-        const bool ok = in[u] && in_reach(bx, v[u], rc2);
+        const float d2 = reach2(bf, v[u]);
+        const int part = __float_as_int(v[u].w);
+        bool ok = in[u] && d2 < rc2f;
+        if (in[u] && !(fabsf(d2 - rc2f) > tol)) {
+          const double q[3] = {pos[3 * (size_t)part], pos[3 * (size_t)part + 1],
+                               pos[3 * (size_t)part + 2]};
+          ok = in_reach(bx, q, rc2);
+        }
         const u64 mask = __ballot(ok);
-        if (ok) out[count + __popcll(mask & below)] = part[u];
+        if (ok) out[count + __popcll(mask & below)] = part;
         count += __popcll(mask);
       }
     }
@@ -1865,8 +1895,10 @@ Lists* treepm_build(int n, const double* x, double rcut, int ncrit, hipStream_t 
   hipLaunchKernelGGL(k_group_box, grid_for(ng, 4), dim3(256), 0, st, ng, gnode, T.nd, R->pos, box);
   R->jcnt = R->mem.get<int>(ng);
   R->joff = R->mem.get<int>(ng + 1);
-  double* cpos = B.tmp.get<double>(3 * (size_t)np);
-  hipLaunchKernelGGL(k_cell_pos, grid_for(np), dim3(256), 0, st, np, cpart, R->pos, cpos);
+  float4* cpos = B.tmp.get<float4>(np);
+  int* wide = B.tmp.get<int>(1);
+  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, 1, 0, wide);
+  hipLaunchKernelGGL(k_cell_pos, grid_for(np), dim3(256), 0, st, np, cpart, R->pos, cpos, wide);
   // One walk: each group writes its list at its candidate offset (the
   // candidate count bounds the list length), then the lists are packed.
   int* ccand = B.tmp.get<int>(ng);
@@ -1878,7 +1910,7 @@ Lists* treepm_build(int n, const double* x, double rcut, int ncrit, hipStream_t 
   const int ncand = B.wait()[kSlotTotal];
   int* scratch = B.tmp.get<int>(std::max(ncand, 1));
   hipLaunchKernelGGL(k_treepm_jlist, grid_for(ng, 4), dim3(256), 0, st, ng, box, cpos,
-                     gr, cstart, cpart, rcut, R->jcnt, soff, scratch);
+                     gr, cstart, R->pos, wide, fine_reach(rcut), rcut, R->jcnt, soff, scratch);
   PGAMD_HIP_CHECK(hipGetLastError());
   B.scan(R->jcnt, R->joff, ng, kSlotTotal);
   R->nj = B.wait()[kSlotTotal];
