@@ -90,9 +90,10 @@ __global__ void k_scan_total(const int* __restrict__ in, int* __restrict__ out, 
 }
 
 // Exclusive scan of n <= kSmallScan ints in one block: all of a thread's
-// loads (four consecutive ints of every tile) go out together, wavefronts scan
+// loads (four consecutive ints of every tile; in and out are aligned to 16
+// bytes, as all allocations are) go out together, wavefronts scan
 // their part of each tile, the block scans the wavefronts' sums.  out[n] =
-// total, also written to *host (unless null).  14029 ints: 5 us; the library's
+// total, also written to *host (unless null).  14029 ints: 4 us; the library's
 // scan and a launch for the total take 9, in three launches.
 constexpr int kSmallScanThreads = 1024;
 constexpr int kScanTiles = 8;
@@ -107,8 +108,15 @@ __global__ __launch_bounds__(kSmallScanThreads) void k_scan_small(const int* __r
 #pragma unroll
   for (int t = 0; t < kScanTiles; ++t) {
     const int i = 4 * (t * kSmallScanThreads + (int)threadIdx.x);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) v[t][q] = i + q < n ? in[i + q] : 0;
+    int4 x = make_int4(0, 0, 0, 0);
+    if (i + 3 < n)
+      x = *reinterpret_cast<const int4*>(in + i);
+    else if (i < n)
+      x = make_int4(in[i], i + 1 < n ? in[i + 1] : 0, i + 2 < n ? in[i + 2] : 0, 0);
+    v[t][0] = x.x;
+    v[t][1] = x.y;
+    v[t][2] = x.z;
+    v[t][3] = x.w;
   }
 #pragma unroll
   for (int t = 0; t < kScanTiles; ++t) {
@@ -146,12 +154,16 @@ __global__ __launch_bounds__(kSmallScanThreads) void k_scan_small(const int* __r
   for (int t = 0; t < kScanTiles; ++t) {
     if (4 * t * kSmallScanThreads >= n) break;
     const int k = t * kWaves + wave;
-    int at = (k > 0 ? s[k - 1] : 0) + end[t] - (v[t][0] + v[t][1] + v[t][2] + v[t][3]);
+    const int at = (k > 0 ? s[k - 1] : 0) + end[t] - (v[t][0] + v[t][1] + v[t][2] + v[t][3]);
     const int i = 4 * (t * kSmallScanThreads + (int)threadIdx.x);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (i + q < n) out[i + q] = at;
-      at += v[t][q];
+    const int4 x = make_int4(at, at + v[t][0], at + v[t][0] + v[t][1],
+                             at + v[t][0] + v[t][1] + v[t][2]);
+    if (i + 3 < n) {
+      *reinterpret_cast<int4*>(out + i) = x;
+    } else if (i < n) {
+      out[i] = x.x;
+      if (i + 1 < n) out[i + 1] = x.y;
+      if (i + 2 < n) out[i + 2] = x.z;
     }
   }
 }
