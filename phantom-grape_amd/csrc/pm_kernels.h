@@ -15,11 +15,12 @@
 //      depend on the order in which the atomics land, nor on the order of the
 //      particles inside a brick, and the force is the same bit for bit on
 //      every run;
-//   2. real-to-complex FFT (hipFFT, FP64);
+//   2. real-to-complex FFT (FP64; hipFFT, but for the transforms along x of
+//      meshes of 32 to 256 points that are powers of two: pm_green_x);
 //   3. Green's function -4 pi S(k a)^2 / (k^2 W(k)^2), with S the S2 form
 //      factor and W the TSC window, times -i k for each axis (spectral
 //      gradient), normalised by 1/M^3;
-//   4. three complex-to-real FFTs;
+//   4. three complex-to-real FFTs (the same);
 //   5. TSC interpolation of the mesh accelerations back to the particles.
 // G = 1, uniform neutralising background (k = 0 dropped), as in Ewald
 // summation.

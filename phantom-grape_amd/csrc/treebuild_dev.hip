@@ -3,7 +3,7 @@
 //
 // Same algorithm and same output as the host builder libpgtree.so
 // (treebuild.cpp), array for array: Morton keys (21 bits per axis), a stable
-// radix sort, the octree split level by level, bottom-up moments, i-groups of
+// radix sort, the octree (its nodes level by level), bottom-up moments, i-groups of
 // <= ncrit particles in Morton order, TreePM ghosts and grid-based j-lists
 // in grid-cell order, the Barnes-Hut walk with the opening test of
 // PG5/newton_quad/source.cpp:660-707, and groups ordered by decreasing cost.
@@ -1194,7 +1194,7 @@ __device__ inline int xcd_block(int b, int nb) {
 // particles and cells go.  A depth-first walk can keep only the work of the
 // stack entries before the first one that opens children, and runs twice, the
 // first time for the list lengths: 0.67 + 0.81 ms for 2^21 particles at
-// theta = 0.5 (14029 groups that open 793 nodes on average), against 0.63 +
+// theta = 0.5 (14029 groups that open 793 nodes on average), against 0.62 +
 // 0.31 ms.  Bound: the vector cache, whose lookups and misses of the
 // children's loads (64 lanes of 32 bytes a step) a step waits for.
 //
