@@ -1194,7 +1194,7 @@ __device__ inline int xcd_block(int b, int nb) {
 // particles and cells go.  A depth-first walk can keep only the work of the
 // stack entries before the first one that opens children, and runs twice, the
 // first time for the list lengths: 0.67 + 0.81 ms for 2^21 particles at
-// theta = 0.5 (14029 groups that open 793 nodes on average), against 0.62 +
+// theta = 0.5 (14029 groups that open 793 nodes on average), against 0.22 +
 // 0.31 ms.  Bound: the vector cache, whose lookups and misses of the
 // children's loads (64 lanes of 32 bytes a step) a step waits for.
 //
@@ -1216,13 +1216,22 @@ struct OpenPool {
   int4* rec;    // [chunks][kOpenChunk]
   int4* sum;    // the same: k_bh_list's working entries of groups too large for LDS
   int* wait;    // the same: the entry at a ring position beyond the ring
-  int* used;    // [0] chunks handed out, [1] != 0: the pool or a group's table was too small,
-                // [2] != 0: some group is too large for k_bh_list's LDS
+  // [0] != 0: the pool or a group's table was too small, [1] != 0: some group
+  // is too large for k_bh_list's LDS; then, a cache line each, the chunks
+  // handed out of every part of the pool
+  int* used;
   int* chunk;   // [group][kOpenGroupChunks]
   int* level;   // [group][kOpenLevels]: first entry of each level, then the number of
                 // entries; the last int is the number of levels (0: no entries)
-  int chunks;
+  int chunks;   // of each part
 };
+// Parts of the pool with a counter of their own: a group begins with the part
+// of its number and goes on to the next where that is used up.  The 57000
+// chunks of a 2^21-particle build, taken from one counter, kept the walk
+// waiting for that address: 627 us, with 64 counters 219.
+constexpr int kPoolParts = 64;
+constexpr int kPoolLine = 32;  // ints
+constexpr int kPoolUsed = (1 + kPoolParts) * kPoolLine;
 
 // Opened children, own particles and own cells of an entry.
 __device__ inline int open_count(unsigned b) {
@@ -1267,12 +1276,17 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_open(
   int nch = 0;
   // one more chunk for this group; false: none left
   auto grow = [&]() {
-    int c = 0;
-    if (lane == 0) c = atomicAdd(&pool.used[0], 1);
-    c = __builtin_amdgcn_readfirstlane(c);
-    if (nch == kOpenGroupChunks || c >= pool.chunks) {
+    int c = -1;
+    for (int t = 0; t < kPoolParts && nch < kOpenGroupChunks && c < 0; ++t) {
+      const int part = (g + t) % kPoolParts;
+      int k = 0;
+      if (lane == 0) k = atomicAdd(&pool.used[(1 + part) * kPoolLine], 1);
+      k = __builtin_amdgcn_readfirstlane(k);
+      if (k < pool.chunks) c = part * pool.chunks + k;
+    }
+    if (c < 0) {
       if (lane == 0) {
-        pool.used[1] = 1;
+        pool.used[0] = 1;
         pcnt[g] = 0;
         ccnt[g] = 0;
         level[kOpenLevels - 1] = 0;
@@ -1399,7 +1413,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_open(
     level[kOpenLevels - 1] = nlev;
     pcnt[g] = np;
     ccnt[g] = nc;
-    if (tail > kListEntries) pool.used[2] = 1;
+    if (tail > kListEntries) pool.used[1] = 1;
   }
 }
 
@@ -2005,14 +2019,14 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   // of them, more for smaller theta (nodes within a distance 1 / theta).
   const double more = std::min(8.0, std::max(1.0, std::pow(0.5 / theta, 3)));
   OpenPool pool{};
-  pool.chunks = (int)std::min(1e6, 64.0 + 5.0 * ng * more);
-  const size_t entries = (size_t)pool.chunks * kOpenChunk;
+  pool.chunks = (int)std::ceil(std::min(1e6, 64.0 + 5.0 * ng * more) / kPoolParts);
+  const size_t entries = (size_t)pool.chunks * kPoolParts * kOpenChunk;
   pool.rec = B.tmp.get<int4>(entries);
   pool.wait = B.tmp.get<int>(entries);
-  pool.chunk = B.tmp.get<int>((size_t)ng * (kOpenGroupChunks + kOpenLevels) + 3);
+  pool.chunk = B.tmp.get<int>((size_t)ng * (kOpenGroupChunks + kOpenLevels));
   pool.level = pool.chunk + (size_t)ng * kOpenGroupChunks;
-  pool.used = pool.level + (size_t)ng * kOpenLevels;
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, 3, 0, pool.used);
+  pool.used = B.tmp.get<int>(kPoolUsed);
+  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(1024), 0, st, kPoolUsed, 0, pool.used);
   hipLaunchKernelGGL(k_bh_open, wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2, pool,
                      R->jcnt, R->ccnt);
   PGAMD_HIP_CHECK(hipGetLastError());
@@ -2024,12 +2038,12 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
     R->nc = host[kSlotTotal2];
     return host;
   };
-  hipLaunchKernelGGL(k_copy_ints, dim3(1), dim3(64), 0, st, 3, pool.used,
+  hipLaunchKernelGGL(k_copy_ints, dim3(1), dim3(64), 0, st, 2, pool.used,
                      host_dev(host_ints()) + kSlotPool);
   PGAMD_HIP_CHECK(hipGetLastError());
   const volatile int* host = offsets();
-  const bool opened = host[kSlotPool + 1] == 0;
-  const bool big = host[kSlotPool + 2] != 0;
+  const bool opened = host[kSlotPool] == 0;
+  const bool big = host[kSlotPool + 1] != 0;
   if (!opened) {
     hipLaunchKernelGGL((k_bh_walk<false>), wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2,
                        R->jcnt, R->ccnt, nullptr, nullptr, nullptr, nullptr);
