@@ -1117,14 +1117,15 @@ __device__ inline double bh_box_d2(const double* __restrict__ gc, double li,
 }
 
 // Node data the Barnes-Hut walk reads for one child: what it becomes if it is
-// opened, and its centre of mass (32 bytes), and for the lists its particle
-// range and cell index (nodes of more than one particle).  Arrays of 16 bytes
-// a node: the eight lanes that examine a node's children (numbered
+// opened, and its centre of mass (32 bytes), and for the lists its item.
+// Arrays of 16 bytes a node: the eight lanes that examine a node's children (numbered
 // consecutively in octant order) read 128 consecutive bytes of each, where
 // 64-byte records made every lane of every load a cache line of its own; the
 // walk is bound by the lookups and misses of the vector cache.
 struct WalkNodes {
-  int4* range;  // {lo, hi, cell, 0}
+  // what a list holds of the node: its cell, or its only particle (from a
+  // 16-byte record of range and cell k_bh_list took 313 us, so 288)
+  int* item;
   // {x, y} of the queue entry (below) and com x as two words
   int4* ex;
   double2* yz;  // com y, z
@@ -1164,7 +1165,7 @@ __global__ void k_walk_nodes(int nn, int nleaf, Nodes nd, WalkNodes out) {
   }
   const bool leaf = hi - lo <= nleaf || mask == 0;
   const u64 cx = (u64)__double_as_longlong(nd.com[3 * k]);
-  out.range[k] = make_int4(lo, hi, hi - lo > 1 ? nd.cell[k] : -1, 0);
+  out.item[k] = hi - lo > 1 ? nd.cell[k] : lo;
   out.ex[k] = make_int4(leaf ? lo : first, leaf ? (int)(kLeafEntry | (unsigned)(hi - lo)) : mask,
                         (int)(unsigned)cx, (int)(unsigned)(cx >> 32));
   out.yz[k] = make_double2(nd.com[3 * k + 1], nd.com[3 * k + 2]);
@@ -1195,7 +1196,7 @@ __device__ inline int xcd_block(int b, int nb) {
 // stack entries before the first one that opens children, and runs twice, the
 // first time for the list lengths: 0.67 + 0.81 ms for 2^21 particles at
 // theta = 0.5 (14029 groups that open 793 nodes on average), against 0.22 +
-// 0.31 ms.  Bound: the vector cache, whose lookups and misses of the
+// 0.29 ms.  Bound: the vector cache, whose lookups and misses of the
 // children's loads (64 lanes of 32 bytes a step) a step waits for.
 //
 // Leaves need no examining and go to the pool as they are found; the other
@@ -1425,7 +1426,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_open(
 // kListEntries in the pool.
 template <bool BIG>
 __global__ __launch_bounds__(kListThreads) void k_bh_list(
-    int ng, OpenPool pool, const int4* __restrict__ range, const int* __restrict__ poff,
+    int ng, OpenPool pool, const int* __restrict__ item, const int* __restrict__ poff,
     const int* __restrict__ coff, int* __restrict__ plist, int* __restrict__ clist) {
   __shared__ int4 s_ent[BIG ? 1 : kListEntries];
   __shared__ int s_x[BIG ? 1 : kListEntries];  // first child or particle
@@ -1489,8 +1490,8 @@ __global__ __launch_bounds__(kListThreads) void k_bh_list(
   const int o = tid & 7;
   const unsigned above = 0xffu & ~((2u << o) - 1u);  // octants listed before this one
   for (int k0 = tid >> 3; k0 < n; k0 += 4 * (kListThreads / 8)) {
-    int4 r[4], w[4];
-    int x[4];
+    int4 r[4];
+    int x[4], w[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {  // four entries' loads in flight
       const int k = k0 + u * (kListThreads / 8);
@@ -1498,7 +1499,7 @@ __global__ __launch_bounds__(kListThreads) void k_bh_list(
       x[u] = k < n ? (BIG ? pool.rec[at(k)].x : s_x[k]) : 0;
       const unsigned b = (unsigned)r[u].x;
       if (!(b & kLeafEntry) && (((b >> 8 | b >> 16) >> o) & 1u))
-        w[u] = range[x[u] + __popc(b & ((1u << o) - 1u))];
+        w[u] = item[x[u] + __popc(b & ((1u << o) - 1u))];
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -1507,9 +1508,9 @@ __global__ __launch_bounds__(kListThreads) void k_bh_list(
         const int cnt = (int)(b & ~kLeafEntry);
         for (int p = o; p < cnt; p += 8) pl[r[u].z + p] = x[u] + p;
       } else if ((m1 >> o) & 1u) {
-        pl[r[u].z + __popc(m1 & above)] = w[u].x;
+        pl[r[u].z + __popc(m1 & above)] = w[u];
       } else if ((m2 >> o) & 1u) {
-        cl[r[u].w + __popc(m2 & above)] = w[u].z;
+        cl[r[u].w + __popc(m2 & above)] = w[u];
       }
     }
   }
@@ -1526,7 +1527,7 @@ __global__ void k_bh_whole(int ng, const int* __restrict__ pcnt, const int* __re
   const int gk = gnode[g];
   const double gc[3] = {nd.c[3 * gk], nd.c[3 * gk + 1], nd.c[3 * gk + 2]};
   if (bh_box_d2(gc, 0.5 * ldexp(L, -nd.lev[gk]), load_walk(wn, 0).com) * th2 >= L * L)
-    clist[coff[g]] = wn.range[0].z;
+    clist[coff[g]] = nd.cell[0];
 }
 
 // For builds whose groups open more nodes than k_bh_open's pool or chunk
@@ -1568,7 +1569,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_walk(
   const WalkNode root = load_walk(wn, 0);
   // the whole tree as one cell (source.cpp:832-840)
   if (bh_box_d2(gc, li, root.com) * th2 >= L * L) {
-    if (FILL && lane == 0) cl[0] = wn.range[0].z;
+    if (FILL && lane == 0) cl[0] = nd.cell[0];
     nc = 1;
   } else {
     if (lane == 0)
@@ -1601,9 +1602,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_walk(
         else
           kind = 3;
         if (FILL) {
-          const int4 r = wn.range[k];
-          lo = r.x;
-          cell = r.z;
+          lo = cell = wn.item[k];
         }
       }
       // The serial walk would expand the entries from the top until one
@@ -2009,7 +2008,7 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   R->ccnt = R->mem.get<int>(ng);
   R->coff = R->mem.get<int>(ng + 1);
   WalkNodes wn;
-  wn.range = B.tmp.get<int4>(T.nn);
+  wn.item = B.tmp.get<int>(T.nn);
   wn.ex = B.tmp.get<int4>(T.nn);
   wn.yz = B.tmp.get<double2>(T.nn);
   hipLaunchKernelGGL(k_walk_nodes, grid_for(T.nn), dim3(256), 0, st, T.nn, nleaf, T.nd, wn);
@@ -2053,11 +2052,11 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   R->jlist = R->mem.get<int>(R->nj);
   R->clist = R->mem.get<int>(R->nc);
   if (opened) {
-    hipLaunchKernelGGL(k_bh_list<false>, dim3(ng), dim3(kListThreads), 0, st, ng, pool, wn.range,
+    hipLaunchKernelGGL(k_bh_list<false>, dim3(ng), dim3(kListThreads), 0, st, ng, pool, wn.item,
                        R->joff, R->coff, R->jlist, R->clist);
     if (big) {
       pool.sum = B.tmp.get<int4>(entries);
-      hipLaunchKernelGGL(k_bh_list<true>, dim3(ng), dim3(kListThreads), 0, st, ng, pool, wn.range,
+      hipLaunchKernelGGL(k_bh_list<true>, dim3(ng), dim3(kListThreads), 0, st, ng, pool, wn.item,
                          R->joff, R->coff, R->jlist, R->clist);
     }
     hipLaunchKernelGGL(k_bh_whole, grid_for(ng), dim3(256), 0, st, ng, R->jcnt, R->ccnt, wn,
