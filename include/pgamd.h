@@ -184,7 +184,10 @@ int pg5t_batch_launch_shape(int mode, int *out2);
  * assignment on a mesh^3 grid, FFT, Green's function -4 pi S(k a)^2 /
  * (k^2 W(k)^2), spectral gradient and TSC interpolation.  pos[n][3] in the
  * unit box [0, 1), mass[n], acc[n][3]: device FP64; acc is written.  Table
- * force + this = the S2-softened periodic Newtonian force. */
+ * force + this = the S2-softened periodic Newtonian force.  Calls share one
+ * workspace: the library runs them one after the other on the device,
+ * whichever streams they are queued on (replays of a captured call are the
+ * caller's to order). */
 int pg5t_pm_force(int n, const double *pos, const double *mass, int mesh, double eps_pm,
                   double *acc, void *stream);
 

@@ -1414,6 +1414,11 @@ struct PmCache {
   DevBuf bricks;  // per brick: count, start; then the chunks and their number
   DevBuf place, order, part;  // per particle: place in its brick, sorted index and data
   DevBuf fix;  // pm_mass_part's block sums, then the fixed-point scale
+  // Every call works in these buffers and plans, so a call runs after the
+  // previous one, whichever streams the two were queued on: the previous call's
+  // stream and an event at its end (pm_begin_on, pm_done_on).
+  hipStream_t last = nullptr;
+  hipEvent_t done = nullptr;
 };
 // The three inverse transforms run as one batch up to this mesh (36 -> 24 us
 // each at 128^3); beyond it one after the other, which needs a third of the
@@ -1448,9 +1453,40 @@ void pm_twiddles(PmCache& c) {
       hipMemcpy(c.twiddle.ptr, tw.data(), sizeof(double2) * tw.size(), hipMemcpyHostToDevice));
 }
 
-void pm_setup(PmCache& c, int M) {
+// Whether st is being captured into a graph: a captured call neither waits for
+// an event from outside the capture nor records one that calls outside it would
+// wait for.  Its replays are the caller's to order against other calls.
+bool pm_captured(hipStream_t st) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  PGAMD_HIP_CHECK(hipStreamIsCapturing(st, &s));
+  return s != hipStreamCaptureStatusNone;
+}
+
+// The end of the previous call (there was one).  A call on the board's own stream
+// is marked only here; one on a caller's stream at its end (pm_done_on), since
+// the caller may destroy it.
+hipEvent_t pm_end(PmCache& c, hipStream_t own) {
+  if (c.last == own) PGAMD_HIP_CHECK(hipEventRecord(c.done, own));
+  return c.done;
+}
+
+void pm_begin_on(PmCache& c, hipStream_t st, hipStream_t own) {
+  if (c.last && c.last != st)
+    PGAMD_HIP_CHECK(hipStreamWaitEvent(st, pm_end(c, own), 0));
+}
+
+void pm_done_on(PmCache& c, hipStream_t st, hipStream_t own) {
+  if (!c.done)
+    PGAMD_HIP_CHECK(hipEventCreateWithFlags(&c.done, hipEventDisableTiming |
+                                                         hipEventDisableSystemFence));
+  if (st != own) PGAMD_HIP_CHECK(hipEventRecord(c.done, st));
+  c.last = st;
+}
+
+void pm_setup(PmCache& c, int M, hipStream_t own) {
   if (c.M == M) return;
   if (c.M) {
+    if (c.last) PGAMD_HIP_CHECK(hipEventSynchronize(pm_end(c, own)));  // it uses the old plans
     PGAMD_FFT_CHECK(hipfftDestroy(c.fwd));
     PGAMD_FFT_CHECK(hipfftDestroy(c.inv));
   }
@@ -1483,7 +1519,9 @@ void pm_setup(PmCache& c, int M) {
 // 8..1024), with the S2 split at eps_pm (the table's eps_PM, which is also
 // its cut-off radius).  acc[n][3] (device, FP64) is written.  Add the
 // short-range accelerations of the table (pg5t_batch_force or the g5 calls)
-// for the whole TreePM force.  Asynchronous on `stream` (null = the library's).
+// for the whole TreePM force.  Asynchronous on `stream` (null = the library's);
+// calls share one workspace and run on the device one after the other, whichever
+// streams they are queued on.
 PGAMD_API int pg5t_pm_force(int n, const double* pos, const double* mass, int mesh, double eps_pm,
                             double* acc, void* stream) {
   Board* b = board(0, "pg5t_pm_force");
@@ -1496,8 +1534,10 @@ PGAMD_API int pg5t_pm_force(int n, const double* pos, const double* mass, int me
   }
   std::lock_guard<std::mutex> lk(g_pm_mutex);
   PmCache& c = g_pm;
-  pm_setup(c, mesh);
+  pm_setup(c, mesh, b->stream);
   hipStream_t st = stream ? (hipStream_t)stream : b->stream;
+  const bool captured = pm_captured(st);
+  if (!captured) pm_begin_on(c, st, b->stream);
   PGAMD_FFT_CHECK(hipfftSetStream(c.fwd, st));
   PGAMD_FFT_CHECK(hipfftSetStream(c.inv, st));
   const size_t nr = (size_t)mesh * mesh * mesh, nk = (size_t)mesh * mesh * (mesh / 2 + 1);
@@ -1586,5 +1626,6 @@ PGAMD_API int pg5t_pm_force(int n, const double* pos, const double* mass, int me
     hipLaunchKernelGGL(pm::pm_interp_direct, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, pos,
                        mesh, f, acc);
   PGAMD_HIP_CHECK(hipGetLastError());
+  if (!captured) pm_done_on(c, st, b->stream);
   return 0;
 }
