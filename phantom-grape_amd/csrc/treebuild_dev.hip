@@ -421,28 +421,20 @@ __device__ inline int shared_digits(u64 x, u64 y) {
   return d == 0 ? kLevels : (__clzll((long long)d) - 1) / 3;
 }
 
-// out[i] = max of in[max(0, i - w + 1) .. i], w <= kMaxWindow + 1.  FIRST: in[j]
-// = 1 + the digits shared by keys j and j + split (0 if there is no such
-// key).  By doubling in LDS.
+// out[i] = max of v[max(0, i - w + 1) .. i], w <= kMaxWindow + 1, v[j] = 1 + the
+// digits shared by keys j and j + split (0 if there is no such key).  By doubling
+// in LDS.
 constexpr int kWindowOut = 2048;
 constexpr int kMaxWindow = 1024;
-template <bool FIRST>
 __global__ __launch_bounds__(256) void k_window_max(int n, int split, int w,
                                                     const u64* __restrict__ key,
-                                                    const unsigned char* __restrict__ in,
                                                     unsigned char* __restrict__ out) {
   __shared__ unsigned char buf[2][kWindowOut + kMaxWindow];
   const int h = w - 1, m = kWindowOut + h;
   const int j0 = blockIdx.x * kWindowOut - h;
   for (int p = threadIdx.x; p < m; p += 256) {
     const int j = j0 + p;
-    int v = 0;
-    if (FIRST) {
-      if (j >= 0 && j < n - split) v = 1 + shared_digits(key[j], key[j + split]);
-    } else if (j >= 0 && j < n) {
-      v = in[j];
-    }
-    buf[0][p] = (unsigned char)v;
+    buf[0][p] = (unsigned char)(j >= 0 && j < n - split ? 1 + shared_digits(key[j], key[j + split]) : 0);
   }
   __syncthreads();
   int cur = 0, len = 1;  // buf[cur][p] = max over [p - len + 1, p]
@@ -456,6 +448,17 @@ __global__ __launch_bounds__(256) void k_window_max(int n, int split, int w,
     const int i = blockIdx.x * kWindowOut + q, p = q + h;
     if (i < n) out[i] = max(buf[cur][p], buf[cur][p - (w - len)]);
   }
+}
+
+// A window of in (maxima over `len` places) made longer by h <= len places.  Large
+// windows double from kMaxWindow + 1 on, so their launches grow with log2(split):
+// TreePM lists of 2^18 particles with ncrit = 2^17 took 2753 us with one launch
+// per 1024 places of the window, and take 860.
+__global__ __launch_bounds__(256) void k_window_grow(int n, int h,
+                                                     const unsigned char* __restrict__ in,
+                                                     unsigned char* __restrict__ out) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = max(in[i], i >= h ? in[i - h] : (unsigned char)0);
 }
 
 constexpr int kTreeLevels = kLevels + 1;
@@ -1733,6 +1736,7 @@ void build_octree(Build& B, Lists& R, int n, const double* x, const double* m,
                   const double lo[3], double L, int split, Octree& T, u64** skey_out,
                   double** mm_out) {
   hipStream_t st = B.st;
+  split = std::min(split, n);  // no cell holds more than n: the root is not split
   u64* key = B.tmp.get<u64>(n);
   const double s = (double)(1 << kLevels) / L;
   double* mm = m ? B.tmp.get<double>(n) : nullptr;
@@ -1750,17 +1754,14 @@ void build_octree(Build& B, Lists& R, int n, const double* x, const double* m,
     int* perm = nullptr;
     B.sort_keys(key, n, 3 * kLevels, bits, &skey, &perm, long_run);
     hipLaunchKernelGGL(k_gather, grid_for(n), dim3(256), 0, st, n, perm, x, m, R.pos, mm, R.src);
-    // leaf level of every particle: the sliding maximum, in steps of at most
-    // kMaxWindow (maxima over windows of u and v give one over u + v - 1)
-    const dim3 wgrid = grid_for(n, kWindowOut);
-    int left = split;  // of a window of split + 1
-    int w = std::min(left, kMaxWindow) + 1;
-    hipLaunchKernelGGL(k_window_max<true>, wgrid, dim3(256), 0, st, n, split, w, skey, nullptr,
+    // leaf level of every particle: the sliding maximum over split + 1 places (all
+    // are 0 where split = n)
+    int w = std::min(split, kMaxWindow) + 1;
+    hipLaunchKernelGGL(k_window_max, grid_for(n, kWindowOut), dim3(256), 0, st, n, split, w, skey,
                        leaf);
-    for (left -= w - 1; left > 0; left -= w - 1) {
-      w = std::min(left, kMaxWindow) + 1;
-      hipLaunchKernelGGL(k_window_max<false>, wgrid, dim3(256), 0, st, n, split, w, nullptr, leaf,
-                         leaf2);
+    for (int h; split < n && w < split + 1; w += h) {
+      h = std::min(w, split + 1 - w);
+      hipLaunchKernelGGL(k_window_grow, grid_for(n), dim3(256), 0, st, n, h, leaf, leaf2);
       std::swap(leaf, leaf2);
     }
     hipLaunchKernelGGL(k_tree_count, dim3(nb), dim3(256), 0, st, n, skey, leaf, count);
