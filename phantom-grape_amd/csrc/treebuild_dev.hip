@@ -1215,31 +1215,38 @@ __device__ inline int xcd_block(int b, int nb) {
 // {first child, masks, entry of the first opened child, 0}, masks: bits 0-7
 // children, 8-15 those that are single particles, 16-23 accepted cells (the
 // rest are opened); or a leaf.
-constexpr int kOpenChunk = 256;       // entries per chunk
-constexpr int kOpenGroupChunks = 64;  // per group at most: 14 bits of entry index
-constexpr int kOpenRing = 512;        // queued entries in LDS per wavefront
+constexpr int kOpenChunk = 256;        // entries per chunk
+constexpr int kOpenGroupChunks = 256;  // per group at most: 16 bits of entry index
+constexpr int kOpenRing = 512;         // queued entries in LDS per wavefront
 constexpr int kOpenLevels = kLevels + 3;
+constexpr int kRanOut = -1;  // for the number of levels: the pool or the table was too small
 
 struct OpenPool {
   int4* rec;    // [chunks][kOpenChunk]
   int4* sum;    // the same: k_bh_list's working entries of groups too large for LDS
   int* wait;    // the same: the entry at a ring position beyond the ring
-  // [0] != 0: the pool or a group's table was too small, [1] != 0: some group
-  // is too large for k_bh_list's LDS; then, a cache line each, the chunks
-  // handed out of every part of the pool
+  // [0] != 0: some group ran out of pool or table (and is left to the depth-first
+  // walk), [1] != 0: some group is too large for k_bh_list's LDS, then, a
+  // cache line each, the chunks handed out of every part of the pool
   int* used;
-  int* chunk;   // [group][kOpenGroupChunks]
+  int* chunk;   // [group][width]
   int* level;   // [group][kOpenLevels]: first entry of each level, then the number of
-                // entries; the last int is the number of levels (0: no entries)
+                // entries; the last int is the number of levels (0: no entries, or kRanOut)
   int chunks;   // of each part
+  int width;    // chunks of a group at most
 };
 // Parts of the pool with a counter of their own: a group begins with the part
-// of its number and goes on to the next where that is used up.  The 57000
+// of its number and goes on to the next ones where that is used up.  The 57000
 // chunks of a 2^21-particle build, taken from one counter, kept the walk
 // waiting for that address: 627 us, with 64 counters 219.
 constexpr int kPoolParts = 64;
+constexpr int kPoolTries = 8;  // parts that a group asks
 constexpr int kPoolLine = 32;  // ints
 constexpr int kPoolUsed = (1 + kPoolParts) * kPoolLine;
+// Chunks at most: 4 GiB of records, 1 GiB of queue and, where groups are too
+// large for LDS, 4 GiB of working entries, which the cache keeps (to give such
+// blocks back to the device and take them again costs 50 ms a GiB).
+constexpr double kPoolMost = 1 << 20;
 
 // Opened children, own particles and own cells of an entry.
 __device__ inline int open_count(unsigned b) {
@@ -1282,31 +1289,32 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_open(
     return;
   }
   int nch = 0;
-  // one more chunk for this group; false: none left
+  // one more chunk for this group; false: none left, or no room in its table
   auto grow = [&]() {
     int c = -1;
-    for (int t = 0; t < kPoolParts && nch < kOpenGroupChunks && c < 0; ++t) {
+#pragma unroll 1  // unrolled, its registers cost the launch 257 us for 226
+    for (int t = 0; t < kPoolTries && nch < pool.width && c < 0; ++t) {
       const int part = (g + t) % kPoolParts;
       int k = 0;
       if (lane == 0) k = atomicAdd(&pool.used[(1 + part) * kPoolLine], 1);
       k = __builtin_amdgcn_readfirstlane(k);
       if (k < pool.chunks) c = part * pool.chunks + k;
     }
-    if (c < 0) {
-      if (lane == 0) {
-        pool.used[0] = 1;
-        pcnt[g] = 0;
-        ccnt[g] = 0;
-        level[kOpenLevels - 1] = 0;
-      }
-      return false;
-    }
+    if (c < 0) return false;
     if (lane == 0) {
       chunk[nch] = c;
-      pool.chunk[(size_t)g * kOpenGroupChunks + nch] = c;
+      pool.chunk[(size_t)g * pool.width + nch] = c;
     }
     ++nch;
     return true;
+  };
+  auto ran_out = [&]() {
+    if (lane == 0) {
+      pool.used[0] = 1;
+      pcnt[g] = 0;
+      ccnt[g] = 0;
+      level[kOpenLevels - 1] = kRanOut;
+    }
   };
   auto at = [&](int k) { return (size_t)chunk[k / kOpenChunk] * kOpenChunk + k % kOpenChunk; };
   // order LDS, or LDS and pool, writes before the reads of the wavefront's
@@ -1321,7 +1329,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_open(
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   };
-  if (!grow()) return;
+  if (!grow()) return ran_out();
   lds_sync();
   int np = 0, nc = 0;         // listed particles (leaves: this lane's) and cells
   int tail = 1;               // entries
@@ -1365,7 +1373,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_open(
     const u64 below = (1ULL << lane) - 1ULL;
     const int opened = __popcll(ms);
     while ((tail + opened - 1) / kOpenChunk >= nch) {
-      if (!grow()) return;
+      if (!grow()) return ran_out();
       lds_sync();
     }
     head += npop;
@@ -1441,10 +1449,11 @@ __global__ __launch_bounds__(kListThreads) void k_bh_list(
   const int g = xcd_block(blockIdx.x, gridDim.x);
   const int tid = threadIdx.x;
   if (tid < kOpenLevels) s_level[tid] = pool.level[(size_t)g * kOpenLevels + tid];
-  if (tid < kOpenGroupChunks) s_chunk[tid] = pool.chunk[(size_t)g * kOpenGroupChunks + tid];
+  static_assert(kOpenGroupChunks <= kListThreads, "one chunk per thread");
+  if (tid < pool.width) s_chunk[tid] = pool.chunk[(size_t)g * pool.width + tid];
   __syncthreads();
   const int nlev = s_level[kOpenLevels - 1];
-  if (nlev == 0) return;  // uniform
+  if (nlev <= 0) return;  // uniform
   const int n = s_level[nlev];
   if (BIG != (n > kListEntries)) return;  // uniform
   auto at = [&](int k) { return (size_t)s_chunk[k / kOpenChunk] * kOpenChunk + k % kOpenChunk; };
@@ -1537,8 +1546,8 @@ __global__ void k_bh_whole(int ng, const int* __restrict__ pcnt, const int* __re
     clist[coff[g]] = nd.cell[0];
 }
 
-// For builds whose groups open more nodes than k_bh_open's pool or chunk
-// tables hold (small theta).
+// For the groups that open more nodes than k_bh_open's pool or their table has
+// left (level: of the pool), or for all of a build without a pool (level null).
 //
 // One wavefront per group: the depth-first walk of the host builder
 // (source.cpp:832-867 order: the children of an opened node are examined in
@@ -1556,7 +1565,7 @@ __global__ void k_bh_whole(int ng, const int* __restrict__ pcnt, const int* __re
 template <bool FILL>
 __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_walk(
     int ng, const int* __restrict__ gnode, Nodes nd, WalkNodes wn, double L,
-    double th2, int* __restrict__ pcnt, int* __restrict__ ccnt,
+    double th2, const int* __restrict__ level, int* __restrict__ pcnt, int* __restrict__ ccnt,
     const int* __restrict__ poff, const int* __restrict__ coff, int* __restrict__ plist,
     int* __restrict__ clist) {
 #pragma clang fp contract(off)
@@ -1566,6 +1575,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_bh_walk(
   const int lane = threadIdx.x & 63;
   const int g = xcd_block(blockIdx.x, gridDim.x) * kWalkWaves + (threadIdx.x >> 6);
   if (g >= ng) return;  // uniform per wavefront
+  if (level && level[(size_t)g * kOpenLevels + kOpenLevels - 1] != kRanOut) return;  // the same
   int3* stk = s_stack[threadIdx.x >> 6];
   const int gk = gnode[g];
   const double gc[3] = {nd.c[3 * gk], nd.c[3 * gk + 1], nd.c[3 * gk + 2]};
@@ -1956,6 +1966,34 @@ Lists* treepm_build(int n, const double* x, double rcut, int ncrit, hipStream_t 
   return R;
 }
 
+// The pool of a build of ng groups over nn nodes; rec is null where the
+// depth-first walk is to do it alone.
+//
+// Opened nodes of a group on average (halo of 2^21 particles, groups of up to 512,
+// leaves of 8): 793 at theta = 0.5, 2206 at 0.3, 5858 at 0.2, 8666 at 0.17, about
+// theta^-2.25; in groups of up to 16 444 at 0.5.  The pool has room for 1280 (768)
+// of them and as much more for smaller theta, and a group for 16384 or 65536.
+// Where most groups would open more than that the walk takes all of them.
+OpenPool open_pool(Build& B, int ng, int nn, double theta, int ncrit) {
+  OpenPool p{};
+  const double all = std::ceil(nn / (double)kOpenChunk);  // chunks of all nodes
+  const double each =
+      std::min(all, (ncrit < 128 ? 3.0 : 5.0) * std::max(1.0, std::pow(0.5 / theta, 2.25)));
+  if (each > kOpenGroupChunks) return p;
+  p.width = each > 40 ? kOpenGroupChunks : 64;
+  // a power of two, as the cache's blocks; a group's table can be filled from the
+  // parts it asks
+  size_t chunks = (size_t)kPoolParts / kPoolTries * p.width;
+  while (chunks < std::min(64 + ng * each, kPoolMost)) chunks *= 2;
+  p.chunks = (int)(chunks / kPoolParts);
+  p.rec = B.tmp.get<int4>(chunks * kOpenChunk);
+  p.wait = B.tmp.get<int>(chunks * kOpenChunk);
+  p.chunk = B.tmp.get<int>((size_t)ng * p.width);
+  p.level = B.tmp.get<int>((size_t)ng * kOpenLevels);
+  p.used = B.tmp.get<int>(kPoolUsed);
+  return p;
+}
+
 Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit, int nleaf,
                 hipStream_t st) {
   Lists* R = new Lists();
@@ -2019,21 +2057,6 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   hipLaunchKernelGGL(k_walk_nodes, grid_for(T.nn), dim3(256), 0, st, T.nn, nleaf, T.nd, wn);
   PGAMD_HIP_CHECK(hipGetLastError());
   const dim3 wgrid((ng + kWalkWaves - 1) / kWalkWaves), wblock(64 * kWalkWaves);
-  // About 900 opened nodes a group at theta = 0.5 and 2^21 particles; 1280
-  // of them, more for smaller theta (nodes within a distance 1 / theta).
-  const double more = std::min(8.0, std::max(1.0, std::pow(0.5 / theta, 3)));
-  OpenPool pool{};
-  pool.chunks = (int)std::ceil(std::min(1e6, 64.0 + 5.0 * ng * more) / kPoolParts);
-  const size_t entries = (size_t)pool.chunks * kPoolParts * kOpenChunk;
-  pool.rec = B.tmp.get<int4>(entries);
-  pool.wait = B.tmp.get<int>(entries);
-  pool.chunk = B.tmp.get<int>((size_t)ng * (kOpenGroupChunks + kOpenLevels));
-  pool.level = pool.chunk + (size_t)ng * kOpenGroupChunks;
-  pool.used = B.tmp.get<int>(kPoolUsed);
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(1024), 0, st, kPoolUsed, 0, pool.used);
-  hipLaunchKernelGGL(k_bh_open, wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2, pool,
-                     R->jcnt, R->ccnt);
-  PGAMD_HIP_CHECK(hipGetLastError());
   auto offsets = [&] {
     B.scan(R->jcnt, R->joff, ng, kSlotTotal);
     B.scan(R->ccnt, R->coff, ng, kSlotTotal2);
@@ -2042,15 +2065,25 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
     R->nc = host[kSlotTotal2];
     return host;
   };
-  hipLaunchKernelGGL(k_copy_ints, dim3(1), dim3(64), 0, st, 2, pool.used,
-                     host_dev(host_ints()) + kSlotPool);
-  PGAMD_HIP_CHECK(hipGetLastError());
-  const volatile int* host = offsets();
-  const bool opened = host[kSlotPool] == 0;
-  const bool big = host[kSlotPool + 1] != 0;
-  if (!opened) {
+  OpenPool pool = open_pool(B, ng, T.nn, theta, ncrit);
+  const bool opened = pool.rec != nullptr;
+  bool walks = !opened, big = false;
+  if (opened) {
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(1024), 0, st, kPoolUsed, 0, pool.used);
+    hipLaunchKernelGGL(k_bh_open, wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2, pool,
+                       R->jcnt, R->ccnt);
+    hipLaunchKernelGGL(k_copy_ints, dim3(1), dim3(64), 0, st, 2, pool.used,
+                       host_dev(host_ints()) + kSlotPool);
+    PGAMD_HIP_CHECK(hipGetLastError());
+    const volatile int* host = offsets();
+    walks = host[kSlotPool] != 0;
+    big = host[kSlotPool + 1] != 0;
+    if (big) pool.sum = B.tmp.get<int4>((size_t)pool.chunks * kPoolParts * kOpenChunk);
+  }
+  if (walks) {
     hipLaunchKernelGGL((k_bh_walk<false>), wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2,
-                       R->jcnt, R->ccnt, nullptr, nullptr, nullptr, nullptr);
+                       opened ? pool.level : nullptr, R->jcnt, R->ccnt, nullptr, nullptr, nullptr,
+                       nullptr);
     PGAMD_HIP_CHECK(hipGetLastError());
     offsets();
   }
@@ -2059,17 +2092,16 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   if (opened) {
     hipLaunchKernelGGL(k_bh_list<false>, dim3(ng), dim3(kListThreads), 0, st, ng, pool, wn.item,
                        R->joff, R->coff, R->jlist, R->clist);
-    if (big) {
-      pool.sum = B.tmp.get<int4>(entries);
+    if (big)
       hipLaunchKernelGGL(k_bh_list<true>, dim3(ng), dim3(kListThreads), 0, st, ng, pool, wn.item,
                          R->joff, R->coff, R->jlist, R->clist);
-    }
     hipLaunchKernelGGL(k_bh_whole, grid_for(ng), dim3(256), 0, st, ng, R->jcnt, R->ccnt, wn,
                        R->coff, gnode, T.nd, L, th2, R->clist);
-  } else {
-    hipLaunchKernelGGL((k_bh_walk<true>), wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2,
-                       nullptr, nullptr, R->joff, R->coff, R->jlist, R->clist);
   }
+  if (walks)
+    hipLaunchKernelGGL((k_bh_walk<true>), wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2,
+                       opened ? pool.level : nullptr, nullptr, nullptr, R->joff, R->coff, R->jlist,
+                       R->clist);
   PGAMD_HIP_CHECK(hipGetLastError());
   finish(B, *R, true);
   return R;
