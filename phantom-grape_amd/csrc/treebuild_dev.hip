@@ -42,11 +42,15 @@ constexpr int kLevels = 21;  // bits per axis of the Morton key
 // hipMalloc / hipFree calls (hipFree also waits for the whole device).  A
 // build releases its temporaries after its stream has drained, lists release
 // theirs in pgt_dev_free after a device synchronisation; both run under the
-// library's mutex.  The cache holds its peak size until the process ends.
+// library's mutex.  The cache holds its peak size until the process ends, or
+// until the device has no memory left for another block.
 struct Cache {
   std::map<size_t, std::vector<void*>> free;
   std::unordered_map<void*, size_t> size;
-  void* get(size_t bytes) {
+  // null if the device has no memory left, also after the unused blocks are
+  // given back
+  void* try_get(size_t bytes) {
+    if (bytes > (size_t)1 << 48) return nullptr;  // a length beyond the range of int
     size_t b = 256;
     while (b < bytes) b <<= 1;
     std::vector<void*>& v = free[b];
@@ -55,10 +59,30 @@ struct Cache {
       v.pop_back();
       return p;
     }
-    void* p = nullptr;
-    PGAMD_HIP_CHECK(hipMalloc(&p, b));
-    size[p] = b;
+    void* p = try_malloc(b);
+    if (!p) {
+      for (auto& f : free) {
+        for (void* q : f.second) {
+          PGAMD_HIP_CHECK(hipFree(q));
+          size.erase(q);
+        }
+        f.second.clear();
+      }
+      p = try_malloc(b);
+    }
+    if (p) size[p] = b;
     return p;
+  }
+  void* get(size_t bytes) {
+    void* p = try_get(bytes);
+    if (!p) PGAMD_HIP_CHECK(hipErrorOutOfMemory);
+    return p;
+  }
+  static void* try_malloc(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
   }
   void put(void* p) { free[size.at(p)].push_back(p); }
 };
@@ -70,6 +94,12 @@ struct Mem {
   T* get(size_t n) {
     void* p = g_cache.get(std::max<size_t>(n, 1) * sizeof(T));
     ptrs.push_back(p);
+    return static_cast<T*>(p);
+  }
+  template <class T>
+  T* try_get(size_t n) {
+    void* p = g_cache.try_get(std::max<size_t>(n, 1) * sizeof(T));
+    if (p) ptrs.push_back(p);
     return static_cast<T*>(p);
   }
   void free_all() {
@@ -230,6 +260,7 @@ inline dim3 grid_for(long long n, int threads = 256) {
 struct Build {
   hipStream_t st;
   Mem tmp;
+  Mem pool;  // of OpenPool: given up first where the device has no memory left
   void* cub = nullptr;
   size_t cub_bytes = 0;
   explicit Build(hipStream_t s) : st(s) {}
@@ -237,6 +268,7 @@ struct Build {
     PGAMD_HIP_CHECK(hipStreamSynchronize(st));
     if (cub) g_cache.put(cub);
     tmp.free_all();
+    pool.free_all();
   }
   void* cub_tmp(size_t bytes) {
     if (bytes > cub_bytes) {
@@ -1986,11 +2018,15 @@ OpenPool open_pool(Build& B, int ng, int nn, double theta, int ncrit) {
   size_t chunks = (size_t)kPoolParts / kPoolTries * p.width;
   while (chunks < std::min(64 + ng * each, kPoolMost)) chunks *= 2;
   p.chunks = (int)(chunks / kPoolParts);
-  p.rec = B.tmp.get<int4>(chunks * kOpenChunk);
-  p.wait = B.tmp.get<int>(chunks * kOpenChunk);
-  p.chunk = B.tmp.get<int>((size_t)ng * p.width);
-  p.level = B.tmp.get<int>((size_t)ng * kOpenLevels);
-  p.used = B.tmp.get<int>(kPoolUsed);
+  p.rec = B.pool.try_get<int4>(chunks * kOpenChunk);
+  p.wait = B.pool.try_get<int>(chunks * kOpenChunk);
+  p.chunk = B.pool.try_get<int>((size_t)ng * p.width);
+  p.level = B.pool.try_get<int>((size_t)ng * kOpenLevels);
+  p.used = B.pool.try_get<int>(kPoolUsed);
+  if (!p.rec || !p.wait || !p.chunk || !p.level || !p.used) {
+    B.pool.free_all();
+    p.rec = nullptr;
+  }
   return p;
 }
 
@@ -2066,8 +2102,13 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
     return host;
   };
   OpenPool pool = open_pool(B, ng, T.nn, theta, ncrit);
-  const bool opened = pool.rec != nullptr;
-  bool walks = !opened, big = false;
+  bool opened = pool.rec != nullptr, walks = !opened, big = false;
+  // without the pool (its kernels have ended) the walk lists all groups
+  auto give_up = [&] {
+    B.pool.free_all();
+    opened = false;
+    walks = true;
+  };
   if (opened) {
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(1024), 0, st, kPoolUsed, 0, pool.used);
     hipLaunchKernelGGL(k_bh_open, wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2, pool,
@@ -2078,7 +2119,8 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
     const volatile int* host = offsets();
     walks = host[kSlotPool] != 0;
     big = host[kSlotPool + 1] != 0;
-    if (big) pool.sum = B.tmp.get<int4>((size_t)pool.chunks * kPoolParts * kOpenChunk);
+    if (big) pool.sum = B.pool.try_get<int4>((size_t)pool.chunks * kPoolParts * kOpenChunk);
+    if (big && !pool.sum) give_up();
   }
   if (walks) {
     hipLaunchKernelGGL((k_bh_walk<false>), wgrid, wblock, 0, st, ng, gnode, T.nd, wn, L, th2,
@@ -2087,8 +2129,11 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
     PGAMD_HIP_CHECK(hipGetLastError());
     offsets();
   }
-  R->jlist = R->mem.get<int>(R->nj);
-  R->clist = R->mem.get<int>(R->nc);
+  R->jlist = R->mem.try_get<int>(R->nj);
+  R->clist = R->jlist ? R->mem.try_get<int>(R->nc) : nullptr;
+  if (!R->clist && opened) give_up();
+  if (!R->jlist) R->jlist = R->mem.get<int>(R->nj);
+  if (!R->clist) R->clist = R->mem.get<int>(R->nc);
   if (opened) {
     hipLaunchKernelGGL(k_bh_list<false>, dim3(ng), dim3(kListThreads), 0, st, ng, pool, wn.item,
                        R->joff, R->coff, R->jlist, R->clist);
