@@ -1421,13 +1421,19 @@ struct PmCache {
   hipEvent_t done = nullptr;
 };
 // The three inverse transforms run as one batch up to this mesh (36 -> 24 us
-// each at 128^3); beyond it one after the other, which needs a third of the
-// FFT's work memory.
+// each at 128^3; the whole call 209 -> 176 us at 96^3, 711 -> 665 at 192^3, 1169 ->
+// 1154 at 240^3); beyond it one after the other, which needs a third of the
+// FFT's work memory and costs 0.3 to 2 % (2.24 -> 2.20 ms at 288^3, 9.64 -> 9.61 at
+// 512^3).
 constexpr int kPmBatchMesh = 256;
-// Particles per brick from which the brick sort pays: below it the boxes of
-// 10^3 points are mostly empty and the particles go straight to the mesh.
-// Clumpy boxes on a 128^3 mesh, straight / sorted: 198 / 185 us at 4.0
-// particles per brick, 217 / 189 us at 7.3; 192^3 565 / 577 us at 4.7.
+// Particles per brick from which the brick sort is worth its launches: below, the
+// boxes of 10^3 points are mostly empty and the particles go straight to the
+// mesh.  Straight / sorted in us at 2, 3 and 4 particles a brick, uniform (clumpy):
+// 128^3 162 / 165 (163 / 158), 164 / 165 (169 / 160), 170 / 168 (174 / 164); 192^3 526 / 567
+// (528 / 550), 545 / 574 (551 / 561), 562 / 582 (572 / 571); 256^3 907 / 1008 (907 / 960),
+// 990 / 1031 (977 / 994), 1067 / 1041 (1053 / 1018); 512^3 10308 / 10777
+// (10223 / 10522), 10943 / 10964 (10842 / 10728), 11574 / 11069 (11435 / 10891); 64^3 to
+// 100^3 sorted at any density.
 constexpr int kPmPerBrick = 3;
 PmCache g_pm;
 std::mutex g_pm_mutex;
@@ -1554,11 +1560,14 @@ PGAMD_API int pg5t_pm_force(int n, const double* pos, const double* mass, int me
   double4* part = nullptr;
   const int max_chunks = sorted ? (int)(nbricks + n / pm::kChunk) : 0;
   int* count = nullptr;
+  const int ntiles = nbricks <= pm::kLdsBricks ? 0 : ceil_div(nbricks, 1024);  // of pm_scan
+  int2* tiles = nullptr;
   if (sorted) {
-    c.bricks.reserve(sizeof(pm::Chunk) * (size_t)max_chunks +
+    c.bricks.reserve(sizeof(pm::Chunk) * (size_t)max_chunks + sizeof(int2) * (size_t)ntiles +
                      sizeof(int) * (2 * (size_t)nbricks + 1));
     chunks = c.bricks.as<pm::Chunk>();
-    count = reinterpret_cast<int*>(chunks + max_chunks);
+    tiles = reinterpret_cast<int2*>(chunks + max_chunks);
+    count = reinterpret_cast<int*>(tiles + ntiles);
   }
   c.fix.reserve(sizeof(double) * (pm::kMassBlocks + 1));
   double* msum = c.fix.as<double>();
@@ -1585,15 +1594,22 @@ PGAMD_API int pg5t_pm_force(int n, const double* pos, const double* mass, int me
       else
         hipLaunchKernelGGL(pm::pm_count<false>, cgrid, cblock, 0, st, n, pos, mesh, nb, count,
                            place);
-      hipLaunchKernelGGL(pm::pm_scan, dim3(1), dim3(1024), 0, st, (int)nbricks, count, start,
-                         chunks, nchunks, msum, mesh, scale);
+      if (ntiles) {
+        hipLaunchKernelGGL(pm::pm_tile_sums, dim3(ntiles), dim3(1024), 0, st, (int)nbricks, count,
+                           tiles);
+        hipLaunchKernelGGL(pm::pm_scan<true>, dim3(ntiles), dim3(1024), 0, st, (int)nbricks, count,
+                           tiles, start, chunks, nchunks, msum, mesh, scale);
+      } else {
+        hipLaunchKernelGGL(pm::pm_scan<false>, dim3(1), dim3(1024), 0, st, (int)nbricks, count,
+                           nullptr, start, chunks, nchunks, msum, mesh, scale);
+      }
       hipLaunchKernelGGL(pm::pm_scatter, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, pos, mass,
                          start, place, order, part);
       hipLaunchKernelGGL(pm::pm_assign, dim3(max_chunks), dim3(pm::kBrickThreads), 0, st, nchunks,
                          chunks, part, mesh, nb, scale, fixed);
     } else {
-      hipLaunchKernelGGL(pm::pm_scan, dim3(1), dim3(1024), 0, st, 0, nullptr, nullptr, nullptr,
-                         nullptr, msum, mesh, scale);
+      hipLaunchKernelGGL(pm::pm_scan<false>, dim3(1), dim3(1024), 0, st, 0, nullptr, nullptr, nullptr,
+                         nullptr, nullptr, msum, mesh, scale);
       hipLaunchKernelGGL(pm::pm_assign_direct, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, pos,
                          mass, mesh, scale, fixed);
     }
