@@ -150,8 +150,8 @@ __global__ __launch_bounds__(kThreads) void radix_scatter(
 // Pairs sorted by the bits from `shift` up, into the order of all bits: every
 // pair of a run of equal upper bits counts the ones before it.  A run of more
 // than kMaxRun pairs sets *long_run and is left unsorted; its pairs see that from
-// the pair kMaxRun places away, without counting (where they counted up to 2048
-// first, 2^20 pairs in runs of 2048 took 3.26 ms to build lists of, now 2.09).
+// the pair kMaxRun places away, without counting (counting up to 2048 others first
+// made lists of 2^20 particles in runs of 2048 1.2 ms slower).
 // Runs of 512 cost about as much to count as to sort again with all bits.
 constexpr int kMaxRun = 512;
 template <class K>

@@ -2056,7 +2056,7 @@ Lists* bh_build(int n, const double* x, const double* m, double theta, int ncrit
   double* mm = nullptr;
   build_octree(B, *R, n, x, m, lo, L, std::max(1, std::min(ncrit, nleaf)), T, &skey, &mm);
   // moments: all leaves at once, then the inner nodes, deepest level first
-  // (2^21 particles: 62 + 103 + 28 us; 16 launches over whole levels took 240)
+  // (2^21 particles: 54 + 103 + 29 us; 16 launches over whole levels took 240)
   hipLaunchKernelGGL(k_leaf_moments, grid_for(T.nn), dim3(256), 0, st, T.nn, T.nd, R->pos, mm);
   int top = 0;
   while (top <= kLevels && T.level.v[top + 1] - T.level.v[top] <= kTopNodes) ++top;
