@@ -17,6 +17,7 @@
 #include "treepm_batch.h"
 #include "pm_kernels.h"
 
+#include <hip/hip_ext.h>
 #include <hipfft/hipfft.h>
 
 #include <algorithm>
@@ -1470,7 +1471,8 @@ bool pm_captured(hipStream_t st) {
 
 // The end of the previous call (there was one).  A call on the board's own stream
 // is marked only here; one on a caller's stream at its end (pm_done_on), since
-// the caller may destroy it.
+// the caller may destroy it, by its last launch: an event recorded after it would
+// take the stream 1.3 us more.
 hipEvent_t pm_end(PmCache& c, hipStream_t own) {
   if (c.last == own) PGAMD_HIP_CHECK(hipEventRecord(c.done, own));
   return c.done;
@@ -1481,12 +1483,18 @@ void pm_begin_on(PmCache& c, hipStream_t st, hipStream_t own) {
     PGAMD_HIP_CHECK(hipStreamWaitEvent(st, pm_end(c, own), 0));
 }
 
-void pm_done_on(PmCache& c, hipStream_t st, hipStream_t own) {
+// Queues a call's last launch (unless captured), which marks its end.
+template <class K, class... A>
+void pm_done_on(PmCache& c, hipStream_t st, hipStream_t own, bool captured, K kernel, dim3 grid,
+                dim3 block, A... args) {
   if (!c.done)
     PGAMD_HIP_CHECK(hipEventCreateWithFlags(&c.done, hipEventDisableTiming |
                                                          hipEventDisableSystemFence));
-  if (st != own) PGAMD_HIP_CHECK(hipEventRecord(c.done, st));
-  c.last = st;
+  if (captured || st == own)
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, args...);
+  else
+    hipExtLaunchKernelGGL(kernel, grid, block, 0, st, nullptr, c.done, 0, args...);
+  if (!captured) c.last = st;
 }
 
 void pm_setup(PmCache& c, int M, hipStream_t own) {
@@ -1636,12 +1644,11 @@ PGAMD_API int pg5t_pm_force(int n, const double* pos, const double* mass, int me
     PGAMD_FFT_CHECK(hipfftExecZ2D(c.inv, reinterpret_cast<hipfftDoubleComplex*>(fk + d * nk),
                                   f + d * nr));
   if (sorted)
-    hipLaunchKernelGGL(pm::pm_interp, dim3(max_chunks), dim3(pm::kBrickThreads), 0, st, nchunks,
-                       chunks, order, part, mesh, nb, f, acc);
-  else if (n > 0)
-    hipLaunchKernelGGL(pm::pm_interp_direct, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, pos,
-                       mesh, f, acc);
+    pm_done_on(c, st, b->stream, captured, pm::pm_interp, dim3(max_chunks), dim3(pm::kBrickThreads),
+               nchunks, chunks, order, part, mesh, nb, f, acc);
+  else  // no particles: the launch only marks the end
+    pm_done_on(c, st, b->stream, captured, pm::pm_interp_direct, dim3(std::max(1, ceil_div(n, 256))),
+               dim3(256), n, pos, mesh, f, acc);
   PGAMD_HIP_CHECK(hipGetLastError());
-  if (!captured) pm_done_on(c, st, b->stream);
   return 0;
 }
