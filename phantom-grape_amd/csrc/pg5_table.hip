@@ -1612,7 +1612,7 @@ PGAMD_API int pg5t_pm_force(int n, const double* pos, const double* mass, int me
                            nullptr, start, chunks, nchunks, msum, mesh, scale);
       }
       hipLaunchKernelGGL(pm::pm_scatter, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, pos, mass,
-                         start, place, order, part);
+                         mesh, start, place, order, part);
       hipLaunchKernelGGL(pm::pm_assign, dim3(max_chunks), dim3(pm::kBrickThreads), 0, st, nchunks,
                          chunks, part, mesh, nb, scale, fixed);
     } else {

@@ -29,17 +29,19 @@
 
 namespace pm {
 
-// Nearest mesh point of a position x along one axis, before wrapping.  Every
-// kernel takes it from here, with one rounding: a particle's brick is the one
-// its stencil lies in, so whether x M is rounded on the way (at x = -0.5 / M that
-// decides between two points) must not differ from kernel to kernel.
-__device__ inline double mesh_point(double x, int M) { return floor(fma(x, (double)M, 0.5)); }
+// x M, rounded.  Every kernel takes a particle's mesh point from this value: its
+// brick is the one its stencil lies in, so whether the product is rounded before
+// 0.5 is added (at x = -0.5 / M that decides between two points) must not differ
+// from kernel to kernel, as it does where the compiler fuses the two.
+__device__ inline double mesh_units(double x, int M) {
+#pragma clang fp contract(off)
+  return x * (double)M;
+}
 
-// Nearest mesh point and TSC weights along one axis; the distance from the point is
-// taken from the unrounded x M.
-__device__ inline int tsc(double x, int M, double w[3]) {
-  const double g = mesh_point(x, M);
-  const double d = fma(x, (double)M, -g);
+// Nearest mesh point and TSC weights along one axis, u in mesh units.
+__device__ inline int tsc(double u, double w[3]) {
+  const double g = floor(u + 0.5);
+  const double d = u - g;
   w[0] = 0.5 * (0.5 - d) * (0.5 - d);
   w[1] = 0.75 - d * d;
   w[2] = 0.5 * (0.5 + d) * (0.5 + d);
@@ -51,8 +53,10 @@ __device__ inline int wrap(int i, int m) {
   return i < 0 ? i + m : i;
 }
 
-// Nearest mesh point, wrapped into [0, M).
-__device__ inline int nearest(double x, int M) { return wrap((int)mesh_point(x, M), M); }
+// Nearest mesh point of the position x, wrapped into [0, M).
+__device__ inline int nearest(double x, int M) {
+  return wrap((int)floor(mesh_units(x, M) + 0.5), M);
+}
 
 // Fixed-point scale of the mass assignment.  Every mesh point receives at
 // most sum |m| M^3 (TSC weights of a particle sum to 1), so with
@@ -267,9 +271,9 @@ __global__ __launch_bounds__(1024) void pm_scan(int bricks, const int* __restric
   if ((!TILES || blockIdx.x == gridDim.x - 1) && tid == 0 && nchunks) *nchunks = run.y;
 }
 
-// Sorted copies: index, and position with the mass.
+// Sorted copies: index, and position in mesh units with the mass.
 __global__ __launch_bounds__(256) void pm_scatter(int n, const double* __restrict__ pos,
-                                                  const double* __restrict__ mass,
+                                                  const double* __restrict__ mass, int M,
                                                   const int* __restrict__ start,
                                                   const int2* __restrict__ place,
                                                   int* __restrict__ order,
@@ -279,8 +283,8 @@ __global__ __launch_bounds__(256) void pm_scatter(int n, const double* __restric
   const int2 at = place[p];
   const int k = start[at.x] + at.y;
   order[k] = p;
-  part[k] = make_double4(pos[3 * (size_t)p], pos[3 * (size_t)p + 1], pos[3 * (size_t)p + 2],
-                         mass[p]);
+  part[k] = make_double4(mesh_units(pos[3 * (size_t)p], M), mesh_units(pos[3 * (size_t)p + 1], M),
+                         mesh_units(pos[3 * (size_t)p + 2], M), mass[p]);
 }
 
 // v[r % 3] for r in [0, 5).
@@ -316,8 +320,7 @@ __global__ __launch_bounds__(kBrickThreads) void pm_assign(
   for (int k = ck.k0 + tid; k < ck.k1; k += kBrickThreads) {
     const double4 q = part[k];
     double vx[3], vy[3], vz[3];
-    const int gx = wrap(tsc(q.x, M, vx), M), gy = wrap(tsc(q.y, M, vy), M),
-              gz = wrap(tsc(q.z, M, vz), M);
+    const int gx = wrap(tsc(q.x, vx), M), gy = wrap(tsc(q.y, vy), M), gz = wrap(tsc(q.z, vz), M);
     const int first = ((gx - 1 - ox) * kBox + gy - 1 - oy) * kBox + gz - 1 - oz;
     const double qm = q.w * m3;  // mass / h^3 in fixed-point units
     // the weights in this lane's order
@@ -360,9 +363,9 @@ __global__ __launch_bounds__(256) void pm_assign_direct(int n, const double* __r
   const int p = blockIdx.x * 256 + threadIdx.x;
   if (p >= n) return;
   double wx[3], wy[3], wz[3];
-  const int gx = tsc(pos[3 * (size_t)p], M, wx);
-  const int gy = tsc(pos[3 * (size_t)p + 1], M, wy);
-  const int gz = tsc(pos[3 * (size_t)p + 2], M, wz);
+  const int gx = tsc(mesh_units(pos[3 * (size_t)p], M), wx);
+  const int gy = tsc(mesh_units(pos[3 * (size_t)p + 1], M), wy);
+  const int gz = tsc(mesh_units(pos[3 * (size_t)p + 2], M), wz);
   const double qm = mass[p] * ((double)M * (double)M * (double)M * scale[0]);
   for (int a = 0; a < 3; ++a) {
     const size_t ix = (size_t)wrap(gx + a - 1, M) * M;
@@ -570,8 +573,7 @@ __global__ __launch_bounds__(kBrickThreads) void pm_interp(
   for (int k = ck.k0 + tid; k < ck.k1; k += kBrickThreads) {
     const double4 q = part[k];
     double wx[3], wy[3], wz[3];
-    const int gx = wrap(tsc(q.x, M, wx), M), gy = wrap(tsc(q.y, M, wy), M),
-              gz = wrap(tsc(q.z, M, wz), M);
+    const int gx = wrap(tsc(q.x, wx), M), gy = wrap(tsc(q.y, wy), M), gz = wrap(tsc(q.z, wz), M);
     const int first = ((gx - 1 - ox) * kBox + gy - 1 - oy) * kBox + gz - 1 - oz;
     double ax = 0.0, ay = 0.0, az = 0.0;
 #pragma unroll
@@ -603,9 +605,9 @@ __global__ __launch_bounds__(256) void pm_interp_direct(int n, const double* __r
   if (p >= n) return;
   const size_t nr = (size_t)M * M * M;
   double wx[3], wy[3], wz[3];
-  const int gx = tsc(pos[3 * (size_t)p], M, wx);
-  const int gy = tsc(pos[3 * (size_t)p + 1], M, wy);
-  const int gz = tsc(pos[3 * (size_t)p + 2], M, wz);
+  const int gx = tsc(mesh_units(pos[3 * (size_t)p], M), wx);
+  const int gy = tsc(mesh_units(pos[3 * (size_t)p + 1], M), wy);
+  const int gz = tsc(mesh_units(pos[3 * (size_t)p + 2], M), wz);
   double ax = 0.0, ay = 0.0, az = 0.0;
   for (int a = 0; a < 3; ++a) {
     const size_t ix = (size_t)wrap(gx + a - 1, M) * M;
