@@ -163,23 +163,17 @@ __global__ __launch_bounds__(256) void radix_finish(int n, int shift, const K* _
   if (i >= n) return;
   const K own = kin[i], up = own >> shift;
   int at = i;
-  const bool ahead = n - i > kMaxRun && kin[i + kMaxRun] >> shift == up;
-  if (ahead || (i >= kMaxRun && kin[i - kMaxRun] >> shift == up)) {
-    *long_run = 1;
-  } else {  // fewer than 2 kMaxRun pairs to look at
-    int lo = i - 1, hi = i + 1;
-    for (; lo >= 0; --lo) {
-      const K k = kin[lo];
-      if (k >> shift != up) break;
-      at -= k > own;  // comes after this one
+  auto same = [&](int j) { return j >= 0 && j < n && kin[j] >> shift == up; };
+  if (same(i - 1) || same(i + 1)) {
+    if ((n - i > kMaxRun && same(i + kMaxRun)) || same(i - kMaxRun)) {
+      *long_run = 1;
+    } else {  // fewer than 2 kMaxRun pairs to look at
+      int lo = i - 1, hi = i + 1;
+      for (; same(lo); --lo) at -= kin[lo] > own;  // comes after this one
+      for (; same(hi); ++hi) at += kin[hi] < own;
+      // the middle of a long run, whose pairs all keep their places
+      if (hi - lo - 1 > kMaxRun) at = i;
     }
-    for (; hi < n; ++hi) {
-      const K k = kin[hi];
-      if (k >> shift != up) break;
-      at += k < own;
-    }
-    // the middle of a long run, whose pairs all keep their places
-    if (hi - lo - 1 > kMaxRun) at = i;
   }
   kout[at] = own;
   vout[at] = vin[i];
